@@ -66,6 +66,7 @@ struct StageParams {
   int cur_stale;       // stale + immediate staling of the reconstructor
   double dt;           // timestep of this stage (dt/2 for the VL half step)
   double gamma;
+  double igm1;         // 1 / (gamma - 1)
   double density_floor;
   double pressure_floor;
   double theta;
@@ -122,7 +123,7 @@ __device__ __forceinline__ void floor_and_sync(double rho, const double v[3],
                                                double ggm1, double &etot,
                                                double &eint,
                                                bool *floored = nullptr) {
-  const double inv_rho = 1. / rho;
+  const double inv_rho = qrcp(rho);
   const double eint_floor = pfloor * (1. / (gamma - 1.)) * inv_rho;
   const double v2 = (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
   double non_thermal_e = 0.5 * v2;
@@ -321,8 +322,78 @@ __device__ __forceinline__ double center_efield(double vj, double vk, double bj,
 
 struct FluxConsts {
   double gm1, gamma, theta, dfloor, pfloor;
+  double igm1;  // 1 / (gamma - 1)
   unsigned long long *dbg;  // debug counters or null
 };
+
+// The flux through one face.
+template <typename T>
+struct FaceFlux {
+  T u[5];    // density, momentum x..z, total energy (slots S_RHO .. S_E)
+  T bj, bk;  // of the two transverse B components (D + 1, D + 2)
+  T e, vb;   // dual energy: internal-energy flux, interface velocity
+};
+
+// The Riemann solve of a face along D from its two reconstructed states (by
+// slot; the normal B component of both is bface).
+template <typename T, int RIEMANN, bool MHD, int D, bool DE>
+__device__ __forceinline__ void solve_face(const T wl[S_N], const T wr[S_N], T bface,
+                                           const FluxConsts &fc, FaceFlux<T> &f) {
+  constexpr int DJ = (D + 1) % 3, DK = (D + 2) % 3;
+  const T gamma = (T)fc.gamma;
+  T fo[8];
+  T vbar = T(0);
+  T *vb = DE ? &vbar : nullptr;
+  T eint_l = T(0), eint_r = T(0);
+  if (DE) {
+    eint_l = specific_eint(wl[S_RHO], wl[S_E], gamma);
+    eint_r = specific_eint(wr[S_RHO], wr[S_E], gamma);
+  }
+  if (MHD) {
+    T l8[8], r8[8];
+    l8[L_D] = wl[S_RHO]; r8[L_D] = wr[S_RHO];
+    l8[L_BI] = bface; r8[L_BI] = bface;
+    l8[L_BJ] = wl[S_BX + DJ]; r8[L_BJ] = wr[S_BX + DJ];
+    l8[L_BK] = wl[S_BX + DK]; r8[L_BK] = wr[S_BX + DK];
+    l8[L_VI] = wl[S_VX + D]; r8[L_VI] = wr[S_VX + D];
+    l8[L_VJ] = wl[S_VX + DJ]; r8[L_VJ] = wr[S_VX + DJ];
+    l8[L_VK] = wl[S_VX + DK]; r8[L_VK] = wr[S_VX + DK];
+    l8[L_E] = wl[S_E]; r8[L_E] = wr[S_E];
+    if (RIEMANN == RS_HLLD) {
+      hlld(l8, r8, gamma, (T)fc.igm1, fo, vb);
+    } else {
+      hlle_mhd(l8, r8, gamma, fo, vb);
+    }
+    f.u[S_RHO] = fo[L_D];
+    f.u[S_VX + D] = fo[L_VI];
+    f.u[S_VX + DJ] = fo[L_VJ];
+    f.u[S_VX + DK] = fo[L_VK];
+    f.u[S_E] = fo[L_E];
+    f.bj = fo[L_BJ];
+    f.bk = fo[L_BK];
+  } else {
+    T l5[5], r5[5];
+    l5[H_D] = wl[S_RHO]; r5[H_D] = wr[S_RHO];
+    l5[H_VI] = wl[S_VX + D]; r5[H_VI] = wr[S_VX + D];
+    l5[H_VJ] = wl[S_VX + DJ]; r5[H_VJ] = wr[S_VX + DJ];
+    l5[H_VK] = wl[S_VX + DK]; r5[H_VK] = wr[S_VX + DK];
+    l5[H_E] = wl[S_E]; r5[H_E] = wr[S_E];
+    hllc(l5, r5, gamma, fo, vb);
+    f.u[S_RHO] = fo[H_D];
+    f.u[S_VX + D] = fo[H_VI];
+    f.u[S_VX + DJ] = fo[H_VJ];
+    f.u[S_VX + DK] = fo[H_VK];
+    f.u[S_E] = fo[H_E];
+  }
+  if (DE) {
+    // the dual-energy outputs of the solve (EnzoRiemannHLLD.hpp:404-447,
+    // EnzoRiemannHLL.hpp:322-344, EnzoRiemannHLLC.hpp:159-170): the
+    // internal-energy flux from the stored density flux (slot 0 of either
+    // LUT), and vi_bar
+    f.e = upwind_eint_flux(eint_l, eint_r, fo[0]);
+    f.vb = vbar;
+  }
+}
 
 // Flux through the face between cell c and c + e_D (D fixed at compile
 // time so the i/j/k permutation costs nothing): reconstruction of both
@@ -375,61 +446,22 @@ __device__ __forceinline__ void flux_face(const BlockDesc<FluxT> &b, const Src &
       wr[q] = rv;
     }
   }
-  const T gamma = (T)fc.gamma;
-  T fo[8];
-  T vbar = T(0);
-  T *vb = DE ? &vbar : nullptr;
-  T eint_l = T(0), eint_r = T(0);
-  if (DE) {
-    eint_l = specific_eint(wl[S_RHO], wl[S_E], gamma);
-    eint_r = specific_eint(wr[S_RHO], wr[S_E], gamma);
-  }
+  T bface = T(0);
   if (MHD) {
     const int bnx = b.mx + (D == 0), bny = b.my + (D == 1);
-    const T bface =
-        (T)gld(bfi, (k + (D == 2)) * bny * bnx + (j + (D == 1)) * bnx + i + (D == 0));
-    T l8[8], r8[8];
-    l8[L_D] = wl[S_RHO]; r8[L_D] = wr[S_RHO];
-    l8[L_BI] = bface; r8[L_BI] = bface;
-    l8[L_BJ] = wl[S_BX + DJ]; r8[L_BJ] = wr[S_BX + DJ];
-    l8[L_BK] = wl[S_BX + DK]; r8[L_BK] = wr[S_BX + DK];
-    l8[L_VI] = wl[S_VX + D]; r8[L_VI] = wr[S_VX + D];
-    l8[L_VJ] = wl[S_VX + DJ]; r8[L_VJ] = wr[S_VX + DJ];
-    l8[L_VK] = wl[S_VX + DK]; r8[L_VK] = wr[S_VX + DK];
-    l8[L_E] = wl[S_E]; r8[L_E] = wr[S_E];
-    if (RIEMANN == RS_HLLD) {
-      hlld(l8, r8, gamma, fo, vb);
-    } else {
-      hlle_mhd(l8, r8, gamma, fo, vb);
-    }
-    gst(b.F[D][S_RHO], c, (FluxT)fo[L_D]);
-    gst(b.F[D][S_VX + D], c, (FluxT)fo[L_VI]);
-    gst(b.F[D][S_VX + DJ], c, (FluxT)fo[L_VJ]);
-    gst(b.F[D][S_VX + DK], c, (FluxT)fo[L_VK]);
-    gst(b.F[D][S_E], c, (FluxT)fo[L_E]);
-    gst(b.F[D][S_BX + DJ], c, (FluxT)fo[L_BJ]);
-    gst(b.F[D][S_BX + DK], c, (FluxT)fo[L_BK]);
-  } else {
-    T l5[5], r5[5];
-    l5[H_D] = wl[S_RHO]; r5[H_D] = wr[S_RHO];
-    l5[H_VI] = wl[S_VX + D]; r5[H_VI] = wr[S_VX + D];
-    l5[H_VJ] = wl[S_VX + DJ]; r5[H_VJ] = wr[S_VX + DJ];
-    l5[H_VK] = wl[S_VX + DK]; r5[H_VK] = wr[S_VX + DK];
-    l5[H_E] = wl[S_E]; r5[H_E] = wr[S_E];
-    hllc(l5, r5, gamma, fo, vb);
-    gst(b.F[D][S_RHO], c, (FluxT)fo[H_D]);
-    gst(b.F[D][S_VX + D], c, (FluxT)fo[H_VI]);
-    gst(b.F[D][S_VX + DJ], c, (FluxT)fo[H_VJ]);
-    gst(b.F[D][S_VX + DK], c, (FluxT)fo[H_VK]);
-    gst(b.F[D][S_E], c, (FluxT)fo[H_E]);
+    bface = (T)gld(bfi, (k + (D == 2)) * bny * bnx + (j + (D == 1)) * bnx + i + (D == 0));
+  }
+  FaceFlux<T> f;
+  solve_face<T, RIEMANN, MHD, D, DE>(wl, wr, bface, fc, f);
+#pragma unroll
+  for (int q = 0; q < 5; q++) gst(b.F[D][q], c, (FluxT)f.u[q]);
+  if (MHD) {
+    gst(b.F[D][S_BX + DJ], c, (FluxT)f.bj);
+    gst(b.F[D][S_BX + DK], c, (FluxT)f.bk);
   }
   if (DE) {
-    // the dual-energy outputs of the solve (EnzoRiemannHLLD.hpp:404-447,
-    // EnzoRiemannHLL.hpp:322-344, EnzoRiemannHLLC.hpp:159-170): the
-    // internal-energy flux from the stored density flux (slot 0 of either
-    // LUT), and vi_bar
-    gst(b.Fe[D], c, (double)upwind_eint_flux(eint_l, eint_r, fo[0]));
-    gst(b.Vb[D], c, (double)vbar);
+    gst(b.Fe[D], c, (double)f.e);
+    gst(b.Vb[D], c, (double)f.vb);
   }
 }
 
@@ -471,6 +503,7 @@ __device__ __forceinline__ void flux_cells(const BlockDesc<FluxT> *__restrict__ 
   FluxConsts fc;
   fc.gm1 = sp.gamma - 1.0;
   fc.gamma = sp.gamma;
+  fc.igm1 = sp.igm1;
   fc.theta = sp.theta;
   fc.dfloor = sp.density_floor;
   fc.pfloor = sp.pressure_floor;
@@ -566,6 +599,7 @@ k_flux_zp(const BlockDesc<FluxT> *__restrict__ blocks, StageParams sp, int zplan
   FluxConsts fc;
   fc.gm1 = sp.gamma - 1.0;
   fc.gamma = sp.gamma;
+  fc.igm1 = sp.igm1;
   fc.theta = sp.theta;
   fc.dfloor = sp.density_floor;
   fc.pfloor = sp.pressure_floor;
@@ -664,24 +698,18 @@ __device__ __forceinline__ double *const *center_e(const BlockDesc<FluxT> &b,
 // of the four cells around it (compute_center_efield, :267-292) and the
 // face fluxes of B and density.  FP64, never contracted: the same bits in
 // every kernel and build that evaluates it.
-template <int AX, typename FluxT>
-__device__ __forceinline__ double edge_emf(const BlockDesc<FluxT> &b, double *const *Ecs,
-                                           long c, long sj, long sk) {
+// With j, k the axes after AX: Ec* the centre E at the cell and its j, k
+// and jk neighbours; Fj, Fj_kp1 the j-face fluxes of B_k at the cell and its
+// k neighbour, Fk, Fk_jp1 the k-face fluxes of B_j at the cell and its j
+// neighbour, and D* the density fluxes of the same faces.
+__device__ __forceinline__ double edge_value(double Ec, double Ec_jp1, double Ec_kp1,
+                                             double Ec_jkp1, double Ej, double Ej_kp1, double Ek,
+                                             double Ek_jp1, double Dj, double Dj_kp1, double Dk,
+                                             double Dk_jp1) {
 #pragma clang fp contract(off)
-  constexpr int aj = (AX + 1) % 3, ak = (AX + 2) % 3;
-  const double *Eci = Ecs[AX];
-  const double Ec = Eci[c], Ec_jp1 = Eci[c + sj], Ec_kp1 = Eci[c + sk],
-               Ec_jkp1 = Eci[c + sj + sk];
+  const double Wj = upwind_weight(Dj), Wj_kp1 = upwind_weight(Dj_kp1);
+  const double Wk = upwind_weight(Dk), Wk_jp1 = upwind_weight(Dk_jp1);
   // face E: j-faces carry -F_j(B_k), k-faces +F_k(B_j)
-  const FluxT *Fj = b.F[aj][S_BX + ak];
-  const FluxT *Fk = b.F[ak][S_BX + aj];
-  const double Ej = (double)Fj[c], Ej_kp1 = (double)Fj[c + sk];
-  const double Ek = (double)Fk[c], Ek_jp1 = (double)Fk[c + sj];
-  const double Wj = upwind_weight((double)b.F[aj][S_RHO][c]);
-  const double Wj_kp1 = upwind_weight((double)b.F[aj][S_RHO][c + sk]);
-  const double Wk = upwind_weight((double)b.F[ak][S_RHO][c]);
-  const double Wk_jp1 = upwind_weight((double)b.F[ak][S_RHO][c + sj]);
-
   double dEdj_r = Wk_jp1 * (Ec_jp1 + Ej) + (1 - Wk_jp1) * (Ec_jkp1 + Ej_kp1);
   double dEdj_l = Wk * (-Ej - Ec) + (1 - Wk) * (-Ej_kp1 - Ec_kp1);
   double dEdk_r = Wj_kp1 * (Ec_kp1 - Ek) + (1 - Wj_kp1) * (Ec_jkp1 - Ek_jp1);
@@ -690,6 +718,17 @@ __device__ __forceinline__ double edge_emf(const BlockDesc<FluxT> &b, double *co
   Ej_sum *= -1;
   double Ek_sum = Ek + Ek_jp1;
   return 0.25 * (Ej_sum + Ek_sum + (dEdj_l - dEdj_r) + (dEdk_l - dEdk_r));
+}
+template <int AX, typename FluxT>
+__device__ __forceinline__ double edge_emf(const BlockDesc<FluxT> &b, double *const *Ecs,
+                                           long c, long sj, long sk) {
+  constexpr int aj = (AX + 1) % 3, ak = (AX + 2) % 3;
+  const double *Eci = Ecs[AX];
+  const FluxT *Fj = b.F[aj][S_BX + ak], *Fk = b.F[ak][S_BX + aj];
+  const FluxT *Dj = b.F[aj][S_RHO], *Dk = b.F[ak][S_RHO];
+  return edge_value(Eci[c], Eci[c + sj], Eci[c + sk], Eci[c + sj + sk], (double)Fj[c],
+                    (double)Fj[c + sk], (double)Fk[c], (double)Fk[c + sj], (double)Dj[c],
+                    (double)Dj[c + sk], (double)Dk[c], (double)Dk[c + sj]);
 }
 
 // Whether the edge EMF along axis ax at cell-shaped index p is one the
@@ -826,14 +865,15 @@ __device__ __forceinline__ double cfl_speed(double d, double vx, double vy, doub
   double sig;
   if (MHD) {
     double B2 = ((bx * bx) + ((by * by) + (bz * bz)));
-    double cs2 = gamma * p / d;
-    double va2 = B2 / d;
-    sig = sqrt(va2 + cs2);
+    const double inv = qrcp(d);
+    double cs2 = qdiv_inv(gamma * p, d, inv);
+    double va2 = qdiv_inv(B2, d, inv);
+    sig = qsqrt(va2 + cs2);
   } else {
-    sig = sqrt(gamma * p / d);
+    sig = qsqrt(qdiv(gamma * p, d));
   }
-  return dmin3(cw[0] / (fabs(vx) + sig), cw[1] / (fabs(vy) + sig),
-               cw[2] / (fabs(vz) + sig));
+  return dmin3(qdiv(cw[0], fabs(vx) + sig), qdiv(cw[1], fabs(vy) + sig),
+               qdiv(cw[2], fabs(vz) + sig));
 }
 template <bool MHD>
 __device__ __forceinline__ double cfl_cell(double d, double vx, double vy, double vz,
@@ -870,6 +910,149 @@ __device__ __forceinline__ void block_min_to(unsigned long long *result, double 
     if (m < __hip_atomic_load(result, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
       atomicMin(result, m);
   }
+}
+
+// ----------------------------------------------------- end of an update
+
+// Start-of-step values of one cell: the base of its update.
+struct CellBase {
+  double rho, v[3], e, ei;
+};
+
+// Loads and stores at a byte offset from a field's (uniform) base pointer:
+// the offset is one 32-bit register for every field of a shape, and the
+// instruction adds the base itself.
+template <typename P>
+__device__ __forceinline__ P ldo(const P *base, unsigned off) {
+  return *(const __attribute__((address_space(1))) P *)(
+      (const __attribute__((address_space(1))) char *)base + off);
+}
+template <typename P>
+__device__ __forceinline__ void sto(P *base, unsigned off, P v) {
+  *(__attribute__((address_space(1))) P *)((__attribute__((address_space(1))) char *)base +
+                                           off) = v;
+}
+// Index of a cell in the field arrays: an element index, or (the marched
+// stages) a byte offset in an FP64 field.
+struct CellIndex {
+  long c;
+  __device__ __forceinline__ double load(const double *p) const { return gld(p, (int)c); }
+  template <typename P>
+  __device__ __forceinline__ void store(P *p, P v) const {
+    gst(p, c, v);
+  }
+};
+struct CellOffset {
+  unsigned off;
+  __device__ __forceinline__ double load(const double *p) const { return ldo(p, off); }
+  __device__ __forceinline__ void store(double *p, double v) const { sto(p, off, v); }
+  __device__ __forceinline__ void store(float *p, float v) const { sto(p, off >> 1, v); }
+};
+
+// The end of a cell's update, shared by the kernels that run it: gravity,
+// the conserved update of u0 by dU (and dUe), the floors or the dual-energy
+// synchronisation, and the writes of the new state at cell c (bc: its
+// centre B, written by the caller where it is stored in FP64).  HALF_P: the
+// half-step state gets the pressure in the place of the total energy.
+// Returns the cell's CFL term when sp.cfl asks for it, else DBL_MAX.
+template <typename FluxT, bool MHD, bool DE, bool HALF_P, class Cell>
+__device__ __forceinline__ double cell_finish(const BlockDesc<FluxT> &b, const StageParams &sp,
+                                              double dt, const Cell &c, const CellBase &u0,
+                                              double dU[5], double dUe, const double bc[3]) {
+#pragma clang fp contract(off)
+  constexpr bool HALF_F32 = std::is_same<FluxT, float>::value && !DE;
+  double local = 1.7976931348623157e308;
+  // gravity (EnzoSourceGravity::calculate_source, EnzoSourceGravity.cpp:
+  // 17-69) on the stage with index 1, from the start-of-step state, after
+  // the flux divergence (EnzoMHDIntegratorStageCommands.cpp:180-182,
+  // 265-295)
+  if (sp.stage == 1 && b.acc[0] != nullptr) {
+    const double rho = u0.rho;
+    const double ax = c.load(b.acc[0]), ay = c.load(b.acc[1]), az = c.load(b.acc[2]);
+    dU[1] += dt * rho * ax;
+    dU[2] += dt * rho * ay;
+    dU[3] += dt * rho * az;
+    dU[4] += dt * rho * ((u0.v[0] * ax) + (u0.v[1] * ay) + (u0.v[2] * az));
+  }
+  // the update base is always the start-of-step state
+  double old_rho = u0.rho;
+  double new_rho = u0.rho + dU[0];
+  if (sp.dbg) debug_count(sp.dbg, DBG_DENSITY_FLOOR, new_rho < sp.density_floor);
+  new_rho = dmax(new_rho, sp.density_floor);
+  double inv_new_rho = qrcp(new_rho);
+  double v[3];
+#pragma unroll
+  for (int q = 0; q < 3; q++) v[q] = (u0.v[q] * old_rho + dU[q + 1]) * inv_new_rho;
+  double etot = (u0.e * old_rho + dU[4]) * inv_new_rho;
+  double eint = 0.;
+  if (DE) eint = (u0.ei * old_rho + dUe) * inv_new_rho;
+  // energy floor (and synchronisation)
+  const double b2 = MHD ? (bc[0] * bc[0] + bc[1] * bc[1] + bc[2] * bc[2]) : 0.;
+  bool floored = false;
+  floor_and_sync<MHD, DE>(new_rho, v, b2, sp.gamma, sp.pressure_floor, sp.eta, sp.ggm1, etot,
+                          eint, sp.dbg ? &floored : nullptr);
+  if (sp.dbg) {
+    debug_count(sp.dbg, DBG_ENERGY_FLOOR, floored);
+    bool finite = isfinite(new_rho) && isfinite(v[0]) && isfinite(v[1]) && isfinite(v[2]) &&
+                  isfinite(etot) && isfinite(b2);
+    if (DE) finite = finite && isfinite(eint);
+    debug_count(sp.dbg, DBG_NONFINITE, !finite);
+  }
+  if (HALF_F32 && !sp.is_final) {
+    // the mixed path keeps the half-step state as FP32 primitives (b.Up)
+    // plus the FP64 centre E of the next stage's edge EMFs
+    float *const *Up = b.Up;
+    c.store(Up[S_RHO], (float)new_rho);
+    c.store(Up[S_VX], (float)v[0]);
+    c.store(Up[S_VY], (float)v[1]);
+    c.store(Up[S_VZ], (float)v[2]);
+    c.store(Up[S_E], (float)prim_pressure<MHD>(new_rho, v[0], v[1], v[2], etot, bc[0], bc[1],
+                                              bc[2], sp.gamma - 1.0));
+    if (MHD) {
+      c.store(Up[S_BX], (float)bc[0]);
+      c.store(Up[S_BY], (float)bc[1]);
+      c.store(Up[S_BZ], (float)bc[2]);
+      c.store(b.Ech[0], center_efield(v[1], v[2], bc[1], bc[2]));
+      c.store(b.Ech[1], center_efield(v[2], v[0], bc[2], bc[0]));
+      c.store(b.Ech[2], center_efield(v[0], v[1], bc[0], bc[1]));
+    }
+    return local;
+  }
+  if (HALF_P && !sp.is_final) {
+    c.store(b.Ut[S_RHO], new_rho);
+    c.store(b.Ut[S_VX], v[0]);
+    c.store(b.Ut[S_VY], v[1]);
+    c.store(b.Ut[S_VZ], v[2]);
+    // load_prim's pressure of this state
+    c.store(b.Ut[S_E], DE ? (sp.gamma - 1.0) * new_rho * eint
+                          : prim_pressure<MHD>(new_rho, v[0], v[1], v[2], etot, bc[0], bc[1],
+                                               bc[2], sp.gamma - 1.0));
+    return local;
+  }
+  double *const *Uo = sp.is_final ? b.U : b.Ut;
+  c.store(Uo[S_RHO], new_rho);
+  c.store(Uo[S_VX], v[0]);
+  c.store(Uo[S_VY], v[1]);
+  c.store(Uo[S_VZ], v[2]);
+  if (sp.cfl) {
+    double p;
+    if (DE) {
+      // the timestep synchronises the energies of the cell once more, in
+      // place, before its pressure (EnzoMethodMHDVlct.cpp:563-568)
+      floor_and_sync<MHD, DE>(new_rho, v, b2, sp.gamma, sp.pressure_floor, sp.eta, sp.ggm1,
+                              etot, eint);
+      p = (sp.gamma - 1.0) * new_rho * eint;
+      local = cfl_speed<MHD>(new_rho, v[0], v[1], v[2], bc[0], bc[1], bc[2], p, sp.gamma,
+                             b.cw);
+    } else {
+      local = cfl_cell<MHD>(new_rho, v[0], v[1], v[2], etot, bc[0], bc[1], bc[2], sp.gamma,
+                            b.cw, p);
+    }
+    if (b.pressure) c.store(b.pressure, p);
+  }
+  c.store(Uo[S_E], etot);
+  if (DE) c.store(sp.is_final ? b.ei : b.eit, eint);
+  return local;
 }
 
 // --------------------------------------------------------------- k_cells
@@ -983,84 +1166,14 @@ __device__ __forceinline__ double cell_stage(const BlockDesc<FluxT> &b, const St
         dUe -= dtdx * pc * (b.Vb[d][c] - b.Vb[d][c - str[d]]);
       }
     }
-    // gravity (EnzoSourceGravity::calculate_source, EnzoSourceGravity.cpp:
-    // 17-69) on the stage with index 1, from the start-of-step state, after
-    // the flux divergence (EnzoMHDIntegratorStageCommands.cpp:180-182,
-    // 265-295)
-    if (sp.stage == 1 && b.acc[0] != nullptr) {
-      const double rho = b.U[S_RHO][c];
-      const double ax = b.acc[0][c], ay = b.acc[1][c], az = b.acc[2][c];
-      dU[1] += dt * rho * ax;
-      dU[2] += dt * rho * ay;
-      dU[3] += dt * rho * az;
-      dU[4] += dt * rho * ((b.U[S_VX][c] * ax) + (b.U[S_VY][c] * ay) +
-                           (b.U[S_VZ][c] * az));
-    }
-    // the update base is always the start-of-step state
-    double old_rho = b.U[S_RHO][c];
-    double new_rho = b.U[S_RHO][c] + dU[0];
-    if (sp.dbg) debug_count(sp.dbg, DBG_DENSITY_FLOOR, new_rho < sp.density_floor);
-    new_rho = dmax(new_rho, sp.density_floor);
-    double inv_new_rho = 1. / new_rho;
-    double v[3];
-  #pragma unroll
-    for (int q = 1; q < 4; q++)
-      v[q - 1] = (b.U[fq[q]][c] * old_rho + dU[q]) * inv_new_rho;
-    double etot = (b.U[S_E][c] * old_rho + dU[4]) * inv_new_rho;
-    double eint = 0.;
-    if (DE) eint = (b.ei[c] * old_rho + dUe) * inv_new_rho;
-    // energy floor (and synchronisation)
-    const double b2 = MHD ? (bc[0] * bc[0] + bc[1] * bc[1] + bc[2] * bc[2]) : 0.;
-    bool floored = false;
-    floor_and_sync<MHD, DE>(new_rho, v, b2, sp.gamma, sp.pressure_floor, sp.eta, sp.ggm1,
-                            etot, eint, sp.dbg ? &floored : nullptr);
-    if (sp.dbg) {
-      debug_count(sp.dbg, DBG_ENERGY_FLOOR, floored);
-      bool finite = isfinite(new_rho) && isfinite(v[0]) && isfinite(v[1]) &&
-                    isfinite(v[2]) && isfinite(etot) && isfinite(b2);
-      if (DE) finite = finite && isfinite(eint);
-      debug_count(sp.dbg, DBG_NONFINITE, !finite);
-    }
-    if (to_f32) {
-      float *const *Up = b.Up;
-      gst(Up[S_RHO], c, (float)new_rho);
-      gst(Up[S_VX], c, (float)v[0]);
-      gst(Up[S_VY], c, (float)v[1]);
-      gst(Up[S_VZ], c, (float)v[2]);
-      gst(Up[S_E], c, (float)prim_pressure<MHD>(new_rho, v[0], v[1], v[2], etot, bc[0], bc[1],
-                                                bc[2], sp.gamma - 1.0));
-      if (MHD) {
-        gst(Up[S_BX], c, (float)bc[0]);
-        gst(Up[S_BY], c, (float)bc[1]);
-        gst(Up[S_BZ], c, (float)bc[2]);
-        gst(b.Ech[0], c, center_efield(v[1], v[2], bc[1], bc[2]));
-        gst(b.Ech[1], c, center_efield(v[2], v[0], bc[2], bc[0]));
-        gst(b.Ech[2], c, center_efield(v[0], v[1], bc[0], bc[1]));
-      }
-      return;
-    }
-    Uo[S_RHO][c] = new_rho;
-    Uo[S_VX][c] = v[0];
-    Uo[S_VY][c] = v[1];
-    Uo[S_VZ][c] = v[2];
-    if (cfl) {
-      double p;
-      if (DE) {
-        // the timestep synchronises the energies of the cell once more, in
-        // place, before its pressure (EnzoMethodMHDVlct.cpp:563-568)
-        floor_and_sync<MHD, DE>(new_rho, v, b2, sp.gamma, sp.pressure_floor, sp.eta,
-                                sp.ggm1, etot, eint);
-        p = (sp.gamma - 1.0) * new_rho * eint;
-        local = cfl_speed<MHD>(new_rho, v[0], v[1], v[2], bc[0], bc[1], bc[2], p, sp.gamma,
-                               b.cw);
-      } else {
-        local = cfl_cell<MHD>(new_rho, v[0], v[1], v[2], etot, bc[0], bc[1], bc[2],
-                              sp.gamma, b.cw, p);
-      }
-      if (b.pressure) b.pressure[c] = p;
-    }
-    Uo[S_E][c] = etot;
-    if (DE) (sp.is_final ? b.ei : b.eit)[c] = eint;
+    CellBase u0;
+    u0.rho = b.U[S_RHO][c];
+    u0.v[0] = b.U[S_VX][c];
+    u0.v[1] = b.U[S_VY][c];
+    u0.v[2] = b.U[S_VZ][c];
+    u0.e = b.U[S_E][c];
+    if (DE) u0.ei = b.ei[c];
+    local = cell_finish<FluxT, MHD, DE, false>(b, sp, dt, CellIndex{c}, u0, dU, dUe, bc);
   };
   if (in_box) {
     body();

@@ -613,6 +613,7 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
       sp.dts = dts ? dts + c0 : nullptr;
       sp.dt_factor = (!is_final) ? 0.5 : 1.0;
       sp.gamma = m->gamma;
+      sp.igm1 = 1. / (m->gamma - 1.);
       sp.density_floor = m->dfloor;
       sp.pressure_floor = m->pfloor;
       sp.theta = m->theta;

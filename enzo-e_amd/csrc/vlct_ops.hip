@@ -210,7 +210,7 @@ __global__ void k_op_riemann(KMap pl, KMap pr, KMap fx8, Box box, int dim,
       eint_l = specific_eint(l[L_D], l[L_E], gamma);
       eint_r = specific_eint(r[L_D], r[L_E], gamma);
     }
-    if (RIEMANN == RS_HLLD) hlld(l, r, gamma, o, vb);
+    if (RIEMANN == RS_HLLD) hlld(l, r, gamma, 1. / (gamma - 1.), o, vb);
     else hlle_mhd(l, r, gamma, o, vb);
     for (int q = 0; q < 8; q++) fx8.p[src[q]][f] = o[q];
   } else {

@@ -32,17 +32,88 @@ enum : int { H_D = 0, H_VI, H_VJ, H_VK, H_E };
 enum : int { RS_HLLE = 0, RS_HLLC = 1, RS_HLLD = 2 };
 enum : int { RC_NN = 0, RC_PLM = 1, RC_PLM_ATHENA = 2 };
 
-// Division and square root: exact IEEE operations in FP64 (reference
-// parity); hardware reciprocal / square root (about 1 ulp) in FP32, where
-// the mixed-precision path is judged by its L1 error instead.
-__device__ __forceinline__ double qdiv(double a, double b) { return a / b; }
+// Division and square root: correctly rounded in FP64 (reference parity);
+// hardware reciprocal / square root (about 1 ulp) in FP32, where the
+// mixed-precision path is judged by its L1 error instead.
+//
+// The FP64 division without the operand scaling that covers the ends of the
+// exponent range: the hardware's reciprocal (24 good bits), two Newton
+// steps, the product and one correction by the exact residual; 1 / b takes
+// one cubic step and the correction (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990).  The hardware's
+// fix-up puts zeros, infinities and NaN right.  9 and 7 instructions instead
+// of 11, and none of the wait states that the scaled form's flag costs.
+// Rounded as IEEE division for 2^-1000 < |b| < 2^1000 and quotients and
+// residuals in the normal range.  With the shared reciprocals (qdiv_inv) and
+// the roots below the FP64 flux kernels, bound by their instruction issue,
+// take 1.51 and 2.11 ms on a 256^3 block (nearest neighbour, PLM) instead
+// of 1.67 and 2.23.
+__device__ __forceinline__ double qrcp(double b) {
+  const double y0 = __builtin_amdgcn_rcp(b);
+  const double e = __builtin_fma(-b, y0, 1.0);
+  const double y = __builtin_fma(__builtin_fma(e, e, e), y0, y0);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, y, 1.0), y, y), b, 1.0);
+}
+__device__ __forceinline__ float qrcp(float b) { return __builtin_amdgcn_rcpf(b); }
+__device__ __forceinline__ double qdiv(double a, double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+  const double q = a * y;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
+}
 __device__ __forceinline__ float qdiv(float a, float b) {
   return a * __builtin_amdgcn_rcpf(b);
 }
-__device__ __forceinline__ double qsqrt(double a) { return sqrt(a); }
+// The FP64 square root without the scaling steps that a general one needs:
+// from the hardware's reciprocal root, one Goldschmidt step and two
+// corrections of g by the exact residual x - g g (Markstein, "IA-64 and
+// Elementary Functions", 2000), 10 instructions, for 2^-767 <= x < 2^769;
+// sqrt() outside (zeros, negatives, NaN among them).  Correctly rounded
+// either way.  The pair form takes two roots side by side, so that their
+// dependent chains overlap, behind one test.
+__device__ __forceinline__ double root_tame(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+__device__ __forceinline__ unsigned root_key(double x) {
+  return (unsigned)(__double2hiint(x) - 0x10000000);
+}
+constexpr unsigned ROOT_KEYS = 0x60000000u;  // keys of the tame range lie below
+__device__ __forceinline__ double qsqrt(double x) {
+  double g = root_tame(x);
+  if (__builtin_expect(root_key(x) >= ROOT_KEYS, 0)) g = sqrt(x);
+  return g;
+}
+__device__ __forceinline__ void qsqrt2(double a, double b, double &ra, double &rb) {
+  ra = root_tame(a);
+  rb = root_tame(b);
+  const unsigned ka = root_key(a), kb = root_key(b);
+  if (__builtin_expect((ka > kb ? ka : kb) >= ROOT_KEYS, 0)) {
+    ra = sqrt(a);
+    rb = sqrt(b);
+  }
+}
+__device__ __forceinline__ void qsqrt2(float a, float b, float &ra, float &rb) {
+  ra = __builtin_amdgcn_sqrtf(a);
+  rb = __builtin_amdgcn_sqrtf(b);
+}
 __device__ __forceinline__ float qsqrt(float a) {
   return __builtin_amdgcn_sqrtf(a);
 }
+// a / b where inv = 1 / b is at hand: in FP64 the product and one correction
+// by the exact residual, which rounds as the division does when inv is the
+// correctly rounded reciprocal: 4 instructions.
+__device__ __forceinline__ double qdiv_inv(double a, double b, double inv) {
+  const double q = a * inv;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), inv, q), b, a);
+}
+__device__ __forceinline__ float qdiv_inv(float a, float, float inv) { return a * inv; }
 
 template <typename T> __device__ __forceinline__ T dmin(T a, T b) {
   return (b < a) ? b : a;  // std::min
@@ -102,18 +173,28 @@ __device__ __forceinline__ T limiter_athena(T vm1, T v, T vp1) {
   return qdiv(T(2) * temp, dv_l + dv_r);
 }
 
-// EnzoEOSIdeal::fast_magnetosonic_speed<-1> (EnzoEOSIdeal.hpp:111-140);
-// std::pow(x, 2) == x*x exactly.
+// EnzoEOSIdeal::fast_magnetosonic_speed<-1> (EnzoEOSIdeal.hpp:111-140) of
+// the two states of a face, side by side; std::pow(x, 2) == x*x exactly.
+// w in the MHD LUT order.
 template <typename T>
-__device__ __forceinline__ T fast_ms_speed(T d, T p, T bi, T bj, T bk,
-                                           T gamma) {
-  const T B2 = ((bi * bi) + ((bj * bj) + (bk * bk)));
-  const T cs2 = qdiv(gamma * p, d);
-  const T inv_density = qdiv(T(1), d);
-  const T va2 = B2 * inv_density;
-  const T va2_cos2 = (bi * bi) * inv_density;
-  const T sum = cs2 + va2;
-  return qsqrt(T(0.5) * (va2 + cs2 + qsqrt(sum * sum - T(4) * cs2 * va2_cos2)));
+__device__ __forceinline__ void fast_ms_speeds(const T wl[8], const T wr[8], T gamma, T &cl,
+                                               T &cr) {
+  const T *w[2] = {wl, wr};
+  T sum[2], rad[2], s1[2], rt[2];
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    const T d = w[s][L_D], bi = w[s][L_BI], bj = w[s][L_BJ], bk = w[s][L_BK];
+    const T B2 = ((bi * bi) + ((bj * bj) + (bk * bk)));
+    const T inv_density = qrcp(d);
+    const T cs2 = qdiv_inv(gamma * w[s][L_E], d, inv_density);
+    const T va2 = B2 * inv_density;
+    const T va2_cos2 = (bi * bi) * inv_density;
+    sum[s] = va2 + cs2;
+    s1[s] = cs2 + va2;
+    rad[s] = s1[s] * s1[s] - T(4) * cs2 * va2_cos2;
+  }
+  qsqrt2(rad[0], rad[1], rt[0], rt[1]);
+  qsqrt2(T(0.5) * (sum[0] + rt[0]), T(0.5) * (sum[1] + rt[1]), cl, cr);
 }
 
 template <typename T> struct Cons1D { T d, mx, my, mz, e, by, bz; };
@@ -140,11 +221,11 @@ __device__ __forceinline__ T upwind_eint_flux(T eint_l, T eint_r, T density_flux
 // MHD LUT order; flux[L_BI] is 0.  vbar (dual energy, may be null): the
 // interface velocity of :418-447 -- the left/right normal velocity outside
 // the fan, else the contact speed scaled by the outer state's coefficient.
+// igm1: 1 / (gamma - 1), the same for every face of a launch.
 template <typename T>
-__device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma,
+__device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma, T igm1,
                                      T flx[8], T *vbar = nullptr) {
   const T SMALL_NUMBER = T(1.0e-8);
-  const T igm1 = qdiv(T(1), gamma - T(1));
   T spd[5];
   Cons1D<T> ul, ur, ulst, uldst, urdst, urst, fl, fr;
   // the outer states' physical fluxes are formed where the fan region is
@@ -181,10 +262,8 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma,
   ur.by = wri[L_BJ];
   ur.bz = wri[L_BK];
 
-  T cfl = fast_ms_speed(wli[L_D], pressure_l, wli[L_BI], wli[L_BJ], wli[L_BK],
-                        gamma);
-  T cfr = fast_ms_speed(wri[L_D], pressure_r, wri[L_BI], wri[L_BJ], wri[L_BK],
-                        gamma);
+  T cfl, cfr;
+  fast_ms_speeds(wli, wri, gamma, cfl, cfr);
 
   spd[0] = dmin(wli[L_VI] - cfl, wri[L_VI] - cfr);
   spd[4] = dmax(wli[L_VI] + cfl, wri[L_VI] + cfr);
@@ -199,12 +278,14 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma,
 
   T sdml = spd[0] - spd[2];
   T sdmr = spd[4] - spd[2];
+  T sdml_inv = qrcp(sdml);
+  T sdmr_inv = qrcp(sdmr);
   if (vbar) {
     // as soon as the outer and contact speeds are known (fewer live
     // registers through the rest of the solve): l_coef = (S_l - vx_L) /
     // (S_l - S_M) = sdl / sdml, r_coef = sdr / sdmr
-    const T l_coef = qdiv(sdl, sdml);
-    const T r_coef = qdiv(sdr, sdmr);
+    const T l_coef = qdiv_inv(sdl, sdml, sdml_inv);
+    const T r_coef = qdiv_inv(sdr, sdmr, sdmr_inv);
     if (spd[0] > T(0)) {
       *vbar = wli[L_VI];
     } else if (spd[4] < T(0)) {
@@ -215,14 +296,12 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma,
       *vbar = spd[2] * r_coef;
     }
   }
-  T sdml_inv = qdiv(T(1), sdml);
-  T sdmr_inv = qdiv(T(1), sdmr);
   ulst.d = ul.d * sdl * sdml_inv;
   urst.d = ur.d * sdr * sdmr_inv;
-  T ulst_d_inv = qdiv(T(1), ulst.d);
-  T urst_d_inv = qdiv(T(1), urst.d);
-  T sqrtdl = qsqrt(ulst.d);
-  T sqrtdr = qsqrt(urst.d);
+  T ulst_d_inv = qrcp(ulst.d);
+  T urst_d_inv = qrcp(urst.d);
+  T sqrtdl, sqrtdr;
+  qsqrt2(ulst.d, urst.d, sqrtdl, sqrtdr);
 
   spd[1] = spd[2] - qdiv(fabs(bxi), sqrtdl);
   spd[3] = spd[2] + qdiv(fabs(bxi), sqrtdr);
@@ -231,19 +310,41 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma,
   T ptstr = ptr + ur.d * sdr * (spd[2] - wri[L_VI]);
   T ptst = T(0.5) * (ptstr + ptstl);
 
+  // the transverse star states of both sides, side by side, then the rare
+  // side whose Alfven wave sits on the outer one
   ulst.mx = ulst.d * spd[2];
-  if (fabs(ul.d * sdl * sdml - bxsq) < (SMALL_NUMBER)*ptst) {
-    ulst.my = ulst.d * wli[L_VJ];
-    ulst.mz = ulst.d * wli[L_VK];
-    ulst.by = ul.by;
-    ulst.bz = ul.bz;
-  } else {
-    T tmp = qdiv(bxi * (sdl - sdml), ul.d * sdl * sdml - bxsq);
-    ulst.my = ulst.d * (wli[L_VJ] - ul.by * tmp);
-    ulst.mz = ulst.d * (wli[L_VK] - ul.bz * tmp);
-    tmp = qdiv(ul.d * (sdl * sdl) - bxsq, ul.d * sdl * sdml - bxsq);
-    ulst.by = ul.by * tmp;
-    ulst.bz = ul.bz * tmp;
+  urst.mx = urst.d * spd[2];
+  {
+    const T denl = ul.d * sdl * sdml - bxsq, denr = ur.d * sdr * sdmr - bxsq;
+    const T denl_inv = qrcp(denl), denr_inv = qrcp(denr);
+    T tmpl = qdiv_inv(bxi * (sdl - sdml), denl, denl_inv);
+    T tmpr = qdiv_inv(bxi * (sdr - sdmr), denr, denr_inv);
+    ulst.my = ulst.d * (wli[L_VJ] - ul.by * tmpl);
+    ulst.mz = ulst.d * (wli[L_VK] - ul.bz * tmpl);
+    urst.my = urst.d * (wri[L_VJ] - ur.by * tmpr);
+    urst.mz = urst.d * (wri[L_VK] - ur.bz * tmpr);
+    tmpl = qdiv_inv(ul.d * (sdl * sdl) - bxsq, denl, denl_inv);
+    tmpr = qdiv_inv(ur.d * (sdr * sdr) - bxsq, denr, denr_inv);
+    ulst.by = ul.by * tmpl;
+    ulst.bz = ul.bz * tmpl;
+    urst.by = ur.by * tmpr;
+    urst.bz = ur.bz * tmpr;
+    const bool flat_l = fabs(denl) < (SMALL_NUMBER)*ptst;
+    const bool flat_r = fabs(denr) < (SMALL_NUMBER)*ptst;
+    if (__builtin_expect(flat_l || flat_r, 0)) {
+      if (flat_l) {
+        ulst.my = ulst.d * wli[L_VJ];
+        ulst.mz = ulst.d * wli[L_VK];
+        ulst.by = ul.by;
+        ulst.bz = ul.bz;
+      }
+      if (flat_r) {
+        urst.my = urst.d * wri[L_VJ];
+        urst.mz = urst.d * wri[L_VK];
+        urst.by = ur.by;
+        urst.bz = ur.bz;
+      }
+    }
   }
   T vbstl =
       (ulst.mx * bxi + (ulst.my * ulst.by + ulst.mz * ulst.bz)) * ulst_d_inv;
@@ -251,21 +352,6 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma,
             bxi * (wli[L_VI] * bxi + (wli[L_VJ] * ul.by + wli[L_VK] * ul.bz) -
                    vbstl)) *
            sdml_inv;
-
-  urst.mx = urst.d * spd[2];
-  if (fabs(ur.d * sdr * sdmr - bxsq) < (SMALL_NUMBER)*ptst) {
-    urst.my = urst.d * wri[L_VJ];
-    urst.mz = urst.d * wri[L_VK];
-    urst.by = ur.by;
-    urst.bz = ur.bz;
-  } else {
-    T tmp = qdiv(bxi * (sdr - sdmr), ur.d * sdr * sdmr - bxsq);
-    urst.my = urst.d * (wri[L_VJ] - ur.by * tmp);
-    urst.mz = urst.d * (wri[L_VK] - ur.bz * tmp);
-    tmp = qdiv(ur.d * (sdr * sdr) - bxsq, ur.d * sdr * sdmr - bxsq);
-    urst.by = ur.by * tmp;
-    urst.bz = ur.bz * tmp;
-  }
   T vbstr =
       (urst.mx * bxi + (urst.my * urst.by + urst.mz * urst.bz)) * urst_d_inv;
   urst.e = (sdr * ur.e - ptr * wri[L_VI] + ptst * spd[2] +
@@ -277,7 +363,7 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma,
     uldst = ulst;
     urdst = urst;
   } else {
-    T invsumd = qdiv(T(1), sqrtdl + sqrtdr);
+    T invsumd = qrcp(sqrtdl + sqrtdr);
     T bxsig = (bxi > T(0) ? T(1) : T(-1));
     uldst.d = ulst.d;
     urdst.d = urst.d;
@@ -306,7 +392,7 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma,
                          ((urst.mz * urst_d_inv) - (ulst.mz * ulst_d_inv)));
     uldst.bz = urdst.bz = tmp;
 
-    tmp = spd[2] * bxi + qdiv(uldst.my * uldst.by + uldst.mz * uldst.bz, uldst.d);
+    tmp = spd[2] * bxi + qdiv_inv(uldst.my * uldst.by + uldst.mz * uldst.bz, uldst.d, ulst_d_inv);
     uldst.e = ulst.e - sqrtdl * bxsig * (vbstl - tmp);
     urdst.e = urst.e + sqrtdr * bxsig * (vbstr - tmp);
   }
@@ -389,7 +475,7 @@ __device__ __forceinline__ void mhd_cons_flux(const T w[8], T gamma, T cons[8],
   for (int i = 4; i < 8; i++) cons[i] = w[i] * w[L_D];
   {
     T density = w[L_D];
-    T internal_edens = qdiv(w[L_E], gamma - T(1));
+    T internal_edens = qdiv_inv(w[L_E], gamma - T(1), qrcp(gamma - T(1)));
     const T vi = w[L_VI], vj = w[L_VJ], vk = w[L_VK];
     const T kinetic = T(0.5) * density * ((vi * vi) + ((vj * vj) + (vk * vk)));
     T magnetic = T(0.5) * ((w[L_BI] * w[L_BI]) +
@@ -421,13 +507,13 @@ __device__ __forceinline__ void hlle_mhd(const T wl[8], const T wr[8],
   T cl[8], cr[8], fl[8], fr[8];
   mhd_cons_flux(wl, gamma, cl, fl);
   mhd_cons_flux(wr, gamma, cr, fr);
-  T c_l = fast_ms_speed(wl[L_D], wl[L_E], wl[L_BI], wl[L_BJ], wl[L_BK], gamma);
-  T c_r = fast_ms_speed(wr[L_D], wr[L_E], wr[L_BI], wr[L_BJ], wr[L_BK], gamma);
+  T c_l, c_r;
+  fast_ms_speeds(wl, wr, gamma, c_l, c_r);
   T left_speed = (wl[L_VI] - c_l);
   T right_speed = (wr[L_VI] + c_r);
-  T sqrtrho_l = qsqrt(wl[L_D]);
-  T sqrtrho_r = qsqrt(wr[L_D]);
-  T inv_sqrtrho_tot = qdiv(T(1), sqrtrho_l + sqrtrho_r);
+  T sqrtrho_l, sqrtrho_r;
+  qsqrt2(wl[L_D], wr[L_D], sqrtrho_l, sqrtrho_r);
+  T inv_sqrtrho_tot = qrcp(sqrtrho_l + sqrtrho_r);
   T vi_roe = (sqrtrho_l * wl[L_VI] + sqrtrho_r * wr[L_VI]) * inv_sqrtrho_tot;
   T vj_roe = (sqrtrho_l * wl[L_VJ] + sqrtrho_r * wr[L_VJ]) * inv_sqrtrho_tot;
   T vk_roe = (sqrtrho_l * wl[L_VK] + sqrtrho_r * wr[L_VK]) * inv_sqrtrho_tot;
@@ -438,11 +524,12 @@ __device__ __forceinline__ void hlle_mhd(const T wl[8], const T wr[8],
                       ((wl[L_BJ] * wl[L_BJ]) + (wl[L_BK] * wl[L_BK])));
   ptot_r += T(0.5) * ((wr[L_BI] * wr[L_BI]) +
                       ((wr[L_BJ] * wr[L_BJ]) + (wr[L_BK] * wr[L_BK])));
-  T h_l = qdiv(cl[L_E] + ptot_l, wl[L_D]);
-  T h_r = qdiv(cr[L_E] + ptot_r, wr[L_D]);
+  T h_l = qdiv_inv(cl[L_E] + ptot_l, wl[L_D], qrcp(wl[L_D]));
+  T h_r = qdiv_inv(cr[L_E] + ptot_r, wr[L_D], qrcp(wr[L_D]));
   T h_roe = (sqrtrho_l * h_l + sqrtrho_r * h_r) * inv_sqrtrho_tot;
   // roe_cfast_
   T rho_roe = sqrtrho_l * sqrtrho_r;
+  T rho_roe_inv = qrcp(rho_roe);
   T bi_roe = wl[L_BI];
   T bj_roe = (sqrtrho_l * wr[L_BJ] + sqrtrho_r * wl[L_BJ]) * inv_sqrtrho_tot;
   T bk_roe = (sqrtrho_l * wr[L_BK] + sqrtrho_r * wl[L_BK]) * inv_sqrtrho_tot;
@@ -452,13 +539,15 @@ __device__ __forceinline__ void hlle_mhd(const T wl[8], const T wr[8],
   T dbk = wl[L_BK] - wr[L_BK];
   T x_prime =
       ((dbj * dbj + dbk * dbk) * T(0.5) * (gamma_prime - T(1)) * inv_sqrtrho_tot);
-  T y_prime = qdiv((gamma_prime - T(1)) * (wl[L_D] + wr[L_D]) * T(0.5), rho_roe);
+  T y_prime =
+      qdiv_inv((gamma_prime - T(1)) * (wl[L_D] + wr[L_D]) * T(0.5), rho_roe, rho_roe_inv);
   T tilde_a2 =
-      (gamma_prime * (h_roe - T(0.5) * v_roe2 - qdiv(b_roe2, rho_roe)) - x_prime);
-  T tilde_vai2 = qdiv(bi_roe * bi_roe, rho_roe);
-  T tilde_va2 = (tilde_vai2 + qdiv((gamma_prime - y_prime) *
-                                       (bj_roe * bj_roe + bk_roe * bk_roe),
-                                   rho_roe));
+      (gamma_prime * (h_roe - T(0.5) * v_roe2 - qdiv_inv(b_roe2, rho_roe, rho_roe_inv)) -
+       x_prime);
+  T tilde_vai2 = qdiv_inv(bi_roe * bi_roe, rho_roe, rho_roe_inv);
+  T tilde_va2 = (tilde_vai2 + qdiv_inv((gamma_prime - y_prime) *
+                                           (bj_roe * bj_roe + bk_roe * bk_roe),
+                                       rho_roe, rho_roe_inv));
   T s = tilde_a2 + tilde_va2;
   T c_roe = qsqrt(T(0.5) * (tilde_a2 + tilde_va2 +
                             qsqrt(s * s - T(4) * tilde_a2 * tilde_vai2)));
@@ -466,7 +555,7 @@ __device__ __forceinline__ void hlle_mhd(const T wl[8], const T wr[8],
   T bm = fmin(vi_roe - c_roe, left_speed);
   bp = fmax(bp, T(0));
   bm = fmin(bm, T(0));
-  T inv_speed_diff = qdiv(T(1), bp - bm);
+  T inv_speed_diff = qrcp(bp - bm);
 #pragma unroll
   for (int f = 0; f < 8; f++) {
     flux[f] = ((bp * fl[f] - bm * fr[f] + (cr[f] - cl[f]) * bp * bm) *
@@ -492,7 +581,7 @@ __device__ __forceinline__ void hllc(const T wl[5], const T wr[5], T gamma,
       c[s][H_D] = w[s][H_D];
       for (int i = 1; i < 5; i++) c[s][i] = w[s][i] * w[s][H_D];
       T density = w[s][H_D];
-      T internal_edens = qdiv(w[s][H_E], gamma - T(1));
+      T internal_edens = qdiv_inv(w[s][H_E], gamma - T(1), qrcp(gamma - T(1)));
       const T vi = w[s][H_VI], vj = w[s][H_VJ], vk = w[s][H_VK];
       const T kinetic =
           T(0.5) * density * ((vi * vi) + ((vj * vj) + (vk * vk)));
@@ -501,19 +590,21 @@ __device__ __forceinline__ void hllc(const T wl[5], const T wr[5], T gamma,
   }
   T cs_l, cs_r;
   {
-    T c_l = qsqrt(qdiv(gamma * pressure_l, wl[H_D]));
-    T c_r = qsqrt(qdiv(gamma * pressure_r, wr[H_D]));
+    const T inv_l = qrcp(wl[H_D]), inv_r = qrcp(wr[H_D]);
+    T c_l, c_r;
+    qsqrt2(qdiv_inv(gamma * pressure_l, wl[H_D], inv_l),
+           qdiv_inv(gamma * pressure_r, wr[H_D], inv_r), c_l, c_r);
     T left_speed = (wl[H_VI] - c_l);
     T right_speed = (wr[H_VI] + c_r);
-    T sqrtrho_l = qsqrt(wl[H_D]);
-    T sqrtrho_r = qsqrt(wr[H_D]);
-    T inv_sqrtrho_tot = qdiv(T(1), sqrtrho_l + sqrtrho_r);
+    T sqrtrho_l, sqrtrho_r;
+    qsqrt2(wl[H_D], wr[H_D], sqrtrho_l, sqrtrho_r);
+    T inv_sqrtrho_tot = qrcp(sqrtrho_l + sqrtrho_r);
     T vi_roe = (sqrtrho_l * wl[H_VI] + sqrtrho_r * wr[H_VI]) * inv_sqrtrho_tot;
     T vj_roe = (sqrtrho_l * wl[H_VJ] + sqrtrho_r * wr[H_VJ]) * inv_sqrtrho_tot;
     T vk_roe = (sqrtrho_l * wl[H_VK] + sqrtrho_r * wr[H_VK]) * inv_sqrtrho_tot;
     T v_roe2 = vi_roe * vi_roe + vj_roe * vj_roe + vk_roe * vk_roe;
-    T h_l = qdiv(cons_l[H_E] + pressure_l, wl[H_D]);
-    T h_r = qdiv(cons_r[H_E] + pressure_r, wr[H_D]);
+    T h_l = qdiv_inv(cons_l[H_E] + pressure_l, wl[H_D], inv_l);
+    T h_r = qdiv_inv(cons_r[H_E] + pressure_r, wr[H_D], inv_r);
     T h_roe = (sqrtrho_l * h_l + sqrtrho_r * h_r) * inv_sqrtrho_tot;
     T temp = h_roe - T(0.5) * v_roe2;
     T c_roe = qsqrt((gamma - T(1)) * dmax(temp, T(0)));
@@ -526,18 +617,19 @@ __device__ __forceinline__ void hllc(const T wl[5], const T wr[5], T gamma,
   T tr = (pressure_r - (cs_r - wr[H_VI]) * wr[H_D] * wr[H_VI]);
   T dl = wl[H_D] * (cs_l - wl[H_VI]);
   T dr = -wr[H_D] * (cs_r - wr[H_VI]);
-  T q1 = qdiv(T(1), dl + dr);
+  T q1 = qrcp(dl + dr);
   T cw = (tr - tl) * q1;
   T cp = (dl * tr + dr * tl) * q1;
   T sl, sr, sm;
-  if (cw >= T(0)) {
-    sl = qdiv(cw, cw - bm);
-    sr = T(0);
-    sm = qdiv(-bm, cw - bm);
-  } else {
-    sl = T(0);
-    sr = qdiv(-cw, bp - cw);
-    sm = qdiv(bp, bp - cw);
+  {
+    // the contact's side: its share of the outer flux, |cw| / (its distance
+    // to the outer speed), and the middle state's
+    const bool left = cw >= T(0);
+    const T den = left ? cw - bm : bp - cw, den_inv = qrcp(den);
+    const T share = qdiv_inv(left ? cw : -cw, den, den_inv);
+    sl = left ? share : T(0);
+    sr = left ? T(0) : share;
+    sm = qdiv_inv(left ? -bm : bp, den, den_inv);
   }
   if (vbar) *vbar = (sl * (wl[H_VI] - bm) + sr * (wr[H_VI] - bp));
   cp = dmax(cp, T(0));
