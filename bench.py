@@ -44,8 +44,15 @@ STEP_BYTES = {("mhd", "fp64"): STEP_BYTES_PER_ZONE_FP64, ("mhd", "mixed"): STEP_
 # Algorithmic bytes per cell of one flux launch: it must read the 11-word
 # state of the cell and write 7 flux components on each of its 3 low faces.
 FLUX_BYTES_PER_CELL = {0: (11 + 21) * 8.0, 1: 11 * 8.0 + 21 * 4.0, 2: (11 + 21) * 8.0}
+# Algorithmic bytes per cell of one marched final stage: it reads the 11-word
+# half-step state (FP64, or 8 FP32 primitives, the centre E and 3 faces), the
+# 5 conserved start-of-step words and 3 faces, and writes the 11-word state
+# and the pressure.
+MARCH_BYTES_PER_CELL = {0: (11 + 8 + 12) * 8.0, 1: 32.0 + (6 + 8 + 12) * 8.0,
+                        2: (11 + 8 + 12) * 8.0}
 # hydro: read 5 words, write 5 fluxes on 3 faces; step: 25 words per zone
 FLUX_BYTES_PER_CELL_HD = {0: (5 + 15) * 8.0, 1: 5 * 8.0 + 15 * 4.0, 2: (5 + 15) * 8.0}
+MARCH_BYTES_PER_CELL_HD = {0: (5 + 5 + 6) * 8.0, 1: 20.0 + 11 * 8.0, 2: (5 + 5 + 6) * 8.0}
 STEP_BYTES_PER_ZONE_HD = 200.0
 WORKLOADS = ["orszag_tang", "fast_wave", "batched_amr", "turbulence", "smr_flux_correct",
              "kelvin_helmholtz", "output", "drop_in"]
@@ -168,21 +175,24 @@ def copy_bandwidth(reps=5):
 # final cell update)
 STEP_LAUNCHES = {"k_refresh": 1, "k_flux_nn": 1, "k_flux_plm": 1, "k_edge": 2,
                  "k_faces": 2, "k_cells": 2}
+# ... with the stages marched
+MARCH_LAUNCHES = {"k_refresh": 1, "k_march_nn": 1, "k_march_plm": 1, "k_shell": 1}
 
 
-def measured_step_traffic(workload, mhd=True):
+def measured_step_traffic(workload, mhd=True, march=False):
     """HBM bytes of one step from the committed counter summary: its
     step_traffic line, else the sum of the step's launches, or None when a
-    kernel of the step has no entry."""
+    kernel of the step has no entry.  march: the marched stages' step."""
     path = os.path.join(ROOT, "profiles", "hbm_traffic.txt")
     if os.path.exists(path):
         with open(path) as f:
             for line in f:
                 p = line.split()
-                if len(p) == 3 and p[0] == "step_traffic" and p[1] == workload:
+                if len(p) == 3 and p[1] == workload and \
+                        p[0] == ("step_traffic_march" if march else "step_traffic"):
                     return float(p[2])
     tot = 0.0
-    for k, n in STEP_LAUNCHES.items():
+    for k, n in (MARCH_LAUNCHES if march else STEP_LAUNCHES).items():
         if not mhd and k in ("k_edge", "k_faces"):
             continue
         t = measured_traffic(k, workload)
@@ -192,7 +202,14 @@ def measured_step_traffic(workload, mhd=True):
     return tot
 
 
-def step_roofline(prec_name, zones, ms_per_step, gpu_ms_per_step, workload, mhd=True):
+def dominant_kernel(prof):
+    """The kernel of the reconstructing stage's fluxes: the marched stage, or
+    the flux launch of the separate ones."""
+    return "k_march_plm" if "k_march_plm" in prof else "k_flux_plm"
+
+
+def step_roofline(prec_name, zones, ms_per_step, gpu_ms_per_step, workload, mhd=True,
+                  march=False):
     """The step against the HBM roofline as the metric defines it: the
     algorithmic bytes of a fully fused step (440 B per MHD zone-update in
     FP64) over the measured wall time per step."""
@@ -200,7 +217,7 @@ def step_roofline(prec_name, zones, ms_per_step, gpu_ms_per_step, workload, mhd=
     achieved = bpz * zones / (ms_per_step * 1e-3) / 1e9
     return {"bound": "hbm", "scope": "step", "achieved": achieved, "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-            "traffic": measured_step_traffic(workload, mhd),
+            "traffic": measured_step_traffic(workload, mhd, march),
             "bytes_per_zone": bpz, "algorithmic_bytes_per_step": bpz * zones,
             "kernel_ms_per_step": gpu_ms_per_step,
             "achieved_over_kernel_time": bpz * zones / (gpu_ms_per_step * 1e-3) / 1e9}
@@ -342,7 +359,9 @@ def timed_run(precision, n, steps, warmup, dual_energy=False, launch_mask=-1, ke
     of the autotuner's."""
     prec = PRECISIONS[precision]
     if launch_mask >= 0:
+        # an order of the separate launches
         os.environ["ENZOE_XCD_REMAP"] = str(launch_mask)
+        structure = max(structure, 0)
     method = ev.VlctMethod(mhd=True, riemann="hlld", reconstruct="plm",
                            theta=2.0, courant=0.4, gamma=5.0 / 3.0,
                            precision=prec,
@@ -376,11 +395,13 @@ def timed_run(precision, n, steps, warmup, dual_energy=False, launch_mask=-1, ke
     del grid, method
     zones = n ** 3
     m = n + 6
-    # dominant kernel: the flux kernel of the full (PLM) stage
-    dom = "k_flux_plm"
+    # dominant kernel: the full (PLM) stage, or its flux kernel
+    dom = dominant_kernel(prof)
     dom_ms = prof.get(dom, (float("nan"), 0))[0]
-    cells = (m - 4) ** 3  # flux box of the PLM stage: [2, m-2)^3
-    dom_bytes = FLUX_BYTES_PER_CELL[prec] * cells
+    if dom == "k_march_plm":
+        dom_bytes = MARCH_BYTES_PER_CELL[prec] * zones
+    else:  # flux box of the PLM stage: [2, m-2)^3
+        dom_bytes = FLUX_BYTES_PER_CELL[prec] * (m - 4) ** 3
     gpu_step_ms = sum(v[0] * v[1] for v in prof.values()) / steps
     return {"precision": precision, "value": zones * steps / el,
             "ms_per_step": el * 1e3 / steps, "prof": prof, "dom": dom,
@@ -394,12 +415,15 @@ def timed_run(precision, n, steps, warmup, dual_energy=False, launch_mask=-1, ke
 
 
 def _roofline(prof, steps, cells_per_step, prec, mhd, workload):
-    """Dominant-kernel roofline: algorithmic flux-kernel bytes of a step
-    over the flux kernel's HIP-event time in that step."""
-    dom = "k_flux_plm"
+    """Dominant-kernel roofline: algorithmic bytes of a step of the marched
+    final stage, or of the flux kernel, over the kernel's HIP-event time in
+    that step."""
+    dom = dominant_kernel(prof)
     avg_ms, count = prof.get(dom, (float("nan"), 0))
     per_step_ms = avg_ms * count / steps
     table = FLUX_BYTES_PER_CELL if mhd else FLUX_BYTES_PER_CELL_HD
+    if dom == "k_march_plm":
+        table = MARCH_BYTES_PER_CELL if mhd else MARCH_BYTES_PER_CELL_HD
     nbytes = table[prec] * cells_per_step
     achieved = nbytes / (per_step_ms * 1e-3) / 1e9
     return {"bound": "hbm", "kernel": dom, "achieved": achieved,
@@ -415,7 +439,7 @@ def _both_rooflines(prof, steps, elapsed, zones_per_step, cells_per_step, precis
     prec = ev.ENZOE_PREC_DOUBLE if precision == "fp64" else ev.ENZOE_PREC_MIXED
     gpu_ms = sum(v[0] * v[1] for v in prof.values()) / steps
     return dict(step_roofline(precision, zones_per_step, elapsed * 1e3 / steps, gpu_ms,
-                              workload, mhd),
+                              workload, mhd, "k_march_plm" in prof),
                 dominant_kernel=_roofline(prof, steps, cells_per_step, prec, mhd, workload))
 
 
@@ -904,7 +928,7 @@ def batched_mixed_leg(steps, cpu=True):
                           "launch_mask": mask,
                           "kernels_ms": {k: round(v[0], 4) for k, v in sorted(prof.items())},
                           "roofline": step_roofline(precision, zones, el * 1e3 / steps, gpu_ms,
-                                                    wl)}
+                                                    wl, march="k_march_plm" in prof)}
     per, mag = grids["mixed"].method.state_l1(grids["mixed"].blocks, grids["fp64"].blocks)
     del grids
     out = {"workload": "turbulence_512x64^3_mach5_beta0.1_vlct_plm_hlld", "steps": steps,
@@ -986,7 +1010,8 @@ def main():
         # the step against the roofline as the metric defines it (440 B per
         # zone-update, fully fused); the dominant kernel's own figure beside it
         "roofline": dict(step_roofline(a.precision, a.n ** 3, r["ms_per_step"],
-                                       r["gpu_step_ms"], r["workload"]),
+                                       r["gpu_step_ms"], r["workload"],
+                                       march="k_march_plm" in r["prof"]),
                          dominant_kernel={
                              "kernel": r["dom"],
                              "achieved": r["achieved"],
@@ -1011,7 +1036,8 @@ def main():
             "mixed_kernels_ms": {k: round(v[0], 4)
                                  for k, v in sorted(mixed["prof"].items())},
             "mixed_roofline": step_roofline("mixed", a.n ** 3, mixed["ms_per_step"],
-                                            mixed["gpu_step_ms"], mixed["workload"]),
+                                            mixed["gpu_step_ms"], mixed["workload"],
+                                            march="k_march_plm" in mixed["prof"]),
             "mixed_dominant_GBs": mixed["achieved"],
             "mixed_traffic": measured_traffic(mixed["dom"], mixed["workload"]),
         }

@@ -844,6 +844,8 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
     for (int mask = 0; mask < 16; mask++)
       if (v == 0 || (mask & (v == 4 ? 4 : 6)) == 0) cand.push_back({v, mask});
   }
+  // the marched stages (setting "auto" of both structure and flux launch)
+  if (ct_fused && fixed < 0 && m->flux_shape < 0) cand.push_back({MARCH_STRUCTURE, 0});
   if (persistent_ok(m) && (fixed == -1 || fixed == 5))
     if (int rc2 = ensure_barrier(m)) rc = rc2;
   // the time of one step of the sample under the forced settings: a timed
@@ -920,7 +922,7 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
   // workgroups for small blocks; z pencils for the nearest-neighbour
   // stage), for the chosen structure, order and rows
   int best_shape = 0;
-  if (best_ctu != 5 && m->flux_shape < 0 && rc == ENZOE_OK) {
+  if (best_ctu < 5 && m->flux_shape < 0 && rc == ENZOE_OK) {
     m->force_mask = best;
     m->force_ctu = best_ctu;
     m->force_rows = best_rows;
@@ -961,7 +963,7 @@ int enzoe_vlct_launch_choice(enzoe_vlct_t m, int mx, int my, int mz, int *mask, 
   if (fused_ct) {
     const int v = ctu_variant(m, mx, my, mz);
     *fused_ct = (v == 5) ? (persistent_ok(m) ? 5 : 0)
-                         : ((m->mhd && ctu_possible(m)) ? v : 0);
+                         : ((m->mhd && ctu_possible(m) && v < 5) ? v : 0);
   }
   return ENZOE_OK;
 }

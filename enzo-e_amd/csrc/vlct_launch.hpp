@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cstring>
 #include <map>
 #include <string>
@@ -17,6 +18,7 @@
 
 #include "../../include/enzoe_vlct.h"
 #include "vlct_kernels.hpp"
+#include "vlct_march.hpp"
 
 namespace enzoe {
 
@@ -170,6 +172,10 @@ inline int ctu_variant(const enzoe_vlct_method *m, int mx, int my, int mz) {
   auto it = m->tuned_ctu.find(shape_key(mx, my, mz));
   return it != m->tuned_ctu.end() ? it->second : 0;
 }
+
+// ... and, chosen by march_ok and not by enzoe_vlct_set_fused_ct, the marched
+// stages
+constexpr int MARCH_STRUCTURE = 6;
 
 // The fused CT update needs the two stages of the VL scheme (its final
 // stage reads the first stage's copy of the start-of-step faces); the
@@ -572,6 +578,128 @@ struct StoreArgs {
   double *const *d_fdtab;
 };
 
+// ------------------------------------------------------- marched stages
+
+// Whether the two stages of nb blocks of this shape run marched (k_march):
+// constrained transport in the VL scheme, fields whose byte offsets fit 32
+// bits, no debug counts (the marched tiles solve the faces of their rings
+// more than once), and no structure or flux-launch shape asked for; then the
+// autotuner's choice for the shape, or else from 2^18 active cells on.
+// Below that the launches are bound by latency, a plane after the other
+// costs more than it saves, and the separate launches win (cycle of 4 blocks
+// of 32^3: 158 against 177 us, one of 48^3: 137 against 144; equal at 8 of
+// 32^3 and one of 64^3: 230, 202; above, 48^3 x 4: 293 against 264, 64^3 x
+// 16: 2180 against 1545).
+inline bool march_ok(const enzoe_vlct_method *m, int mx, int my, int mz, int ghost, int nb) {
+  if (!ctu_possible(m) || m->nstages != 2 || m->d_dbg ||
+      8ull * (mx + 1) * (my + 1) * (mz + 1) >= (1ull << 32))
+    return false;
+  if (m->force_ctu >= 0) return m->force_ctu == MARCH_STRUCTURE;
+  if (m->ctu >= 0 || m->flux_shape >= 0) return false;
+  auto it = m->tuned_ctu.find(shape_key(mx, my, mz));
+  if (it != m->tuned_ctu.end()) return it->second == MARCH_STRUCTURE;
+  const long active = (long)(mx - 2 * ghost) * (my - 2 * ghost) * (mz - 2 * ghost);
+  return active * nb >= (1L << 18);
+}
+
+// Compute units of the current device, cached per device; 256 if unknown.
+inline int device_cus() {
+  static std::atomic<int> cus[16];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return 256;
+  int c = cus[dev].load(std::memory_order_relaxed);
+  if (c == 0) {
+    if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        c <= 0)
+      c = 256;
+    cus[dev].store(c, std::memory_order_relaxed);
+  }
+  return c;
+}
+
+// The tiling of one marched stage over nb blocks with NT-thread workgroups:
+// the tile that covers the update box of a plane with the fewest
+// workgroups (ties: the longer rows), and the share of a workgroup such that
+// the launch fills the device once.  cost: the launch's time in units of one
+// plane of a tile with the device full; a piece of work costs 3 planes more
+// than it updates (the flux work of the planes around it, and its start).
+template <int NT>
+MarchParams march_tiling(int mx, int my, int mz, int cs, int nb, int cus, double &cost) {
+  const int nx = mx - 2 * (cs + 1), ny = my - 2 * (cs + 1), nz = mz - 2 * (cs + 1);
+  MarchParams p{};
+  long tiles = -1;
+  for (int w2 = 10; w2 <= NT / 9; w2++) {
+    if (w2 > nx + 2 && tiles >= 0) break;
+    int h2 = std::min(NT / w2, ny + 2);
+    while ((w2 + 2) * (h2 + 2) > march_plane_cells(NT)) h2--;
+    const int ntx = (nx + w2 - 3) / (w2 - 2), nty = (ny + h2 - 3) / (h2 - 2);
+    if (tiles < 0 || (long)ntx * nty <= tiles) {
+      tiles = (long)ntx * nty;
+      p.w2 = w2;
+      p.h2 = h2;
+      p.ntx = ntx;
+      p.nty = nty;
+    }
+  }
+  p.nz = nz;
+  const long slots = (long)cus * (512 / NT);
+  // even shares over the whole launch (the rings then come from memory
+  // instead of the L2: about an eighth more time a plane)
+  p.zseg = nz;
+  p.nseg = 1;
+  p.total = tiles * nz * nb;
+  p.share = (int)std::min<long>(std::max<long>((p.total + slots - 1) / slots, 4), INT_MAX);
+  cost = 1.12 * (p.share + 3.0 * (1.0 + (double)p.share / nz));
+  // or a segment of a tile to a workgroup, in rounds over the device
+  for (int seg = 1; seg <= std::max(1, nz / 4); seg++) {
+    const int zseg = (nz + seg - 1) / seg;
+    const long wgs = tiles * seg * nb;
+    const double c = (double)((wgs + slots - 1) / slots) * (zseg + 3);
+    if (c < cost) {
+      cost = c;
+      p.zseg = p.share = zseg;
+      p.nseg = (nz + zseg - 1) / zseg;
+      p.total = tiles * p.nseg * nb * (long)zseg;
+    }
+  }
+  return p;
+}
+
+template <typename T, int RECON, int RIEMANN, bool DE, bool HALF, int NT>
+void launch_march_nt(const BlockDesc<T> *d, const MarchParams &mp, const StageParams &sp,
+                     hipStream_t s) {
+  const unsigned wgs = (unsigned)((mp.total + mp.share - 1) / mp.share);
+  hipLaunchKernelGGL((k_march<T, RECON, RIEMANN, DE, HALF, NT>), dim3((wgs + 7u) & ~7u),
+                     dim3(NT), 0, s, d, sp, mp);
+}
+// One marched stage: 512-thread tiles, one a CU, or 256-thread ones, two a
+// CU, whichever covers the blocks' planes in less time (the smaller tile
+// repeats more of its ring but fits small blocks better).
+template <typename T, int RECON, int RIEMANN, bool DE, bool HALF>
+void launch_march(const BlockDesc<T> *d, int nb, int mx, int my, int mz, const StageParams &sp,
+                  hipStream_t s) {
+  const int cus = device_cus();
+  double big, small;
+  const MarchParams p5 = march_tiling<512>(mx, my, mz, sp.cur_stale, nb, cus, big);
+  const MarchParams p2 = march_tiling<256>(mx, my, mz, sp.cur_stale, nb, cus, small);
+  if (big <= small)
+    launch_march_nt<T, RECON, RIEMANN, DE, HALF, 512>(d, p5, sp, s);
+  else
+    launch_march_nt<T, RECON, RIEMANN, DE, HALF, 256>(d, p2, sp, s);
+}
+template <typename T, int RIEMANN, bool DE>
+void dispatch_march(int recon, const BlockDesc<T> *d, int nb, int mx, int my, int mz,
+                    const StageParams &sp, hipStream_t s) {
+  if (sp.stage == 0)
+    launch_march<T, RC_NN, RIEMANN, DE, false>(d, nb, mx, my, mz, sp, s);
+  else if (recon == RC_NN)
+    launch_march<T, RC_NN, RIEMANN, DE, true>(d, nb, mx, my, mz, sp, s);
+  else if (recon == RC_PLM)
+    launch_march<T, RC_PLM, RIEMANN, DE, true>(d, nb, mx, my, mz, sp, s);
+  else
+    launch_march<T, RC_PLM_ATHENA, RIEMANN, DE, true>(d, nb, mx, my, mz, sp, s);
+}
+
 // Bytes of the chunk scratch pool: the larger of 4 GiB and a third of the
 // free device memory, at most 16 GiB (taken once per method).
 inline size_t scratch_budget(enzoe_vlct_method *m) {
@@ -594,6 +722,7 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
                   hipStream_t s, const StoreArgs *st, unsigned long long *cfl,
                   bool timers) {
   const int mx = blocks[0].mx, my = blocks[0].my, mz = blocks[0].mz;
+  const bool march = march_ok(m, mx, my, mz, blocks[0].ghost, std::min(n, chunk));
   for (int c0 = 0; c0 < n; c0 += chunk) {
     const int c1 = std::min(n, c0 + chunk);
     const int nb = c1 - c0;
@@ -627,6 +756,27 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
       // with the fused CFL the final update's launch covers the block
       const int lo = sp.cfl ? 0 : (is_final ? cs : cs + 1);
       const int structure = ctu_variant(m, mx, my, mz);
+      if constexpr (MHD) {
+        if (march) {
+          {
+            KernelTimer kt(s, recon == RC_NN ? "k_march_nn" : "k_march_plm", timers);
+            if (m->riemann == RS_HLLD)
+              dispatch_march<FluxT, RS_HLLD, DE>(recon, d, nb, mx, my, mz, sp, s);
+            else
+              dispatch_march<FluxT, RS_HLLE, DE>(recon, d, nb, mx, my, mz, sp, s);
+          }
+          if (is_final) {
+            // the cells around the update: ring centre B, CFL, pressure
+            const int blo = sp.cfl ? 0 : cs;
+            const long shell = cube(mx, my, mz, blo, blo) - cube(mx, my, mz, cs + 1, cs + 1);
+            KernelTimer kt(s, "k_shell", timers);
+            hipLaunchKernelGGL((k_shell<FluxT, MHD, DE>), dim3(nblk(shell, 256), nb), dim3(256),
+                               0, s, d, sp);
+          }
+          stale += total_staling(recon);
+          continue;
+        }
+      }
       if constexpr (!DE) {
         if (structure == 5 && persistent_ok(m) && m->d_bar) {
           // the stage's four kernels as one persistent launch

@@ -1,0 +1,174 @@
+"""The marched stages (k_march) against the separate launches: the same bits
+in FP64 for every solver, limiter and precision mode, over block shapes at
+the edges of the marched tiles, with per-block time steps, device-driven and
+captured cycles, and states that hold NaN and huge values."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+G = 3
+
+
+def _ev():
+    import enzoe_vlct as ev
+    return ev
+
+
+def _state(n, seed, dual=False):
+    """A rough random state of one block (independent values in neighbouring
+    cells: every branch of the solvers is taken somewhere)."""
+    rng = np.random.default_rng(seed)
+    m = [x + 2 * G for x in n[::-1]]
+    a = {"density": np.exp(0.4 * rng.standard_normal(m))}
+    for c in "xyz":
+        a["velocity_" + c] = 0.7 * rng.standard_normal(m)
+    for ax, c in zip((2, 1, 0), "xyz"):
+        shp = list(m)
+        shp[ax] += 1
+        f = 0.5 * rng.standard_normal(shp) + (0.4 if c == "x" else 0.0)
+        a["bfieldi_" + c] = f
+        a["bfield_" + c] = 0.5 * (np.take(f, range(1, shp[ax]), ax)
+                                  + np.take(f, range(shp[ax] - 1), ax))
+    e = 1.5 * np.exp(0.3 * rng.standard_normal(m)) / a["density"]
+    a["total_energy"] = e + 0.5 * sum(a["velocity_" + c] ** 2 for c in "xyz") \
+        + 0.5 * sum(a["bfield_" + c] ** 2 for c in "xyz") / a["density"]
+    if dual:
+        a["internal_energy"] = e
+    return a
+
+
+def _blocks(ev, n, states, count, dual=False):
+    out = []
+    for i in range(count):
+        b = ev.DeviceBlock(n[0] + 2 * G, n[1] + 2 * G, n[2] + 2 * G, G,
+                           (1.0 / n[0], 1.1 / n[1], 0.9 / n[2]), mhd=True, dual_energy=dual)
+        b.upload(states[i % len(states)])
+        out.append(b)
+    return out
+
+
+def _equal(xs, ys):
+    for i, (x, y) in enumerate(zip(xs, ys)):
+        a, b = x.download(), y.download()
+        for k in a:
+            assert np.array_equal(a[k], b[k], equal_nan=True), (i, k)
+
+
+# (block, count): from 2^18 active cells on the default is the marched launch;
+# sides from one partial tile to several, of both tile sizes
+SHAPES = [((32, 32, 32), 8), ((9, 8, 7), 521), ((13, 41, 29), 17), ((130, 37, 57), 1),
+          ((70, 12, 50), 7), ((16, 16, 16), 64)]
+
+
+@pytest.mark.parametrize("riemann,recon,dual", [("hlld", "plm", False), ("hlld", "nn", False),
+                                                ("hlle", "plm_athena", False),
+                                                ("hlld", "plm", True), ("hlle", "nn", True)])
+@pytest.mark.parametrize("n,count", SHAPES)
+def test_marched_stages_equal_the_separate_launches(n, count, riemann, recon, dual):
+    """Two steps with per-block dt (one block's step zero), the second with
+    the CFL minimum fused: every field, ghost zones included, and the next
+    dt equal bit for bit."""
+    ev = _ev()
+    states = [_state(n, 100 + s, dual) for s in range(min(3, count))]
+    dts = [2e-4 * (1 + (i % 4)) for i in range(count)]
+    if count > 1:
+        dts[1] = 0.0
+    out, nxt = [], []
+    for structure in (-1, 0):
+        m = ev.VlctMethod(mhd=True, riemann=riemann, reconstruct=recon, theta=2.0, courant=0.4,
+                          dual_energy_eta=0.001 if dual else None)
+        m.set_fused_ct(structure)
+        blocks = _blocks(ev, n, states, count, dual)
+        ev.profiling(True)
+        m.compute_dt(blocks, dts)
+        nxt.append(m.compute_timestep(blocks, 1e-4))
+        names = ev.profile_report()
+        ev.profiling(False)
+        assert ("k_march_nn" in names) == (structure == -1)
+        out.append(blocks)
+    assert nxt[0] == nxt[1]
+    _equal(out[0], out[1])
+
+
+def test_marched_stages_spread_nan_and_huge_values_as_the_separate_launches():
+    """Cells with NaN, infinities and magnitudes whose differences overflow
+    take the limiter's general form: the same cells end non-finite, the
+    others keep the same bits."""
+    ev = _ev()
+    n = (40, 36, 48)
+    states = [_state(n, 7 + s) for s in range(4)]
+    for s, (k, j, i) in enumerate([(9, 8, 7), (G, G, G), (30, 20, 44), (50, 41, 3)]):
+        f = states[s]
+        f["velocity_x"][k, j, i] = np.nan
+        f["bfield_y"][k - 2, j, i] = np.inf
+        f["velocity_z"][(k + 9) % 54, j, i] = 1.5e308
+        f["velocity_z"][(k + 10) % 54, j, i] = -1.5e308
+    out = []
+    for structure in (-1, 0):
+        m = ev.VlctMethod(mhd=True, riemann="hlld", reconstruct="plm", theta=2.0, courant=0.4)
+        m.set_fused_ct(structure)
+        blocks = _blocks(ev, n, states, 4)
+        m.compute(blocks, 1e-4)
+        m.compute_timestep(blocks, 1e-4)
+        out.append(blocks)
+    _equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("precision", ["mixed", "fma"])
+def test_marched_stages_of_the_contracted_builds_are_as_close_to_fp64(precision):
+    """The mixed and contracted builds may fuse their flux arithmetic
+    otherwise in another kernel: per field the marched result's L1 distance
+    to the FP64 one is at most twice the separate launches' (both are sums
+    of independent roundings of the same size)."""
+    ev = _ev()
+    n, count = (45, 33, 30), 6
+    states = [_state(n, 50 + s) for s in range(3)]
+    prec = {"mixed": ev.ENZOE_PREC_MIXED, "fma": ev.ENZOE_PREC_DOUBLE_FMA}[precision]
+    res = []
+    for p, structure in ((ev.ENZOE_PREC_DOUBLE, 0), (prec, 0), (prec, -1)):
+        m = ev.VlctMethod(mhd=True, riemann="hlld", reconstruct="plm", theta=1.5, courant=0.4,
+                          precision=p)
+        m.set_fused_ct(structure)
+        blocks = _blocks(ev, n, states, count)
+        for _ in range(2):
+            m.compute(blocks, 2e-4)
+        res.append([b.download() for b in blocks])
+    for k in ("density", "velocity_x", "velocity_y", "velocity_z", "total_energy",
+              "bfieldi_x", "bfieldi_y", "bfieldi_z"):
+        ref = sum(np.abs(b[k]).sum() for b in res[0])
+        d = [sum(np.abs(a[k] - b[k]).sum() for a, b in zip(r, res[0])) / ref for r in res[1:]]
+        assert d[1] <= 2.0 * d[0] + 1e-17, (k, d)
+
+
+def test_marched_cycles_on_the_device_and_from_a_graph_equal_host_driven_ones():
+    """A 64^3 block: cycles enqueued without a graph, and graph replays with
+    eager work of the same method between them, equal host-driven cycles."""
+    ev = _ev()
+    n = (64, 64, 64)
+    state = _state(n, 3)
+    grids = []
+    for _ in range(3):
+        m = ev.VlctMethod(mhd=True, riemann="hlld", reconstruct="plm", theta=2.0, courant=0.3)
+        g = ev.DeviceGrid(m, (1, 1, 1), n, [(1.0 / 64,) * 3])
+        g.upload_from([state])
+        grids.append(g)
+    host, dev, graph = grids
+    t_stop, t = 1.0, 0.0
+    for _ in range(6):
+        t += host.cycle(t, t_stop)
+    dev.evolve_device(0.0, t_stop, ncycles=6, max_calls=1)
+    cg = graph.graph(0.0, t_stop, 2)
+    scratch = _blocks(ev, (40, 40, 40), [_state((40, 40, 40), 5)], 5)
+    for _ in range(3):
+        cg.launch()
+        graph.method.compute(scratch, 1e-4)
+        ev.synchronize()
+    assert cg.time() == t
+    cg.destroy()
+    s = (slice(G, -G),) * 3
+    for other in (dev, graph):
+        a, b = host.blocks[0].download(), other.blocks[0].download()
+        for k in a:
+            if k != "pressure":
+                assert np.array_equal(a[k][s], b[k][s]), k
