@@ -845,7 +845,7 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
       if (v == 0 || (mask & (v == 4 ? 4 : 6)) == 0) cand.push_back({v, mask});
   }
   // the marched stages (setting "auto" of both structure and flux launch)
-  if (ct_fused && fixed < 0 && m->flux_shape < 0) cand.push_back({MARCH_STRUCTURE, 0});
+  if (m->nstages == 2 && fixed < 0 && m->flux_shape < 0) cand.push_back({MARCH_STRUCTURE, 0});
   if (persistent_ok(m) && (fixed == -1 || fixed == 5))
     if (int rc2 = ensure_barrier(m)) rc = rc2;
   // the time of one step of the sample under the forced settings: a timed

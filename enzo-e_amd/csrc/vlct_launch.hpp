@@ -580,18 +580,20 @@ struct StoreArgs {
 
 // ------------------------------------------------------- marched stages
 
-// Whether the two stages of nb blocks of this shape run marched (k_march):
-// constrained transport in the VL scheme, fields whose byte offsets fit 32
-// bits, no debug counts (the marched tiles solve the faces of their rings
-// more than once), and no structure or flux-launch shape asked for; then the
-// autotuner's choice for the shape, or else from 2^18 active cells on.
-// Below that the launches are bound by latency, a plane after the other
-// costs more than it saves, and the separate launches win (cycle of 4 blocks
-// of 32^3: 158 against 177 us, one of 48^3: 137 against 144; equal at 8 of
-// 32^3 and one of 64^3: 230, 202; above, 48^3 x 4: 293 against 264, 64^3 x
-// 16: 2180 against 1545).
+// Whether the two stages of nb blocks of this shape run marched (k_march,
+// k_march_hd): the VL scheme, fields whose byte offsets fit 32 bits, no debug
+// counts (the marched tiles solve the faces of their rings more than once),
+// and no structure or flux-launch shape asked for; then the autotuner's
+// choice for the shape, or else from 2^18 active cells on (FP64 hydro:
+// 3 2^17).  Below that the launches are bound by latency, a plane after
+// the other costs more than it saves, and the separate launches win.  Cycle
+// in us, separate and marched -- MHD: 4 blocks of 32^3 158, 177; one of 48^3
+// 137, 144; 8 of 32^3 229, 230; one of 64^3 202, 202; 4 of 48^3 293, 268; 16
+// of 64^3 2180, 1545.  FP64 hydro: 8 of 32^3 123, 140; one of 64^3 106, 114;
+// 16 of 32^3 201, 163.  Mixed hydro: 4 of 32^3 70, 75; one of 64^3 77, 76;
+// 64 of 16^3 125, 107.
 inline bool march_ok(const enzoe_vlct_method *m, int mx, int my, int mz, int ghost, int nb) {
-  if (!ctu_possible(m) || m->nstages != 2 || m->d_dbg ||
+  if ((m->mhd && !ctu_possible(m)) || m->nstages != 2 || m->d_dbg ||
       8ull * (mx + 1) * (my + 1) * (mz + 1) >= (1ull << 32))
     return false;
   if (m->force_ctu >= 0) return m->force_ctu == MARCH_STRUCTURE;
@@ -599,7 +601,8 @@ inline bool march_ok(const enzoe_vlct_method *m, int mx, int my, int mz, int gho
   auto it = m->tuned_ctu.find(shape_key(mx, my, mz));
   if (it != m->tuned_ctu.end()) return it->second == MARCH_STRUCTURE;
   const long active = (long)(mx - 2 * ghost) * (my - 2 * ghost) * (mz - 2 * ghost);
-  return active * nb >= (1L << 18);
+  const bool light = m->mhd || m->precision == ENZOE_PREC_MIXED;
+  return active * nb >= (light ? 1L << 18 : 3L << 17);
 }
 
 // Compute units of the current device, cached per device; 256 if unknown.
@@ -617,14 +620,15 @@ inline int device_cus() {
   return c;
 }
 
-// The tiling of one marched stage over nb blocks with NT-thread workgroups:
-// the tile that covers the update box of a plane with the fewest
-// workgroups (ties: the longer rows), and the share of a workgroup such that
-// the launch fills the device once.  cost: the launch's time in units of one
-// plane of a tile with the device full; a piece of work costs 3 planes more
+// The tiling of one marched stage over nb blocks with NT-thread workgroups,
+// PER of them on a CU: the tile that covers the update box of a plane with
+// the fewest workgroups (ties: the longer rows), and the workgroups' shares
+// of the planes.  cost: the launch's time in units of one plane of 512
+// threads a CU with the device full; a piece of work costs 3 planes more
 // than it updates (the flux work of the planes around it, and its start).
-template <int NT>
+template <int NT, int PER>
 MarchParams march_tiling(int mx, int my, int mz, int cs, int nb, int cus, double &cost) {
+  constexpr double UNIT = NT * PER / 512.0;
   const int nx = mx - 2 * (cs + 1), ny = my - 2 * (cs + 1), nz = mz - 2 * (cs + 1);
   MarchParams p{};
   long tiles = -1;
@@ -642,19 +646,19 @@ MarchParams march_tiling(int mx, int my, int mz, int cs, int nb, int cus, double
     }
   }
   p.nz = nz;
-  const long slots = (long)cus * (512 / NT);
+  const long slots = (long)cus * PER;
   // even shares over the whole launch (the rings then come from memory
   // instead of the L2: about an eighth more time a plane)
   p.zseg = nz;
   p.nseg = 1;
   p.total = tiles * nz * nb;
   p.share = (int)std::min<long>(std::max<long>((p.total + slots - 1) / slots, 4), INT_MAX);
-  cost = 1.12 * (p.share + 3.0 * (1.0 + (double)p.share / nz));
+  cost = 1.12 * UNIT * (p.share + 3.0 * (1.0 + (double)p.share / nz));
   // or a segment of a tile to a workgroup, in rounds over the device
   for (int seg = 1; seg <= std::max(1, nz / 4); seg++) {
     const int zseg = (nz + seg - 1) / seg;
     const long wgs = tiles * seg * nb;
-    const double c = (double)((wgs + slots - 1) / slots) * (zseg + 3);
+    const double c = UNIT * (double)((wgs + slots - 1) / slots) * (zseg + 3);
     if (c < cost) {
       cost = c;
       p.zseg = p.share = zseg;
@@ -680,8 +684,8 @@ void launch_march(const BlockDesc<T> *d, int nb, int mx, int my, int mz, const S
                   hipStream_t s) {
   const int cus = device_cus();
   double big, small;
-  const MarchParams p5 = march_tiling<512>(mx, my, mz, sp.cur_stale, nb, cus, big);
-  const MarchParams p2 = march_tiling<256>(mx, my, mz, sp.cur_stale, nb, cus, small);
+  const MarchParams p5 = march_tiling<512, 1>(mx, my, mz, sp.cur_stale, nb, cus, big);
+  const MarchParams p2 = march_tiling<256, 2>(mx, my, mz, sp.cur_stale, nb, cus, small);
   if (big <= small)
     launch_march_nt<T, RECON, RIEMANN, DE, HALF, 512>(d, p5, sp, s);
   else
@@ -698,6 +702,63 @@ void dispatch_march(int recon, const BlockDesc<T> *d, int nb, int mx, int my, in
     launch_march<T, RC_PLM, RIEMANN, DE, true>(d, nb, mx, my, mz, sp, s);
   else
     launch_march<T, RC_PLM_ATHENA, RIEMANN, DE, true>(d, nb, mx, my, mz, sp, s);
+}
+
+template <typename T, int RECON, bool DE, bool HALF, int NT, int PER>
+void launch_march_hd_nt(const BlockDesc<T> *d, const MarchParams &mp, const StageParams &sp,
+                        hipStream_t s) {
+  const unsigned wgs = (unsigned)((mp.total + mp.share - 1) / mp.share);
+  hipLaunchKernelGGL((k_march_hd<T, RECON, DE, HALF, NT, NT * PER / 256>),
+                     dim3((wgs + 7u) & ~7u), dim3(NT), 0, s, d, sp, mp);
+}
+// The tiles of the hydrodynamic march by what its registers allow: 167 in the
+// FP64 reconstructing stage (three waves a SIMD: one workgroup of 768 on a
+// CU), 124 in FP64 nearest neighbour and the mixed reconstructing one (four:
+// two of 512), 81 in mixed nearest neighbour (six: three of 512); with
+// dual energy the reconstructing stage takes 192 (two: one of 512).  Beside
+// them 256-thread tiles, as many on a CU.  8 blocks of 128^3, FP64, PLM
+// stage: 1.17 ms with 768, 1.21 with 512, 1.31 with 256, 1.69 with two of
+// 384 (whose registers spill).
+template <typename T, int RECON, bool DE, bool HALF, int NT, int PER, int NT2, int PER2>
+void launch_march_hd_of(const BlockDesc<T> *d, int nb, int mx, int my, int mz,
+                        const StageParams &sp, hipStream_t s) {
+  const int cus = device_cus();
+  double big, small;
+  const MarchParams p = march_tiling<NT, PER>(mx, my, mz, sp.cur_stale, nb, cus, big);
+  const MarchParams q = march_tiling<NT2, PER2>(mx, my, mz, sp.cur_stale, nb, cus, small);
+  if (big <= small)
+    launch_march_hd_nt<T, RECON, DE, HALF, NT, PER>(d, p, sp, s);
+  else
+    launch_march_hd_nt<T, RECON, DE, HALF, NT2, PER2>(d, q, sp, s);
+}
+template <typename T, int RECON, bool DE, bool HALF>
+void launch_march_hd(const BlockDesc<T> *d, int nb, int mx, int my, int mz,
+                     const StageParams &sp, hipStream_t s) {
+  if constexpr (std::is_same<T, float>::value) {
+    if constexpr (RECON == RC_NN)
+      launch_march_hd_of<T, RECON, DE, HALF, 512, 3, 256, 6>(d, nb, mx, my, mz, sp, s);
+    else
+      launch_march_hd_of<T, RECON, DE, HALF, 512, 2, 256, 4>(d, nb, mx, my, mz, sp, s);
+  } else {
+    if constexpr (RECON == RC_NN)
+      launch_march_hd_of<T, RECON, DE, HALF, 512, 2, 256, 4>(d, nb, mx, my, mz, sp, s);
+    else if constexpr (DE)
+      launch_march_hd_of<T, RECON, DE, HALF, 512, 1, 256, 2>(d, nb, mx, my, mz, sp, s);
+    else
+      launch_march_hd_of<T, RECON, DE, HALF, 768, 1, 256, 3>(d, nb, mx, my, mz, sp, s);
+  }
+}
+template <typename T, bool DE>
+void dispatch_march_hd(int recon, const BlockDesc<T> *d, int nb, int mx, int my, int mz,
+                       const StageParams &sp, hipStream_t s) {
+  if (sp.stage == 0)
+    launch_march_hd<T, RC_NN, DE, false>(d, nb, mx, my, mz, sp, s);
+  else if (recon == RC_NN)
+    launch_march_hd<T, RC_NN, DE, true>(d, nb, mx, my, mz, sp, s);
+  else if (recon == RC_PLM)
+    launch_march_hd<T, RC_PLM, DE, true>(d, nb, mx, my, mz, sp, s);
+  else
+    launch_march_hd<T, RC_PLM_ATHENA, DE, true>(d, nb, mx, my, mz, sp, s);
 }
 
 // Bytes of the chunk scratch pool: the larger of 4 GiB and a third of the
@@ -722,7 +783,9 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
                   hipStream_t s, const StoreArgs *st, unsigned long long *cfl,
                   bool timers) {
   const int mx = blocks[0].mx, my = blocks[0].my, mz = blocks[0].mz;
-  const bool march = march_ok(m, mx, my, mz, blocks[0].ghost, std::min(n, chunk));
+  // (stored fluxes come from the separate launches' flux arrays)
+  const bool march =
+      !st && march_ok(m, mx, my, mz, blocks[0].ghost, std::min(n, chunk));
   for (int c0 = 0; c0 < n; c0 += chunk) {
     const int c1 = std::min(n, c0 + chunk);
     const int nb = c1 - c0;
@@ -756,26 +819,26 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
       // with the fused CFL the final update's launch covers the block
       const int lo = sp.cfl ? 0 : (is_final ? cs : cs + 1);
       const int structure = ctu_variant(m, mx, my, mz);
-      if constexpr (MHD) {
-        if (march) {
-          {
-            KernelTimer kt(s, recon == RC_NN ? "k_march_nn" : "k_march_plm", timers);
-            if (m->riemann == RS_HLLD)
-              dispatch_march<FluxT, RS_HLLD, DE>(recon, d, nb, mx, my, mz, sp, s);
-            else
-              dispatch_march<FluxT, RS_HLLE, DE>(recon, d, nb, mx, my, mz, sp, s);
-          }
-          if (is_final) {
-            // the cells around the update: ring centre B, CFL, pressure
-            const int blo = sp.cfl ? 0 : cs;
-            const long shell = cube(mx, my, mz, blo, blo) - cube(mx, my, mz, cs + 1, cs + 1);
-            KernelTimer kt(s, "k_shell", timers);
-            hipLaunchKernelGGL((k_shell<FluxT, MHD, DE>), dim3(nblk(shell, 256), nb), dim3(256),
-                               0, s, d, sp);
-          }
-          stale += total_staling(recon);
-          continue;
+      if (march) {
+        {
+          KernelTimer kt(s, recon == RC_NN ? "k_march_nn" : "k_march_plm", timers);
+          if constexpr (!MHD)
+            dispatch_march_hd<FluxT, DE>(recon, d, nb, mx, my, mz, sp, s);
+          else if (m->riemann == RS_HLLD)
+            dispatch_march<FluxT, RS_HLLD, DE>(recon, d, nb, mx, my, mz, sp, s);
+          else
+            dispatch_march<FluxT, RS_HLLE, DE>(recon, d, nb, mx, my, mz, sp, s);
         }
+        if (is_final && (MHD || sp.cfl)) {
+          // the cells around the update: ring centre B, CFL, pressure
+          const int blo = sp.cfl ? 0 : cs;
+          const long shell = cube(mx, my, mz, blo, blo) - cube(mx, my, mz, cs + 1, cs + 1);
+          KernelTimer kt(s, "k_shell", timers);
+          hipLaunchKernelGGL((k_shell<FluxT, MHD, DE>), dim3(nblk(shell, 256), nb), dim3(256), 0,
+                             s, d, sp);
+        }
+        stale += total_staling(recon);
+        continue;
       }
       if constexpr (!DE) {
         if (structure == 5 && persistent_ok(m) && m->d_bar) {

@@ -121,11 +121,11 @@ __device__ __forceinline__ void march_states(int q, T am, T a, T ap, T theta,
   }
 }
 // Whether a cell's state is outside the range of EXACT = false.
-template <typename T>
+template <bool MHD, typename T>
 __device__ __forceinline__ bool march_wild(const T w[S_N]) {
   T s = fabs(w[0]);
 #pragma unroll
-  for (int q = 1; q < S_N; q++) s += fabs(w[q]);
+  for (int q = 1; q < (MHD ? S_N : S_BX); q++) s += fabs(w[q]);
   return !(s < (T)MARCH_TAME);
 }
 
@@ -159,11 +159,11 @@ struct RawCell {
   double ei;
 };
 // off: the cell's byte offset in an FP64 field
-template <typename T, bool DE, bool HALF>
+template <bool MHD, typename T, bool DE, bool HALF>
 __device__ __forceinline__ void march_load(const BlockDesc<T> &b, unsigned off,
                                            RawCell<T, DE, HALF> &r) {
 #pragma unroll
-  for (int q = 0; q < S_N; q++) {
+  for (int q = 0; q < (MHD ? S_N : S_BX); q++) {
     if constexpr (HALF) {
       if constexpr (std::is_same<T, float>::value)
         r.d[q] = ldo(b.Up[q], off >> 1);
@@ -183,18 +183,60 @@ __device__ __forceinline__ void march_center_e(const P w[S_N], double ec[3]) {
   ec[2] = center_efield((double)w[S_VX], (double)w[S_VY], (double)w[S_BX], (double)w[S_BY]);
 }
 // ... as primitives (load_prim's expressions)
-template <typename T, bool DE, bool HALF>
+template <bool MHD, typename T, bool DE, bool HALF>
 __device__ __forceinline__ void march_prim(const RawCell<T, DE, HALF> &r, double gm1, T w[S_N]) {
 #pragma unroll
-  for (int q = 0; q < S_N; q++)
+  for (int q = 0; q < (MHD ? S_N : S_BX); q++)
     if (HALF || q != S_E) w[q] = (T)r.d[q];
   if constexpr (!HALF) {
     if (DE)
       w[S_E] = (T)(gm1 * r.d[S_RHO] * r.ei);
     else
-      w[S_E] = (T)prim_pressure<true>(r.d[S_RHO], r.d[S_VX], r.d[S_VY], r.d[S_VZ], r.d[S_E],
-                                      r.d[S_BX], r.d[S_BY], r.d[S_BZ], gm1);
+      w[S_E] = (T)prim_pressure<MHD>(r.d[S_RHO], r.d[S_VX], r.d[S_VY], r.d[S_VZ], r.d[S_E],
+                                     MHD ? r.d[S_BX] : 0., MHD ? r.d[S_BY] : 0.,
+                                     MHD ? r.d[S_BZ] : 0., gm1);
   }
+}
+
+// One piece of a workgroup's planes: the column of this thread and the
+// offsets the marches use.  False when the piece holds no plane to update.
+struct MarchPiece {
+  int by, tix, tiy, z0;  // block, tile, first updated plane of the piece
+  int ks, ke;            // updated planes [ks, ke)
+};
+__device__ __forceinline__ bool march_piece(const MarchParams &mp, int cs, long &pos, long last,
+                                            MarchPiece &p) {
+  const unsigned column = (unsigned)((unsigned long)pos / (unsigned)mp.zseg);
+  const int zin = (int)(pos - (long)column * mp.zseg);
+  int zn = (last - pos < mp.zseg - zin) ? (int)(last - pos) : mp.zseg - zin;
+  pos += zn;
+  const int ntile = mp.ntx * mp.nty;
+  const unsigned part = column / (unsigned)ntile;
+  const int tile = (int)(column - part * (unsigned)ntile);
+  p.by = (int)(part / (unsigned)mp.nseg);
+  p.z0 = (int)(part - (unsigned)p.by * (unsigned)mp.nseg) * mp.zseg + zin;
+  if (zn > mp.nz - p.z0) zn = mp.nz - p.z0;  // the last segment may be shorter
+  if (zn <= 0) return false;
+  p.tiy = tile / mp.ntx;
+  p.tix = tile - p.tiy * mp.ntx;
+  p.ks = cs + 1 + p.z0;
+  p.ke = p.ks + zn;
+  return true;
+}
+// The cell of the outer ring that thread r of a reconstructing march brings
+// in: tile coordinates (rx, ry); false for the threads past the ring.
+__device__ __forceinline__ bool march_ring(int r, int w2, int h2, int &rx, int &ry) {
+  const bool ring = r < 2 * (w2 + h2);
+  if (r < 2 * h2) {
+    rx = (r & 1) ? w2 : -1;
+    ry = r >> 1;
+  } else {
+    r -= 2 * h2;
+    rx = r >> 1;
+    ry = (r & 1) ? h2 : -1;
+  }
+  if (!ring) rx = ry = 0;
+  return ring;
 }
 
 // Launch: total / share workgroups (rounded up to a multiple of 8) of NT
@@ -254,23 +296,13 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
   double local = 1.7976931348623157e308;
 
   for (long pos = (long)g * mp.share; pos < last;) {
-    const unsigned column = (unsigned)((unsigned long)pos / (unsigned)mp.zseg);
-    const int zin = (int)(pos - (long)column * mp.zseg);
-    int zn = (last - pos < mp.zseg - zin) ? (int)(last - pos) : mp.zseg - zin;
-    pos += zn;
-    const int ntile = mp.ntx * mp.nty;
-    const unsigned part = column / (unsigned)ntile;
-    const int tile = (int)(column - part * (unsigned)ntile);
-    const int by = (int)(part / (unsigned)mp.nseg);
-    const int z0 = (int)(part - (unsigned)by * (unsigned)mp.nseg) * mp.zseg + zin;
-    if (zn > mp.nz - z0) zn = mp.nz - z0;  // the last segment may be shorter
-    if (zn <= 0) continue;
+    MarchPiece piece;
+    if (!march_piece(mp, cs, pos, last, piece)) continue;
+    const int by = piece.by, tix = piece.tix, tiy = piece.tiy, z0 = piece.z0;
+    const int ks = piece.ks, ke = piece.ke;
     if (zero_step(sp, by)) continue;
     const BlockDesc<T> &b = blocks[by];
     const int mx = b.mx, my = b.my, mz = b.mz;
-    const int tiy = tile / mp.ntx, tix = tile - tiy * mp.ntx;
-    // updated planes [ks, ke)
-    const int ks = cs + 1 + z0, ke = ks + zn;
 
     const bool lane = tid < w2 * h2;
     const int ty = lane ? tid / w2 : 0, tx = lane ? tid - ty * w2 : 0;
@@ -311,17 +343,8 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
     unsigned rcol = 0;
     int rw = 0;
     if constexpr (PLM) {
-      int r = tid, rx = 0, ry = 0;
-      ring = r < 2 * (w2 + h2);
-      if (r < 2 * h2) {
-        rx = (r & 1) ? w2 : -1;
-        ry = r >> 1;
-      } else {
-        r -= 2 * h2;
-        rx = r >> 1;
-        ry = (r & 1) ? h2 : -1;
-      }
-      if (!ring) rx = ry = 0;
+      int rx, ry;
+      ring = march_ring(tid, w2, h2, rx, ry);
       int ri = cs + tix * (w2 - 2) + rx, rj = cs + tiy * (h2 - 2) + ry;
       ri = ri < mx ? ri : mx - 1;
       rj = rj < my ? rj : my - 1;
@@ -358,15 +381,15 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
       T w[S_N];
       const unsigned c0 = (unsigned)k0 * plane + col;
       bool wild = false;
-      march_load(b, c0, raw);
-      march_prim(raw, fc.gm1, w);
+      march_load<true>(b, c0, raw);
+      march_prim<true>(raw, fc.gm1, w);
       if constexpr (F32 && HALF) {
 #pragma unroll
         for (int a = 0; a < 3; a++) ec[a] = ldo(b.Ech[a], c0);
       } else {
         march_center_e(raw.d, ec);
       }
-      if (CHECK) wild = march_wild(w);
+      if (CHECK) wild = march_wild<true>(w);
       if (lane) {
 #pragma unroll
         for (int q = 0; q < S_N; q++) sW[q][wi] = w[q];
@@ -374,13 +397,13 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
 #pragma unroll
       for (int a = 0; a < 3; a++) sEc[a][tid] = ec[a];
       if constexpr (PLM) {
-        march_load(b, c0 - plane, raw);
-        march_prim(raw, fc.gm1, wm);
-        march_load(b, c0 + plane, raw);
-        march_prim(raw, fc.gm1, wp);
-        march_load(b, (unsigned)k0 * plane + rcol, raw);
-        march_prim(raw, fc.gm1, w);
-        if (CHECK) wild = wild || march_wild(wm) || march_wild(wp) || march_wild(w);
+        march_load<true>(b, c0 - plane, raw);
+        march_prim<true>(raw, fc.gm1, wm);
+        march_load<true>(b, c0 + plane, raw);
+        march_prim<true>(raw, fc.gm1, wp);
+        march_load<true>(b, (unsigned)k0 * plane + rcol, raw);
+        march_prim<true>(raw, fc.gm1, w);
+        if (CHECK) wild = wild || march_wild<true>(wm) || march_wild<true>(wp) || march_wild<true>(w);
         if (ring) {
 #pragma unroll
           for (int q = 0; q < S_N; q++) sW[q][rw] = w[q];
@@ -531,7 +554,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
       u0.e = ldo(b.U[S_E], cu);
       if (DE) u0.ei = ldo(b.ei, cu);
       RawCell<T, DE, HALF> nxt, nx2, halo;
-      march_load(b, cn, nxt);
+      march_load<true>(b, cn, nxt);
       fbx = ldo(bfr[0], kn * planex + colx);
       fby = ldo(bfr[1], kn * planey + coly);
       fbz = ldo(bfr[2], cn);
@@ -541,9 +564,9 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
         for (int a = 0; a < 3; a++) echn[a] = ldo(b.Ech[a], cn);
       }
       if constexpr (PLM) {
-        march_load(b, kn * plane + rcol, halo);
+        march_load<true>(b, kn * plane + rcol, halo);
         const unsigned kn2 = (unsigned)((k + 2 < mz) ? k + 2 : mz - 1);
-        march_load(b, kn2 * plane + col, nx2);
+        march_load<true>(b, kn2 * plane + col, nx2);
       }
       lds_barrier();  // the plane's fluxes are in LDS
       // ---- E: edge EMFs
@@ -627,7 +650,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
       {
         T w[S_N];
         double ec[3];
-        march_prim(nxt, fc.gm1, w);
+        march_prim<true>(nxt, fc.gm1, w);
         if constexpr (F32 && HALF) {
 #pragma unroll
           for (int a = 0; a < 3; a++) ec[a] = echn[a];
@@ -638,13 +661,13 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
 #pragma unroll
           for (int q = 0; q < S_N; q++) wm[q] = sW[q][wi];
           T h[S_N];
-          march_prim(halo, fc.gm1, h);
+          march_prim<true>(halo, fc.gm1, h);
           if (ring) {
 #pragma unroll
             for (int q = 0; q < S_N; q++) sW[q][rw] = h[q];
           }
-          march_prim(nx2, fc.gm1, wp);
-          if (CHECK && (march_wild(h) || march_wild(wp))) sWild = 1;
+          march_prim<true>(nx2, fc.gm1, wp);
+          if (CHECK && (march_wild<true>(h) || march_wild<true>(wp))) sWild = 1;
         }
         if (lane) {
 #pragma unroll
@@ -655,6 +678,306 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
       }
       lds_barrier();
     }
+  }
+  if (sp.cfl != nullptr) march_min_to<NT>(sp.cfl, local, wmin);
+}
+
+// The hydrodynamic march: as k_march, with the HLLC solve and without
+// constrained transport.  A step at plane k: the z face below it, which
+// completes the divergence and the update of the cell of plane k - 1; then
+// the x and y faces of plane k.  The right states travel through the rows of
+// LDS that take the fluxes afterwards.  Bound as k_march; 8 blocks of 128^3,
+// FP64: 0.81 + 1.17 ms for the two stages against 1.66 + 1.94 of the separate
+// launches (a third of which wrote the 15 fluxes of a cell and read them
+// back); mixed 0.46 + 0.61 against 1.12 + 1.11.  WAVES: a SIMD's waves that its
+// registers are held to.
+template <typename T, int RECON, bool DE, bool HALF, int NT, int WAVES>
+__global__ void __launch_bounds__(NT, WAVES)
+k_march_hd(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp) {
+  constexpr bool PLM = RECON != RC_NN;
+  constexpr bool F32 = std::is_same<T, float>::value;
+  constexpr bool CHECK = RECON == RC_PLM && !F32;
+  constexpr bool FINAL = HALF;
+  constexpr int NQ = 5;  // density, velocity, pressure
+  static_assert(HALF || !PLM, "the first stage is the nearest-neighbour one");
+  sp.stage = sp.is_final = FINAL ? 1 : 0;
+  sp.dbg = nullptr;
+  if (!FINAL) sp.cfl = nullptr;
+  const unsigned g = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const long last = ((long)g + 1) * mp.share < mp.total ? ((long)g + 1) * mp.share : mp.total;
+
+  FluxConsts fc;
+  fc.gm1 = sp.gamma - 1.0;
+  fc.gamma = sp.gamma;
+  fc.igm1 = sp.igm1;
+  fc.theta = sp.theta;
+  fc.dfloor = sp.density_floor;
+  fc.pfloor = sp.pressure_floor;
+  fc.dbg = nullptr;
+  const T theta = (T)sp.theta;
+
+  constexpr int WN = PLM ? march_plane_cells(NT) : NT;
+  __shared__ T sW[NQ][WN];
+  __shared__ T sF[2 * NQ][NT];  // right states, then fluxes: x rows, y rows
+  __shared__ double sD[DE ? 4 : 1][DE ? NT : 1];
+  __shared__ unsigned long long wmin[NT / 64];
+  __shared__ int sWild;
+
+  const int tid = (int)threadIdx.x;
+  const int w2 = mp.w2, h2 = mp.h2;
+  const int cs = sp.cur_stale;
+  double local = 1.7976931348623157e308;
+
+  for (long pos = (long)g * mp.share; pos < last;) {
+    MarchPiece piece;
+    if (!march_piece(mp, cs, pos, last, piece)) continue;
+    const int by = piece.by, tix = piece.tix, tiy = piece.tiy;
+    const int ks = piece.ks, ke = piece.ke;
+    if (zero_step(sp, by)) continue;
+    const BlockDesc<T> &b = blocks[by];
+    const int mx = b.mx, my = b.my, mz = b.mz;
+
+    const bool lane = tid < w2 * h2;
+    const int ty = lane ? tid / w2 : 0, tx = lane ? tid - ty * w2 : 0;
+    const int i = cs + tix * (w2 - 2) + tx, j = cs + tiy * (h2 - 2) + ty;
+    const int ic = i < mx ? i : mx - 1, jc = j < my ? j : my - 1;
+    const bool upd = lane && tx >= 1 && tx < w2 - 1 && i < mx - cs - 1 && ty >= 1 &&
+                     ty < h2 - 1 && j < my - cs - 1;
+    const double dt = sp.dts ? sp.dts[by] * sp.dt_factor : sp.dt;
+    const double dtdx = uniform(dt / b.cw[0]), dtdy = uniform(dt / b.cw[1]),
+                 dtdz = uniform(dt / b.cw[2]);
+    const int xp = tid + 1 < NT ? tid + 1 : NT - 1, xm = tid > 0 ? tid - 1 : 0;
+    const int yp = tid + w2 < NT ? tid + w2 : NT - 1, ym = tid >= w2 ? tid - w2 : 0;
+    const int ws = PLM ? w2 + 2 : w2;
+    const int wi = PLM ? (ty + 1) * ws + tx + 1 : tid;
+    const unsigned plane = 8u * (unsigned)(mx * my);
+    const unsigned col = 8u * (unsigned)(jc * mx + ic);
+    bool ring = false;
+    unsigned rcol = 0;
+    int rw = 0;
+    if constexpr (PLM) {
+      int rx, ry;
+      ring = march_ring(tid, w2, h2, rx, ry);
+      int ri = cs + tix * (w2 - 2) + rx, rj = cs + tiy * (h2 - 2) + ry;
+      ri = ri < mx ? ri : mx - 1;
+      rj = rj < my ? rj : my - 1;
+      rcol = 8u * (unsigned)(rj * mx + ri);
+      rw = (ry + 1) * ws + rx + 1;
+    }
+
+    // carried from plane to plane
+    T Lz[S_N], wm[S_N], wp[S_N], Fz[NQ];
+    double dU[NQ], dUe = 0., pc = 0.;
+    T FzE = T(0), FzV = T(0);
+    CellBase u0{};
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      Fz[q] = T(0);
+      dU[q] = 0.;
+    }
+#pragma unroll
+    for (int q = 0; q < S_N; q++) Lz[q] = wm[q] = wp[q] = T(0);
+
+    // the left state of the first z face, the planes around the first one
+    if (CHECK && tid == 0) sWild = 0;
+    if (CHECK) lds_barrier();
+    {
+      RawCell<T, DE, HALF> raw;
+      T w[S_N], h[S_N];
+      const unsigned c0 = (unsigned)ks * plane + col;
+      march_load<false>(b, c0 - plane, raw);
+      march_prim<false>(raw, fc.gm1, wm);
+      march_load<false>(b, c0, raw);
+      march_prim<false>(raw, fc.gm1, w);
+      if constexpr (PLM) {
+        march_load<false>(b, c0 - 2u * plane, raw);
+        march_prim<false>(raw, fc.gm1, wp);
+        bool wild = CHECK && (march_wild<false>(wm) || march_wild<false>(w) ||
+                              march_wild<false>(wp));
+        // (the general form of the limiter: one state a piece)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+          T low;
+          march_states<RECON, true>(q, wp[q], wm[q], w[q], theta, fc, low, Lz[q]);
+        }
+        march_load<false>(b, (unsigned)(ks + 1 < mz ? ks + 1 : mz - 1) * plane + col, raw);
+        march_prim<false>(raw, fc.gm1, wp);
+        march_load<false>(b, (unsigned)ks * plane + rcol, raw);
+        march_prim<false>(raw, fc.gm1, h);
+        if (CHECK) wild = wild || march_wild<false>(wp) || march_wild<false>(h);
+        if (CHECK && wild) sWild = 1;
+        if (ring) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) sW[q][rw] = h[q];
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) Lz[q] = wm[q];
+      }
+      if (lane) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) sW[q][wi] = w[q];
+      }
+    }
+    lds_barrier();
+
+    for (int k = ks; k <= ke; k++) {
+      const bool exact = CHECK && __builtin_amdgcn_readfirstlane(sWild) != 0;
+      // ---- z: the face between planes k - 1 and k
+      {
+        T a[S_N], R[S_N], Ln[S_N];
+#pragma unroll
+        for (int q = 0; q < NQ; q++) a[q] = sW[q][wi];
+        if constexpr (PLM) {
+          auto states = [&](auto ex) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++)
+              march_states<RECON, decltype(ex)::value>(q, wm[q], a[q], wp[q], theta, fc, R[q],
+                                                       Ln[q]);
+          };
+          if (!CHECK || exact)
+            states(std::true_type());
+          else
+            states(std::false_type());
+        } else {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) R[q] = Ln[q] = a[q];
+        }
+        FaceFlux<T> f;
+        solve_face<T, RS_HLLC, false, 2, DE>(Lz, R, T(0), fc, f);
+        if (k > ks) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++)
+            dU[q] = flux_difference(dU[q], dtdz, (double)f.u[q], (double)Fz[q]);
+          if (DE) {
+            dUe = flux_difference(dUe, dtdz, (double)f.e, (double)FzE);
+            dUe = source_difference(dUe, dtdz, pc, (double)f.vb, (double)FzV);
+          }
+          if (upd) {
+            const double bc[3] = {0., 0., 0.};
+            const double t = cell_finish<T, false, DE, true>(
+                b, sp, dt, CellOffset{(unsigned)(k - 1) * plane + col}, u0, dU, dUe, bc);
+            local = t < local ? t : local;
+          }
+        }
+        if (k == ke) break;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+          Fz[q] = f.u[q];
+          Lz[q] = Ln[q];
+        }
+        if (DE) {
+          FzE = f.e;
+          FzV = f.vb;
+        }
+      }
+      // ---- x, y: the faces towards i + 1 and j + 1
+      FaceFlux<T> fx, fy;
+      {
+        T Lx[S_N], Ly[S_N], Rx[S_N], Ry[S_N];
+        if constexpr (PLM) {
+          auto states = [&](auto ex) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+              constexpr bool EX = decltype(ex)::value;
+              const T a = sW[q][wi];
+              T rx, ry;
+              march_states<RECON, EX>(q, sW[q][wi - 1], a, sW[q][wi + 1], theta, fc, rx, Lx[q]);
+              march_states<RECON, EX>(q, sW[q][wi - ws], a, sW[q][wi + ws], theta, fc, ry,
+                                      Ly[q]);
+              sF[q][tid] = rx;
+              sF[NQ + q][tid] = ry;
+            }
+          };
+          if (!CHECK || exact)
+            states(std::true_type());
+          else
+            states(std::false_type());
+          lds_barrier();
+#pragma unroll
+          for (int q = 0; q < NQ; q++) {
+            Rx[q] = sF[q][xp];
+            Ry[q] = sF[NQ + q][yp];
+          }
+          lds_barrier();
+        } else {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) {
+            Lx[q] = Ly[q] = sW[q][wi];
+            Rx[q] = sW[q][xp];
+            Ry[q] = sW[q][yp];
+          }
+        }
+        solve_face<T, RS_HLLC, false, 0, DE>(Lx, Rx, T(0), fc, fx);
+        solve_face<T, RS_HLLC, false, 1, DE>(Ly, Ry, T(0), fc, fy);
+      }
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        sF[q][tid] = fx.u[q];
+        sF[NQ + q][tid] = fy.u[q];
+      }
+      if (DE) {
+        sD[0][tid] = (double)fx.e;
+        sD[1][tid] = (double)fx.vb;
+        sD[2][tid] = (double)fy.e;
+        sD[3][tid] = (double)fy.vb;
+      }
+      // loads for the next step: the base of this plane's update, the next
+      // planes
+      const unsigned kn = (unsigned)((k + 1 < mz) ? k + 1 : mz - 1);
+      const unsigned cu = (unsigned)k * plane + col;
+      RawCell<T, DE, HALF> nxt, nx2, halo;
+      march_load<false>(b, kn * plane + col, nxt);
+      if constexpr (PLM) {
+        march_load<false>(b, kn * plane + rcol, halo);
+        const unsigned kn2 = (unsigned)((k + 2 < mz) ? k + 2 : mz - 1);
+        march_load<false>(b, kn2 * plane + col, nx2);
+      }
+      u0.rho = ldo(b.U[S_RHO], cu);
+      u0.v[0] = ldo(b.U[S_VX], cu);
+      u0.v[1] = ldo(b.U[S_VY], cu);
+      u0.v[2] = ldo(b.U[S_VZ], cu);
+      u0.e = ldo(b.U[S_E], cu);
+      if (DE) u0.ei = ldo(b.ei, cu);
+      lds_barrier();  // the plane's fluxes are in LDS
+      // ---- the x and y parts of plane k's divergence
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        dU[q] = flux_difference(0., dtdx, (double)fx.u[q], (double)sF[q][xm]);
+        dU[q] = flux_difference(dU[q], dtdy, (double)fy.u[q], (double)sF[NQ + q][ym]);
+      }
+      if (DE) {
+        pc = dmax((double)sW[S_E][wi], sp.pressure_floor);
+        dUe = flux_difference(0., dtdx, sD[0][tid], sD[0][xm]);
+        dUe = source_difference(dUe, dtdx, pc, sD[1][tid], sD[1][xm]);
+        dUe = flux_difference(dUe, dtdy, sD[2][tid], sD[2][ym]);
+        dUe = source_difference(dUe, dtdy, pc, sD[3][tid], sD[3][ym]);
+      }
+      // ---- the next plane into LDS
+      {
+        T w[S_N];
+        march_prim<false>(nxt, fc.gm1, w);
+        if constexpr (PLM) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) wm[q] = sW[q][wi];
+          T h[S_N];
+          march_prim<false>(halo, fc.gm1, h);
+          if (ring) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) sW[q][rw] = h[q];
+          }
+          march_prim<false>(nx2, fc.gm1, wp);
+          if (CHECK && (march_wild<false>(h) || march_wild<false>(wp))) sWild = 1;
+        }
+        if (!PLM) lds_barrier();  // (the x and y states of this plane have been read)
+        if (lane) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) sW[q][wi] = w[q];
+        }
+      }
+      lds_barrier();
+    }
+    lds_barrier();  // the piece's last reads of LDS
   }
   if (sp.cfl != nullptr) march_min_to<NT>(sp.cfl, local, wmin);
 }

@@ -173,8 +173,8 @@ int enzoe_vlct_compute_dt(enzoe_vlct_t m, const enzoe_block *blocks, int n,
  * and, with the launch-structure setting "auto" (enzoe_vlct_set_fused_ct),
  * for MHD the fused CT + update launch with each of its tile shapes and the
  * orders of its two kernels, and (HLLD MHD or hydro, no dual energy) the
- * persistent launch of a whole stage, and for MHD the marched stages; then,
- * for the chosen one of the others, the rows of the tiled cell order (slabs
+ * persistent launch of a whole stage, and the marched stages; then, for the
+ * chosen one of the others, the rows of the tiled cell order (slabs
  * of 8, 16, 32 or 64 rows, or the plain order), and the other shapes of the flux launch (enzoe_vlct_set_flux_shape).
  * *mask_out (optional) gets the chosen mask: bit 0 k_flux, 1 k_edge,
  * 2 k_faces, 3 k_cells (or the fused launch).  enzoe_vlct_launch_choice:
@@ -721,11 +721,11 @@ int enzoe_vlct_transfer_batch(enzoe_vlct_t m, const enzoe_transfer *items,
  * cell phases in turn with a device-wide barrier between them (HLLD MHD or
  * hydro without the dual-energy formalism; elsewhere, and on the
  * allocation-free entry point, the four launches); -1 (the default): the
- * autotuner's choice per block shape; until it has run, for MHD each stage
- * as one launch that marches tiles of columns through the planes and keeps
- * fluxes, EMFs and faces on the chip (from 2^18 active cells of a call on,
- * where no debug counts and no flux-launch shape are asked for), else the
- * four launches.
+ * autotuner's choice per block shape; until it has run, each stage as one
+ * launch that marches tiles of columns through the planes and keeps fluxes,
+ * EMFs and faces on the chip (two-stage schemes, from 2^18 active cells of a
+ * call on, FP64 hydro 3 2^17, where no debug counts, stored fluxes or
+ * flux-launch shape are asked for), else the four launches.
  * Every variant gives the same bits in FP64 (the mixed and contracted
  * builds: up to the rounding of their contracted flux arithmetic, which the
  * compiler may fuse differently in different kernels).  Not to be changed
