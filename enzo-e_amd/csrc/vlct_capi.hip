@@ -869,6 +869,8 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
     *ms_per_run = ms / reps;
     return ENZOE_OK;
   };
+  // (with three faces per thread, unless another shape is set)
+  m->force_shape = m->flux_shape < 0 ? 0 : -1;
   for (size_t ci = 0; ci < cand.size() && rc == ENZOE_OK; ci++) {
     const int mask = cand[ci].second;
     m->force_mask = mask;
@@ -918,6 +920,7 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
     m->force_ctu = -1;
     m->force_rows = -1;
   }
+  m->force_shape = -1;
   // then the other shapes of the flux launch (one face per thread: more
   // workgroups for small blocks; z pencils for the nearest-neighbour
   // stage), for the chosen structure, order and rows
@@ -957,11 +960,11 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
 int enzoe_vlct_launch_choice(enzoe_vlct_t m, int mx, int my, int mz, int *mask, int *fused_ct,
                              int *tile_rows, int *flux_shape) {
   if (!m) return ENZOE_ERR_ARG;
-  if (flux_shape) *flux_shape = flux_shape_of(m, mx, my, mz);
+  if (flux_shape) *flux_shape = flux_shape_of(m, mx, my, mz, 1);
   if (mask) *mask = launch_mask(m, mx, my, mz);
   if (tile_rows) *tile_rows = tile_rows_of(m, mx, my, mz);
   if (fused_ct) {
-    const int v = ctu_variant(m, mx, my, mz);
+    const int v = ctu_variant(m, mx, my, mz, 1);
     *fused_ct = (v == 5) ? (persistent_ok(m) ? 5 : 0)
                          : ((m->mhd && ctu_possible(m) && v < 5) ? v : 0);
   }

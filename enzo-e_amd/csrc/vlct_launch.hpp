@@ -160,17 +160,21 @@ inline long long shape_key(int mx, int my, int mz) {
   return ((long long)mx << 40) | ((long long)my << 20) | (long long)mz;
 }
 
-// The launch structure of the stages for blocks of this shape: 0 =
-// k_flux, then k_edge + k_faces + k_cells; for MHD 1..3 = k_ctu with tile
+// The launch structure of the stages for blocks of this shape where they do
+// not run marched (march_ok): 0 = k_flux, then k_edge + k_faces + k_cells; for MHD 1..3 = k_ctu with tile
 // CtuTile1..3, 4 = k_edge + k_ctu without its edge phase (faces and cells
 // fused); 5 = the persistent k_stage (persistent_ok); the method's
 // setting, or the autotuner's choice for the shape when the setting is
-// "auto" (-1).
-inline int ctu_variant(const enzoe_vlct_method *m, int mx, int my, int mz) {
+// "auto" (-1).  Until it has run, tile 32 x 4 x 2 for MHD below 2^19 cells,
+// ghost zones included: those calls are bound by latency, and k_ctu is two
+// launches fewer a stage (cycle of one FP64 block of 16^3: 93 against 77 us,
+// of 32^3 100, 91, of 56^3 152, 143; 32 of 16^3 187, 177; 4 of 32^3 151, 153).
+inline int ctu_variant(const enzoe_vlct_method *m, int mx, int my, int mz, int nb) {
   if (m->force_ctu >= 0) return m->force_ctu;
   if (m->ctu >= 0) return m->ctu;
   auto it = m->tuned_ctu.find(shape_key(mx, my, mz));
-  return it != m->tuned_ctu.end() ? it->second : 0;
+  if (it != m->tuned_ctu.end()) return it->second;
+  return (m->mhd && m->nstages == 2 && (long)mx * my * mz * nb < (1L << 19)) ? 2 : 0;
 }
 
 // ... and, chosen by march_ok and not by enzoe_vlct_set_fused_ct, the marched
@@ -380,12 +384,16 @@ inline int tile_rows_for(int mx, int my) {
 // (k_flux); 1, one face per thread (k_flux over three z slices, for blocks
 // too small to fill the device); 2, the nearest-neighbour stage as z
 // pencils with LDS-staged planes (k_flux_zp; the other stages as 0).  The
-// setting, else the autotuner's choice, else 0.
-inline int flux_shape_of(const enzoe_vlct_method *m, int mx, int my, int mz) {
+// setting, else the autotuner's choice, else 1 for launches of fewer than
+// 2^18 cells, ghost zones included (under 4 waves a SIMD with one cell a
+// thread; cycle in us with 0 and 1: 16^3 MHD 77, 67, hydro 53, 48; 4 blocks of
+// 32^3 153, 149 and 86, 83; equal at 56^3).
+inline int flux_shape_of(const enzoe_vlct_method *m, int mx, int my, int mz, int nb) {
   if (m->force_shape >= 0) return m->force_shape;
   if (m->flux_shape >= 0) return m->flux_shape;
   auto it = m->tuned_shape.find(shape_key(mx, my, mz));
-  return it != m->tuned_shape.end() ? it->second : 0;
+  if (it != m->tuned_shape.end()) return it->second;
+  return (long)mx * my * mz * nb < (1L << 18) ? 1 : 0;
 }
 
 // Rows of the tiled cell order for blocks of this shape.
@@ -818,7 +826,7 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
       const bool primf = stage > 0 && half_f32<FluxT>(DE ? 1 : 0);
       // with the fused CFL the final update's launch covers the block
       const int lo = sp.cfl ? 0 : (is_final ? cs : cs + 1);
-      const int structure = ctu_variant(m, mx, my, mz);
+      const int structure = ctu_variant(m, mx, my, mz, nb);
       if (march) {
         {
           KernelTimer kt(s, recon == RC_NN ? "k_march_nn" : "k_march_plm", timers);
@@ -856,7 +864,7 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
       {
         KernelTimer kt(s, recon == RC_NN ? "k_flux_nn" : "k_flux_plm", timers);
         dispatch_flux<FluxT, MHD, DE>(m, recon, primf, d, nb, mx, my, mz, sp, s,
-                                      flux_shape_of(m, mx, my, mz));
+                                      flux_shape_of(m, mx, my, mz, nb));
       }
       const int variant =
           (MHD && ctu_possible(m) && structure >= 1 && structure <= 4) ? structure : 0;

@@ -179,7 +179,8 @@ int enzoe_vlct_compute_dt(enzoe_vlct_t m, const enzoe_block *blocks, int n,
  * *mask_out (optional) gets the chosen mask: bit 0 k_flux, 1 k_edge,
  * 2 k_faces, 3 k_cells (or the fused launch).  enzoe_vlct_launch_choice:
  * the mask, the launch structure (0 = four launches per stage, or where the
- * setting is "auto" the marched stages; 1..5 as enzoe_vlct_set_fused_ct), the tile rows and the flux-launch shape (0..2)
+ * setting is "auto" the marched stages; 1..5 as enzoe_vlct_set_fused_ct; of a
+ * call of one block until the autotuner has run), the tile rows and the flux-launch shape (0..2)
  * calls on blocks of this shape use.                                       */
 int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
                         double dt, enzoe_stream_t stream, int *mask_out);
@@ -725,7 +726,8 @@ int enzoe_vlct_transfer_batch(enzoe_vlct_t m, const enzoe_transfer *items,
  * launch that marches tiles of columns through the planes and keeps fluxes,
  * EMFs and faces on the chip (two-stage schemes, from 2^18 active cells of a
  * call on, FP64 hydro 3 2^17, where no debug counts, stored fluxes or
- * flux-launch shape are asked for), else the four launches.
+ * flux-launch shape are asked for), else variant 2 for MHD launches of fewer
+ * than 2^19 cells (ghost zones included), else the four launches.
  * Every variant gives the same bits in FP64 (the mixed and contracted
  * builds: up to the rounding of their contracted flux arithmetic, which the
  * compiler may fuse differently in different kernels).  Not to be changed
@@ -744,7 +746,8 @@ int enzoe_vlct_check_persistent(enzoe_vlct_t m);
  * through the planes with each plane's primitive states staged in LDS, so
  * a cell's state is loaded and converted about 1.1 times instead of 4
  * (the reconstructing stage as 0); -1 (the default), the autotuner's
- * choice per block shape (0 until it has run).  Every shape gives the same
+ * choice per block shape (until it has run, 1 for launches of fewer than 2^18
+ * cells, ghost zones included, else 0).  Every shape gives the same
  * bits in FP64; the mixed and contracted builds fuse their flux
  * multiply-adds as the compiler finds them in each kernel, so there the
  * shapes agree to the rounding of that arithmetic.                         */
