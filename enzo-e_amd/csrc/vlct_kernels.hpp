@@ -1632,6 +1632,12 @@ static __global__ void k_dt_init(unsigned long long *result) {
   *result = 0x7FEFFFFFFFFFFFFFull;  // numeric_limits<double>::max()
 }
 
+// The minimum word to the host (a pinned word), and ready for the next one.
+static __global__ void k_dt_out(unsigned long long *word, unsigned long long *host) {
+  __hip_atomic_store(host, *word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  *word = 0x7FEFFFFFFFFFFFFFull;
+}
+
 // dt of the cycle on the device: courant * min, clipped so the cycle ends
 // at t_stop (control_stopping.cpp:83-86, as the host driver clips), copied
 // into dts[0..n) for the compute launches; the time advances by dt.  A

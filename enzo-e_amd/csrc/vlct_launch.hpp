@@ -117,6 +117,11 @@ struct enzoe_vlct_method {
   size_t desc_bytes = 0;
   std::vector<char> last_desc;
   unsigned long long *d_dt = nullptr;
+  // the CFL minimum on its way to the host: a pinned word that k_dt_out
+  // writes (null: not allocated), and whether that kernel has left *d_dt
+  // ready for the next minimum
+  unsigned long long *h_dt = nullptr;
+  bool dt_ready = false;
   void *d_ptrtab = nullptr;
   size_t ptrtab_bytes = 0;
   std::vector<char> last_dt_desc;  // host copy of the dt descriptor table
