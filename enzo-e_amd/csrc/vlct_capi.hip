@@ -1015,6 +1015,7 @@ static int grid_refresh(enzoe_vlct_t m, const enzoe_block *blocks, int nbx, int 
   const int ncc = m->mhd ? 8 : 5;
   G.face0 = m->mhd ? ncc : (1 << 20);
   const int nf = ncc + (m->mhd ? 3 : 0) + (m->dual ? 1 : 0);
+  G.nf = nf;
   std::vector<double *> tab((size_t)nf * nb);
   for (int i = 0; i < nb; i++) {
     const enzoe_block &b = blocks[i];
@@ -1052,8 +1053,13 @@ static int grid_refresh(enzoe_vlct_t m, const enzoe_block *blocks, int nbx, int 
     }
     nghost = std::max(nghost, tot - in);
   }
-  hipLaunchKernelGGL(k_refresh, dim3(nblk(nghost, 256), nb, nf), dim3(256), 0, s,
-                     (double *const *)m->d_rtab, G);
+  const long elements =
+      (long)(G.n[0] + 2 * G.g + 1) * (G.n[1] + 2 * G.g + 1) * (G.n[2] + 2 * G.g + 1);
+  const int faces = m->mhd ? 3 : 0;
+  const dim3 grid(nblk(nghost, 256), nb, faces + (int)nblk(nf - faces, 2));
+  auto kernel = elements < (1L << 31) ? k_refresh<unsigned, 2>
+                                      : k_refresh<unsigned long, 2>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, (double *const *)m->d_rtab, G);
   if (hipGetLastError() != hipSuccess) return ENZOE_ERR_HIP;
   return ENZOE_OK;
 }

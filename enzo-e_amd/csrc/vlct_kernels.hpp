@@ -1673,6 +1673,7 @@ struct RefreshGrid {
   int bc[3];     // 0 periodic, 1 outflow
   int face0;     // table index of bfieldi_x (then _y, _z); every other
                  // field is cell-centred
+  int nf;        // fields of the table
   const double *dt;  // device dt of the cycle, or null: a cycle whose dt is
                      // 0 (past its stop time) refreshes nothing
 };
@@ -1711,56 +1712,63 @@ __device__ __forceinline__ bool refresh_axis(const RefreshGrid &G, int a,
 // Decodes the t-th ghost element of an (az, ay, ax) array whose interior is
 // [lo, hi) along each axis: z slabs first, then y slabs of the interior z
 // range, then x slabs of the interior (z, y) range.  Returns false past the
-// last ghost element.
-__device__ __forceinline__ bool ghost_coords(long t, const int ext[3],
-                                             const int lo[3], const int hi[3],
-                                             int &k, int &j, int &i) {
-  const int ax = ext[0], ay = ext[1], az = ext[2];
+// last ghost element.  I: unsigned where the array has fewer than 2^31
+// elements (a 64-bit division is a hundred instructions), else unsigned long.
+template <typename I>
+__device__ __forceinline__ bool ghost_coords(I t, const int ext[3], const int lo[3],
+                                             const int hi[3], int &k, int &j, int &i) {
+  const I ax = (I)ext[0], ay = (I)ext[1];
   const int nxi = hi[0] - lo[0], nyi = hi[1] - lo[1], nzi = hi[2] - lo[2];
-  const long plane = (long)ay * ax;
-  const long cz = (long)(az - nzi) * plane;
+  const I plane = ay * ax;
+  const I cz = (I)(ext[2] - nzi) * plane;
   if (t < cz) {
-    int pz = (int)(t / plane);
-    long r = t - (long)pz * plane;
-    k = pz < lo[2] ? pz : hi[2] + (pz - lo[2]);
-    j = (int)(r / ax);
-    i = (int)(r - (long)j * ax);
+    const I pz = t / plane, r = t - pz * plane, jj = r / ax;
+    k = (int)pz < lo[2] ? (int)pz : hi[2] + ((int)pz - lo[2]);
+    j = (int)jj;
+    i = (int)(r - jj * ax);
     return true;
   }
   t -= cz;
-  const long row = (long)(ay - nyi) * ax;
-  const long cy = (long)nzi * row;
+  const I row = (I)(ext[1] - nyi) * ax;
+  const I cy = (I)nzi * row;
   if (t < cy) {
-    int kk = (int)(t / row);
-    long r = t - (long)kk * row;
-    int py = (int)(r / ax);
-    k = lo[2] + kk;
-    j = py < lo[1] ? py : hi[1] + (py - lo[1]);
-    i = (int)(r - (long)py * ax);
+    const I kk = t / row, r = t - kk * row, py = r / ax;
+    k = lo[2] + (int)kk;
+    j = (int)py < lo[1] ? (int)py : hi[1] + ((int)py - lo[1]);
+    i = (int)(r - py * ax);
     return true;
   }
   t -= cy;
-  const int gx = ax - nxi;
-  const long cx = (long)nzi * nyi * gx;
-  if (t >= cx) return false;
-  long q = t / gx;
-  int px = (int)(t - q * gx);
-  k = lo[2] + (int)(q / nyi);
-  j = lo[1] + (int)(q % nyi);
+  const I gx = (I)(ext[0] - nxi);
+  if (gx == 0 || t >= (I)nzi * (I)nyi * gx) return false;
+  const I q = t / gx, kk = q / (I)nyi;
+  const int px = (int)(t - q * gx);
+  k = lo[2] + (int)kk;
+  j = lo[1] + (int)(q - kk * (I)nyi);
   i = px < lo[0] ? px : hi[0] + (px - lo[0]);
   return true;
 }
 
 // table[f * nb + b] = device pointer of field f of block b; fields
 // face0..face0+2 are the face-centred bfieldi_x..z, the others cell-centred.
-// grid: x = ghost elements, y = block, z = field.
+// grid: x = ghost elements, y = block, z = the face fields (MHD), then the
+// cell-centred ones, PER of them to a thread.
+// Bound by the lines it touches: an x ghost run is 3 cells, 24 bytes of a
+// 128-byte line on either side, which makes 14 GB of 512 64^3 MHD blocks'
+// 7.3 (64 of them: 0.36 ms, 5 TB/s of lines).  Two fields to a thread with
+// 32-bit indices share the index arithmetic, about a dozen divisions, and
+// keep two loads in flight.  One 64^3 x 64 MHD grid / 128^3 x 8 hydro / one
+// 16^3 hydro block: one field a thread with 64-bit indices 411 / 102 / 7.8
+// us, 32-bit 398 / 99 / 6.3, two fields 359 / 83 / 6.5, four 362 / 79 / 8.1,
+// eight 372 / 78 / 13.4 (too few waves for the latency of one block).
+template <typename I, int PER>
 static __global__ void __launch_bounds__(256)
 k_refresh(double *const *__restrict__ table, RefreshGrid G) {
   if (G.dt != nullptr && *G.dt == 0.0) return;
   const int nb = G.nb[0] * G.nb[1] * G.nb[2];
   const int bidx = blockIdx.y;
-  const int f = blockIdx.z;
-  const int fc = (f >= G.face0 && f < G.face0 + 3) ? f - G.face0 : -1;
+  const int faces = G.nf > G.face0 ? 3 : 0;
+  const int fc = (int)blockIdx.z < faces ? (int)blockIdx.z : -1;
   const int bx = bidx % G.nb[0];
   const int by = (bidx / G.nb[0]) % G.nb[1];
   const int bz = bidx / (G.nb[0] * G.nb[1]);
@@ -1771,16 +1779,33 @@ k_refresh(double *const *__restrict__ table, RefreshGrid G) {
     hi[a] = G.g + G.n[a] + (fc == a);
   }
   int k, j, i;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (!ghost_coords(t, ext, lo, hi, k, j, i)) return;
+  const I t = (I)blockIdx.x * blockDim.x + threadIdx.x;
+  if (!ghost_coords<I>(t, ext, lo, hi, k, j, i)) return;
   int sb[3], si[3];
   refresh_axis(G, 0, bx, i, fc == 0, sb[0], si[0]);
   refresh_axis(G, 1, by, j, fc == 1, sb[1], si[1]);
   refresh_axis(G, 2, bz, k, fc == 2, sb[2], si[2]);
   const int sbid = (sb[2] * G.nb[1] + sb[1]) * G.nb[0] + sb[0];
-  double *const *tab = table + (size_t)f * nb;
-  tab[bidx][idx3(k, j, i, ext[1], ext[0])] =
-      tab[sbid][idx3(si[2], si[1], si[0], ext[1], ext[0])];
+  const long dst = idx3(k, j, i, ext[1], ext[0]);
+  const long src = idx3(si[2], si[1], si[0], ext[1], ext[0]);
+  if (fc >= 0) {
+    double *const *tab = table + (size_t)(G.face0 + fc) * nb;
+    gst(tab[bidx], dst, gld(tab[sbid] + src, 0));
+    return;
+  }
+  // (a launch writes ghosts and reads active cells: no element is both)
+  const int q0 = ((int)blockIdx.z - faces) * PER, ncc = G.nf - faces;
+  double v[PER];
+#pragma unroll
+  for (int q = 0; q < PER; q++) {
+    const int f = q0 + q < G.face0 ? q0 + q : q0 + q + faces;
+    if (q0 + q < ncc) v[q] = gld(table[(size_t)f * nb + sbid] + src, 0);
+  }
+#pragma unroll
+  for (int q = 0; q < PER; q++) {
+    const int f = q0 + q < G.face0 ? q0 + q : q0 + q + faces;
+    if (q0 + q < ncc) gst(table[(size_t)f * nb + bidx], dst, v[q]);
+  }
 }
 
 // ------------------------------------------------------- flux corrections

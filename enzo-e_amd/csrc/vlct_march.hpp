@@ -1003,9 +1003,9 @@ k_shell(const BlockDesc<FluxT> *__restrict__ blocks, StageParams sp) {
     h[a] = m[a] - lo - 1 - blo;
   }
   int k, j, i;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
   double local = 1.7976931348623157e308;
-  if (ghost_coords(t, ext, l, h, k, j, i)) {
+  if (ghost_coords<unsigned>(t, ext, l, h, k, j, i)) {
     k += blo;
     j += blo;
     i += blo;

@@ -182,3 +182,41 @@ def test_marched_cycles_on_the_device_and_from_a_graph_equal_host_driven_ones():
         for k in a:
             if k != "pressure":
                 assert np.array_equal(a[k][s], b[k][s]), k
+
+
+@pytest.mark.parametrize("mhd,dual", [(True, False), (True, True), (False, False), (False, True)])
+@pytest.mark.parametrize("n,nblocks,bc", [
+    ((5, 4, 3), (2, 1, 3), "periodic"), ((2, 7, 1), (3, 2, 1), "periodic"),
+    ((33, 18, 9), (1, 2, 2), "periodic"), ((6, 5, 7), (1, 1, 1), "outflow")])
+def test_refresh_copies_every_field(n, nblocks, bc, mhd, dual):
+    """The refresh, two fields to a thread: every ghost element of every
+    field against the index arithmetic in numpy, also for blocks thinner
+    than the ghost zone, with an odd number of fields."""
+    ev = _ev()
+    count = nblocks[0] * nblocks[1] * nblocks[2]
+    states = [_state(n, 40 + i, dual, mhd) for i in range(count)]
+    blocks = _blocks(ev, n, states, count, dual, mhd)
+    m = ev.VlctMethod(mhd=mhd, riemann="hlld" if mhd else "hllc",
+                      dual_energy_eta=0.001 if dual else None)
+    m.refresh(blocks, nblocks, (bc,) * 3)
+    got = [b.download() for b in blocks]
+    for i in range(count):
+        at = (i % nblocks[0], i // nblocks[0] % nblocks[1], i // nblocks[0] // nblocks[1])
+        for name, x in got[i].items():
+            if name == "pressure":  # derived, not refreshed
+                continue
+            src, idx = [], []
+            for a in range(3):      # x, y, z
+                face = name == "bfieldi_" + "xyz"[a]
+                N = n[a] * nblocks[a]
+                e = np.arange(n[a] + 2 * G + face)
+                p = at[a] * n[a] + e - G
+                inside = (e >= G) & (e < G + n[a] + face)
+                q = p % N if bc == "periodic" else np.clip(p, 0, N - 1 + face)
+                last = face & (q == N)
+                src.append(np.where(inside, at[a], np.where(last, nblocks[a] - 1, q // n[a])))
+                idx.append(np.where(inside, e, np.where(last, G + n[a], q % n[a] + G)))
+            b = (src[2][:, None, None] * nblocks[1] + src[1][:, None]) * nblocks[0] + src[0]
+            want = np.stack([s[name] for s in states])[
+                b, idx[2][:, None, None], idx[1][:, None], idx[0]]
+            assert np.array_equal(x, want), (i, name)
