@@ -682,27 +682,33 @@ MarchParams march_tiling(int mx, int my, int mz, int cs, int nb, int cus, double
   return p;
 }
 
-template <typename T, int RECON, int RIEMANN, bool DE, bool HALF, int NT>
+template <typename T, int RECON, int RIEMANN, bool DE, bool HALF, int NT, int WAVES>
 void launch_march_nt(const BlockDesc<T> *d, const MarchParams &mp, const StageParams &sp,
                      hipStream_t s) {
   const unsigned wgs = (unsigned)((mp.total + mp.share - 1) / mp.share);
-  hipLaunchKernelGGL((k_march<T, RECON, RIEMANN, DE, HALF, NT>), dim3((wgs + 7u) & ~7u),
+  hipLaunchKernelGGL((k_march<T, RECON, RIEMANN, DE, HALF, NT, WAVES>), dim3((wgs + 7u) & ~7u),
                      dim3(NT), 0, s, d, sp, mp);
 }
 // One marched stage: 512-thread tiles, one a CU, or 256-thread ones, two a
 // CU, whichever covers the blocks' planes in less time (the smaller tile
-// repeats more of its ring but fits small blocks better).
+// repeats more of its ring but fits small blocks better).  The mixed
+// nearest-neighbour march fits three waves a SIMD (168 registers, 120 KB of
+// LDS): 768-thread tiles or three of 256.  Its Orszag-Tang 256^3 stage took
+// 1.20 ms with two waves, 1.09 with three; the reconstructing one would spill
+// 36 registers.
 template <typename T, int RECON, int RIEMANN, bool DE, bool HALF>
 void launch_march(const BlockDesc<T> *d, int nb, int mx, int my, int mz, const StageParams &sp,
                   hipStream_t s) {
   const int cus = device_cus();
   double big, small;
-  const MarchParams p5 = march_tiling<512, 1>(mx, my, mz, sp.cur_stale, nb, cus, big);
-  const MarchParams p2 = march_tiling<256, 2>(mx, my, mz, sp.cur_stale, nb, cus, small);
+  constexpr int W = std::is_same<T, float>::value && RECON == RC_NN && !DE ? 3 : 2;
+  constexpr int NT = 256 * W;
+  const MarchParams p5 = march_tiling<NT, 1>(mx, my, mz, sp.cur_stale, nb, cus, big);
+  const MarchParams p2 = march_tiling<256, W>(mx, my, mz, sp.cur_stale, nb, cus, small);
   if (big <= small)
-    launch_march_nt<T, RECON, RIEMANN, DE, HALF, 512>(d, p5, sp, s);
+    launch_march_nt<T, RECON, RIEMANN, DE, HALF, NT, W>(d, p5, sp, s);
   else
-    launch_march_nt<T, RECON, RIEMANN, DE, HALF, 256>(d, p2, sp, s);
+    launch_march_nt<T, RECON, RIEMANN, DE, HALF, 256, W>(d, p2, sp, s);
 }
 template <typename T, int RIEMANN, bool DE>
 void dispatch_march(int recon, const BlockDesc<T> *d, int nb, int mx, int my, int mz,

@@ -24,12 +24,15 @@
 // 2020 (nearest neighbour) and 2400 (PLM) VALU instructions a column and
 // plane, a quarter of them for the rings (512 threads of 34 x 15 columns
 // cover 32 x 13 cells), at about two thirds of the issue rate; the rest is
-// waiting at the 4 (NN) or 7 (PLM) barriers of a plane (taken out in a copy,
-// PLM ran 16% faster) and on dependent operations with two waves a SIMD, all
-// that 256 registers and 119 or 143 KB of LDS allow.  Orszag-Tang 256^3,
-// FP64: 1.88 + 2.60 ms for the two stages against 3.19 + 3.82 of the separate
-// launches; mixed 1.31 + 1.77 against 2.35 + 2.23; 64 turbulence blocks of
-// 64^3: 2.28 + 2.72 against 3.87 + 4.19 (FP64).
+// waiting at the 4 (NN) or 6 (PLM) barriers of a plane and on dependent
+// operations with two waves a SIMD, all that 256 registers and 119 or 147 KB
+// of LDS allow.  The mixed path has registers over, and waits for memory and
+// on dependent operations too: three waves a SIMD in its first stage, one
+// barrier and a load of the column's cell less (LATE, CARRY below).
+// Orszag-Tang 256^3, FP64: 1.88 + 2.60 ms for the two stages against 3.19 +
+// 3.82 of the separate launches; mixed 1.09 + 1.64 against 2.35 + 2.23; 64
+// turbulence blocks of 64^3: 2.28 + 2.72 against 3.87 + 4.19 (FP64), 1.43 +
+// 1.79 (mixed).
 #pragma once
 
 #include "vlct_kernels.hpp"
@@ -53,8 +56,9 @@ struct MarchParams {
 };
 
 // Cells of the LDS plane of a reconstructing march (the tile, its ring and
-// one more cell around).
-constexpr int march_plane_cells(int nt) { return nt + nt / 4; }
+// one more cell around; one less than 5/4 of the threads: with dual energy
+// the FP64 march fills the 160 KB).
+constexpr int march_plane_cells(int nt) { return nt + nt / 4 - 1; }
 
 // dU - dtdx (F_hi - F_lo), never contracted (cell_stage's divergence).
 __device__ __forceinline__ double flux_difference(double dU, double dtdx, double hi, double lo) {
@@ -240,14 +244,14 @@ __device__ __forceinline__ bool march_ring(int r, int w2, int h2, int &rx, int &
 }
 
 // Launch: total / share workgroups (rounded up to a multiple of 8) of NT
-// threads; the XCD-contiguous order of wg_coords.  T is the arithmetic and flux type (float: the mixed
-// path).  HALF: the stage reads the half-step state, which the first stage
+// threads, WAVES waves to a SIMD; the XCD-contiguous order of wg_coords.  T
+// is the arithmetic and flux type (float: the mixed path).  HALF: the stage reads the half-step state, which the first stage
 // stored as primitives (mixed path: FP32 and the FP64 centre E beside
 // them; FP64: with the pressure in the place of the total energy); the
 // first stage of the VL scheme is the nearest-neighbour one and reads the
 // start-of-step state.
-template <typename T, int RECON, int RIEMANN, bool DE, bool HALF, int NT>
-__global__ void __launch_bounds__(NT, 2)
+template <typename T, int RECON, int RIEMANN, bool DE, bool HALF, int NT, int WAVES>
+__global__ void __launch_bounds__(NT, WAVES)
 k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp) {
   constexpr bool PLM = RECON != RC_NN;
   constexpr bool F32 = std::is_same<T, float>::value;
@@ -257,6 +261,14 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
   // the stage that reads the half-step state is the final one; the debug
   // counts take the separate launches
   constexpr bool FINAL = HALF;
+  // Mixed path, whose FP32 solves leave registers over: the cell k + 1 stays
+  // in registers until it is the plane's (CARRY; FP64 would spill, and loads
+  // it twice, a plane apart), and the cell update comes after the barrier
+  // that ends the plane instead of a barrier of its own (LATE; in FP64 the
+  // same time with and without spills).  Orszag-Tang 256^3, second stage: 1.77
+  // ms with neither, 1.73 LATE, 1.64 both; first stage 1.30, 1.20 LATE, 1.085
+  // with three waves a SIMD as well.
+  constexpr bool LATE = F32, CARRY = PLM && F32;
   sp.stage = sp.is_final = FINAL ? 1 : 0;
   sp.dbg = nullptr;
   if (!FINAL) sp.cfl = nullptr;
@@ -272,23 +284,27 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
   fc.pfloor = sp.pressure_floor;
   fc.dbg = nullptr;
   const T theta = (T)sp.theta;
-  // LDS.  sW: the plane's primitives; sF: face quantities by slot; sEc: the
-  // centre E of plane k; sX: the right states on their way to the
-  // neighbour, later the edge EMFs.  The face B of plane k - 1 takes the
-  // first slots of sF, whose values (FZ*, FXB) are spent by then.
+  // LDS.  sW: the plane's primitives; sEc: the centre E of plane k; sF: the z
+  // and x face quantities by slot; sX: the x right states on their way to the
+  // neighbour, then the y fluxes; sP: the y right states, then the edge EMFs
+  // (sE).  sB, the face B of plane k - 1: with LATE behind sE, else in the
+  // first rows of sF, whose values (FZ*, FXB) are spent by then.  What takes
+  // an area's place is written at least one barrier after its last read.
   constexpr int WN = PLM ? march_plane_cells(NT) : NT;
-  enum { FZD, FZBX, FZBY, FXB, FYB, FX0, FY0 = FX0 + 5, FN = FY0 + 5 };
-  constexpr int XB = PLM && 7 * sizeof(T) > 24 ? 7 * sizeof(T) : 24;
+  enum { FZD, FZBX, FZBY, FXB, FX0, FN = FX0 + 5 };
+  enum { FY0, FYB = FY0 + 5, FYN };
+  constexpr int EB = LATE ? 40 : 24, PB = PLM && 7 * sizeof(T) > EB ? 7 * sizeof(T) : EB;
   __shared__ T sW[S_N][WN];
-  __shared__ __align__(16) T sF[FN][NT];
+  __shared__ __align__(16) T sF[PLM ? FN : FN + FYN][NT];
   __shared__ double sEc[3][NT];
-  __shared__ __align__(16) char sX[XB * NT];
+  __shared__ T sXs[PLM ? S_N - 1 : 1][PLM ? NT : 1];
+  __shared__ __align__(16) char sP[PB * NT];
   __shared__ double sD[DE ? 4 : 1][DE ? NT : 1];
-  __shared__ unsigned long long wmin[NT / 64];
   __shared__ int sWild;
-  T(*sR)[NT] = reinterpret_cast<T(*)[NT]>(sX);
-  double(*sE)[NT] = reinterpret_cast<double(*)[NT]>(sX);
-  double(*sB)[NT] = reinterpret_cast<double(*)[NT]>(&sF[0][0]);
+  T(*sY)[NT] = reinterpret_cast<T(*)[NT]>(sP);
+  double(*sE)[NT] = reinterpret_cast<double(*)[NT]>(sP);
+  double(*sB)[NT] = LATE ? sE + 3 : reinterpret_cast<double(*)[NT]>(&sF[0][0]);
+  T(*sX)[NT] = PLM ? reinterpret_cast<T(*)[NT]>(&sXs[0][0]) : &sF[FN];
 
   const int tid = (int)threadIdx.x;
   const int w2 = mp.w2, h2 = mp.h2;
@@ -359,7 +375,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
     T Lz[S_N], wm[S_N], wp[S_N];
     T Fz[5];
     T FxBz = T(0), FyBz = T(0), FxD = T(0), FyD = T(0);
-    double dU[5], dUe = 0., pc = 0.;
+    double dU[5], dUe = 0., pc = 0.;  // of the cell of plane k - 1
     T FzE = T(0), FzV = T(0);
     double ecx0 = 0., ecx1 = 0., ecy0 = 0., ecy1 = 0.;
     double Ex = 0., Ey = 0., Ez = 0., Bz = 0.;
@@ -471,7 +487,8 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
       // state in L, the neighbour's right state in R (lo / hi: sW of the
       // cells before and after, nb: the neighbour column, SKIP: the slot of
       // the normal B)
-      auto exchange = [&](auto skip_slot, int lo, int hi, int nb, T L[S_N], T R[S_N]) {
+      auto exchange = [&](auto skip_slot, T(*sR)[NT], int lo, int hi, int nb, T L[S_N],
+                          T R[S_N]) {
         constexpr int SKIP = decltype(skip_slot)::value;
         if constexpr (PLM) {
           auto states = [&](auto ex) {
@@ -504,7 +521,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
       T FxBz_k, FyBz_k;
       {
         T L[S_N], R[S_N];
-        exchange(std::integral_constant<int, S_BX>(), wi - 1, wxp, xp, L, R);
+        exchange(std::integral_constant<int, S_BX>(), sX, wi - 1, wxp, xp, L, R);
         FaceFlux<T> f;
         solve_face<T, RIEMANN, true, 0, DE>(L, R, (T)fbx, fc, f);
 #pragma unroll
@@ -519,22 +536,21 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
       // ---- y: the face towards j + 1
       {
         T L[S_N], R[S_N];
-        if constexpr (PLM) lds_barrier();  // the x states have been read
-        exchange(std::integral_constant<int, S_BY>(), wi - ws, wyp, yp, L, R);
+        exchange(std::integral_constant<int, S_BY>(), sY, wi - ws, wyp, yp, L, R);
         FaceFlux<T> f;
         solve_face<T, RIEMANN, true, 1, DE>(L, R, (T)fby, fc, f);
 #pragma unroll
-        for (int q = 0; q < 5; q++) sF[FY0 + q][tid] = f.u[q];
+        for (int q = 0; q < 5; q++) sX[FY0 + q][tid] = f.u[q];
         FyBz_k = f.bj;
-        sF[FYB][tid] = f.bk;
+        sX[FYB][tid] = f.bk;
         if (DE) {
           sD[2][tid] = (double)f.e;
           sD[3][tid] = (double)f.vb;
         }
       }
       // loads for the rest of this step and for the next plane go out now (the
-      // reconstruction loads the column's cell twice, a plane apart, instead
-      // of keeping it through the solves: 16 registers)
+      // FP64 reconstruction loads the column's cell twice, a plane apart,
+      // instead of keeping it through the solves: 16 registers)
       const unsigned kn = (unsigned)((k + 1 < mz) ? k + 1 : mz - 1);
       const unsigned ku = (unsigned)(k > 0 ? k - 1 : 0);  // the plane to update
       const unsigned cn = kn * plane + col;
@@ -544,17 +560,19 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
       const unsigned fzk = (unsigned)k * plane + col;
       const bool face_step = k >= ks;  // the level below plane k
       const bool cell_step = k > ks;   // plane k - 1
-      // (the update's base first: it is needed first)
       const double b0z = ldo(bf0[2], fzk), b0x = ldo(bf0[0], fxu), b0y = ldo(bf0[1], fyu);
       CellBase u0;
-      u0.rho = ldo(b.U[S_RHO], cu);
-      u0.v[0] = ldo(b.U[S_VX], cu);
-      u0.v[1] = ldo(b.U[S_VY], cu);
-      u0.v[2] = ldo(b.U[S_VZ], cu);
-      u0.e = ldo(b.U[S_E], cu);
-      if (DE) u0.ei = ldo(b.ei, cu);
+      auto load_base = [&]() {
+        u0.rho = ldo(b.U[S_RHO], cu);
+        u0.v[0] = ldo(b.U[S_VX], cu);
+        u0.v[1] = ldo(b.U[S_VY], cu);
+        u0.v[2] = ldo(b.U[S_VZ], cu);
+        u0.e = ldo(b.U[S_E], cu);
+        if (DE) u0.ei = ldo(b.ei, cu);
+      };
+      if constexpr (!LATE) load_base();
       RawCell<T, DE, HALF> nxt, nx2, halo;
-      march_load<true>(b, cn, nxt);
+      if constexpr (!CARRY) march_load<true>(b, cn, nxt);
       fbx = ldo(bfr[0], kn * planex + colx);
       fby = ldo(bfr[1], kn * planey + coly);
       fbz = ldo(bfr[2], cn);
@@ -572,10 +590,10 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
       // ---- E: edge EMFs
       const double Ex_b = Ex, Ey_b = Ey, Ez_b = Ez;  // levels k - 3/2, plane k - 1
       {
-        const double dxm = (double)sF[FX0][tid], dym = (double)sF[FY0][tid];
+        const double dxm = (double)sF[FX0][tid], dym = (double)sX[FY0][tid];
         Ez = edge_value(sEc[2][tid], sEc[2][xp], sEc[2][yp], sEc[2][xyp], (double)sF[FXB][tid],
-                        (double)sF[FXB][yp], (double)sF[FYB][tid], (double)sF[FYB][xp], dxm,
-                        (double)sF[FX0][yp], dym, (double)sF[FY0][xp]);
+                        (double)sF[FXB][yp], (double)sX[FYB][tid], (double)sX[FYB][xp], dxm,
+                        (double)sF[FX0][yp], dym, (double)sX[FY0][xp]);
         const double cx0 = sEc[0][tid], cx1 = sEc[0][yp], cy0 = sEc[1][tid], cy1 = sEc[1][xp];
         if (face_step) {
           const double dz = (double)sF[FZD][tid];
@@ -619,9 +637,9 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
           if (!FINAL) sto(b.bf0[1], fyu, b0y);
         }
       }
-      lds_barrier();
       // ---- U: the cell of plane k - 1
-      if (cell_step && upd) {
+      auto update = [&]() {
+        if (!cell_step || !upd) return;
         const double bc[3] = {half_sum(sB[0][xm], Bx), half_sum(sB[1][ym], By),
                               half_sum(Bz_b, Bz)};
         if (!F32 || FINAL) {
@@ -632,25 +650,35 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
         }
         const double t = cell_finish<T, true, DE, true>(b, sp, dt, CellOffset{cu}, u0, dU, dUe, bc);
         local = t < local ? t : local;
+      };
+      if constexpr (!LATE) {
+        lds_barrier();
+        update();
       }
       // ---- the x and y parts of plane k's divergence
+      double dUn[5], dUen = 0., pcn = 0.;
 #pragma unroll
       for (int q = 0; q < 5; q++) {
-        dU[q] = flux_difference(0., dtdx, (double)sF[FX0 + q][tid], (double)sF[FX0 + q][xm]);
-        dU[q] = flux_difference(dU[q], dtdy, (double)sF[FY0 + q][tid], (double)sF[FY0 + q][ym]);
+        dUn[q] = flux_difference(0., dtdx, (double)sF[FX0 + q][tid], (double)sF[FX0 + q][xm]);
+        dUn[q] = flux_difference(dUn[q], dtdy, (double)sX[FY0 + q][tid], (double)sX[FY0 + q][ym]);
       }
       if (DE) {
-        pc = dmax((double)sW[S_E][wi], sp.pressure_floor);
-        dUe = flux_difference(0., dtdx, sD[0][tid], sD[0][xm]);
-        dUe = source_difference(dUe, dtdx, pc, sD[1][tid], sD[1][xm]);
-        dUe = flux_difference(dUe, dtdy, sD[2][tid], sD[2][ym]);
-        dUe = source_difference(dUe, dtdy, pc, sD[3][tid], sD[3][ym]);
+        pcn = dmax((double)sW[S_E][wi], sp.pressure_floor);
+        dUen = flux_difference(0., dtdx, sD[0][tid], sD[0][xm]);
+        dUen = source_difference(dUen, dtdx, pcn, sD[1][tid], sD[1][xm]);
+        dUen = flux_difference(dUen, dtdy, sD[2][tid], sD[2][ym]);
+        dUen = source_difference(dUen, dtdy, pcn, sD[3][tid], sD[3][ym]);
       }
       // ---- the next plane into LDS
       {
         T w[S_N];
         double ec[3];
-        march_prim<true>(nxt, fc.gm1, w);
+        if constexpr (CARRY) {
+#pragma unroll
+          for (int q = 0; q < S_N; q++) w[q] = wp[q];
+        } else {
+          march_prim<true>(nxt, fc.gm1, w);
+        }
         if constexpr (F32 && HALF) {
 #pragma unroll
           for (int a = 0; a < 3; a++) ec[a] = echn[a];
@@ -676,10 +704,18 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
 #pragma unroll
         for (int a = 0; a < 3; a++) sEc[a][tid] = ec[a];
       }
+      if constexpr (LATE) load_base();
       lds_barrier();
+      if constexpr (LATE) update();  // (the next solves cover its stores)
+#pragma unroll
+      for (int q = 0; q < 5; q++) dU[q] = dUn[q];
+      dUe = dUen;
+      pc = pcn;
     }
   }
-  if (sp.cfl != nullptr) march_min_to<NT>(sp.cfl, local, wmin);
+  // (sF: last read before the barrier that ended the last plane)
+  if (sp.cfl != nullptr)
+    march_min_to<NT>(sp.cfl, local, reinterpret_cast<unsigned long long *>(&sF[0][0]));
 }
 
 // The hydrodynamic march: as k_march, with the HLLC solve and without
