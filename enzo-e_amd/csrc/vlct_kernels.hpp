@@ -398,14 +398,14 @@ __device__ __forceinline__ void solve_face(const T wl[S_N], const T wr[S_N], T b
 // Flux through the face between cell c and c + e_D (D fixed at compile
 // time so the i/j/k permutation costs nothing): reconstruction of both
 // sides, the face-centred normal B (EnzoBfieldMethodCT.cpp:122-166) and the
-// Riemann solve, written at index c of the flux arrays of dim D.
+// Riemann solve (face_flux), written at index c of the flux arrays of dim D
+// (flux_face).
 template <typename T, typename FluxT, int RECON, int RIEMANN, bool MHD, int D,
           bool DE, bool PRIMF, class Src = PrimSource<T, MHD, DE, PRIMF>>
-__device__ __forceinline__ void flux_face(const BlockDesc<FluxT> &b, const Src &src,
+__device__ __forceinline__ void face_flux(const BlockDesc<FluxT> &b, const Src &src,
                                           const double *bfi, int k, int j,
                                           int i, int c, const T wc[S_N],
-                                          const FluxConsts &fc) {
-  constexpr int DJ = (D + 1) % 3, DK = (D + 2) % 3;
+                                          const FluxConsts &fc, FaceFlux<T> &f) {
   const int s = (D == 0) ? 1 : ((D == 1) ? b.mx : b.mx * b.my);
   T wl[S_N], wr[S_N];
   if (RECON == RC_NN) {
@@ -451,8 +451,17 @@ __device__ __forceinline__ void flux_face(const BlockDesc<FluxT> &b, const Src &
     const int bnx = b.mx + (D == 0), bny = b.my + (D == 1);
     bface = (T)gld(bfi, (k + (D == 2)) * bny * bnx + (j + (D == 1)) * bnx + i + (D == 0));
   }
-  FaceFlux<T> f;
   solve_face<T, RIEMANN, MHD, D, DE>(wl, wr, bface, fc, f);
+}
+template <typename T, typename FluxT, int RECON, int RIEMANN, bool MHD, int D,
+          bool DE, bool PRIMF, class Src = PrimSource<T, MHD, DE, PRIMF>>
+__device__ __forceinline__ void flux_face(const BlockDesc<FluxT> &b, const Src &src,
+                                          const double *bfi, int k, int j,
+                                          int i, int c, const T wc[S_N],
+                                          const FluxConsts &fc) {
+  constexpr int DJ = (D + 1) % 3, DK = (D + 2) % 3;
+  FaceFlux<T> f;
+  face_flux<T, FluxT, RECON, RIEMANN, MHD, D, DE, PRIMF>(b, src, bfi, k, j, i, c, wc, fc, f);
 #pragma unroll
   for (int q = 0; q < 5; q++) gst(b.F[D][q], c, (FluxT)f.u[q]);
   if (MHD) {
@@ -1076,10 +1085,30 @@ __device__ __forceinline__ double cell_finish(const BlockDesc<FluxT> &b, const S
 // face_b(k, j, i, f[6]) gives the cell's six face values of the stage's
 // face-centred B (low and high face along x, y, z).  Returns the cell's CFL
 // term (DBL_MAX when it takes none).
-template <typename FluxT, bool MHD, bool DE, typename FaceB>
+// flux: the cell's fluxes through its low and high face along an axis.
+template <typename FluxT>
+struct FluxGlobal {
+  const BlockDesc<FluxT> &b;
+  __device__ __forceinline__ void operator()(int d, int q, long c, long s, double &lo,
+                                             double &hi) const {
+    const int fq[5] = {S_RHO, S_VX, S_VY, S_VZ, S_E};
+    const FluxT *F = b.F[d][fq[q]];
+    hi = (double)F[c];
+    lo = (double)F[c - s];
+  }
+  __device__ __forceinline__ void energy(int d, long c, long s, double &elo, double &ehi,
+                                         double &vlo, double &vhi) const {
+    ehi = b.Fe[d][c];
+    elo = b.Fe[d][c - s];
+    vhi = b.Vb[d][c];
+    vlo = b.Vb[d][c - s];
+  }
+};
+template <typename FluxT, bool MHD, bool DE, typename FaceB, class Flux = FluxGlobal<FluxT>>
 __device__ __forceinline__ double cell_stage(const BlockDesc<FluxT> &b, const StageParams &sp,
                                              int by, int k, int j, int i, bool in_launch,
-                                             bool in_box, const FaceB &face_b) {
+                                             bool in_box, const FaceB &face_b,
+                                             const Flux &flux) {
   // the FP64 update is never contracted into FMAs, also where the including
   // unit allows it: every kernel that runs it (k_cells, k_ctu, k_stage)
   // rounds alike
@@ -1139,7 +1168,6 @@ __device__ __forceinline__ double cell_stage(const BlockDesc<FluxT> &b, const St
     }
     const double dt = sp.dts ? sp.dts[by] * sp.dt_factor : sp.dt;
     const long str[3] = {1, (long)mx, (long)mx * my};
-    const int fq[5] = {S_RHO, S_VX, S_VY, S_VZ, S_E};
     double dU[5];
   #pragma unroll
     for (int q = 0; q < 5; q++) dU[q] = 0.;
@@ -1157,13 +1185,15 @@ __device__ __forceinline__ double cell_stage(const BlockDesc<FluxT> &b, const St
       const double dtdx = dt / b.cw[d];
   #pragma unroll
       for (int q = 0; q < 5; q++) {
-        const FluxT *F = b.F[d][fq[q]];
-        double fr = (double)F[c], fl = (double)F[c - str[d]];
+        double fr, fl;
+        flux(d, q, c, str[d], fl, fr);
         dU[q] -= dtdx * (fr - fl);
       }
       if (DE) {
-        dUe -= dtdx * (b.Fe[d][c] - b.Fe[d][c - str[d]]);
-        dUe -= dtdx * pc * (b.Vb[d][c] - b.Vb[d][c - str[d]]);
+        double el, er, vl, vr;
+        flux.energy(d, c, str[d], el, er, vl, vr);
+        dUe -= dtdx * (er - el);
+        dUe -= dtdx * pc * (vr - vl);
       }
     }
     CellBase u0;
@@ -1245,7 +1275,8 @@ __device__ __forceinline__ void update_cells(const BlockDesc<FluxT> *__restrict_
   const bool in_box = in_launch && k >= lo && j >= lo && i >= lo && k < mz - lo &&
                       j < my - lo && i < mx - lo;
   const FaceBGlobal<FluxT> fb{b, sp.is_final ? b.bfi : b.bft};
-  const double local = cell_stage<FluxT, MHD, DE>(b, sp, by, k, j, i, in_launch, in_box, fb);
+  const double local = cell_stage<FluxT, MHD, DE>(b, sp, by, k, j, i, in_launch, in_box, fb,
+                                                    FluxGlobal<FluxT>{b});
   if (cfl) block_min_to(sp.cfl, local);
 }
 template <typename FluxT, bool MHD, bool DE = false>
@@ -1565,7 +1596,8 @@ k_ctu(const BlockDesc<FluxT> *__restrict__ blocks, StageParams sp) {
   const bool in_box = in_launch && k >= lo && j >= lo && i >= lo && k < mz - lo &&
                       j < my - lo && i < mx - lo;
   const FaceBLds<Tile> fb{sF, o};
-  const double local = cell_stage<FluxT, true, DE>(b, sp, by, k, j, i, in_launch, in_box, fb);
+  const double local = cell_stage<FluxT, true, DE>(b, sp, by, k, j, i, in_launch, in_box, fb,
+                                                    FluxGlobal<FluxT>{b});
   if (cfl) block_min_to(sp.cfl, local);
 }
 

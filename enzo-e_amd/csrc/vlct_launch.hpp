@@ -780,6 +780,44 @@ void dispatch_march_hd(int recon, const BlockDesc<T> *d, int nb, int mx, int my,
     launch_march_hd<T, RC_PLM_ATHENA, DE, true>(d, nb, mx, my, mz, sp, s);
 }
 
+// Whether a hydrodynamic stage of small blocks is one launch of k_tile: no
+// debug counts (the faces between tiles are solved twice), no structure or
+// flux-launch shape asked for or tuned, and fewer than 2^16 cells with ghosts (dual
+// energy: 2^15), where a launch costs more than the repeated faces.  Cycle in
+// us, separate and tiled -- FP64: one block of 12^3 38.4, 36.0; 16^3 39.1,
+// 36.1; 24^3 41.7, 37.0; 32^3 (54872 cells) 48.4, 45.7; 8 of 16^3 (85184)
+// 54.8, 57.5; 48^3 65.9, 70.8.  Dual energy: 24^3 44.2, 38.6; 32^3 51.9, 52.3.
+// Mixed: 16^3 35.8, 30.8; 32^3 40.2, 36.7; 8 of 16^3 46.5, 46.0.
+inline bool tile_ok(const enzoe_vlct_method *m, int mx, int my, int mz, int nb) {
+  if (m->mhd || m->d_dbg || m->force_ctu >= 0 || m->force_shape >= 0 || m->ctu >= 0 ||
+      m->flux_shape >= 0 || m->tuned_ctu.count(shape_key(mx, my, mz)) ||
+      std::min(mx, std::min(my, mz)) < 7)
+    return false;
+  return (long)mx * my * mz * nb < (m->dual ? 1L << 15 : 1L << 16);
+}
+template <typename FluxT, bool DE>
+void dispatch_tile(int recon, bool primf, const BlockDesc<FluxT> *d, int nb, int mx, int my,
+                   int mz, int lo, const StageParams &sp, hipStream_t s) {
+  using Tile = FluxTile<FluxT>;
+  const dim3 grid(((mx - 2 * lo + Tile::TX - 1) / Tile::TX) *
+                      ((my - 2 * lo + Tile::TY - 1) / Tile::TY) *
+                      ((mz - 2 * lo + Tile::TZ - 1) / Tile::TZ),
+                  nb);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(576), 0, s, d, sp);
+  };
+  constexpr bool F32 = half_f32<FluxT>(DE ? 1 : 0);
+  if (F32 && primf) {
+    if (recon == RC_NN) launch(k_tile<FluxT, FluxT, RC_NN, DE, F32>);
+    else if (recon == RC_PLM) launch(k_tile<FluxT, FluxT, RC_PLM, DE, F32>);
+    else launch(k_tile<FluxT, FluxT, RC_PLM_ATHENA, DE, F32>);
+  } else {
+    if (recon == RC_NN) launch(k_tile<FluxT, FluxT, RC_NN, DE, false>);
+    else if (recon == RC_PLM) launch(k_tile<FluxT, FluxT, RC_PLM, DE, false>);
+    else launch(k_tile<FluxT, FluxT, RC_PLM_ATHENA, DE, false>);
+  }
+}
+
 // Bytes of the chunk scratch pool: the larger of 4 GiB and a third of the
 // free device memory, at most 16 GiB (taken once per method).
 inline size_t scratch_budget(enzoe_vlct_method *m) {
@@ -805,6 +843,8 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
   // (stored fluxes come from the separate launches' flux arrays)
   const bool march =
       !st && march_ok(m, mx, my, mz, blocks[0].ghost, std::min(n, chunk));
+  const bool tile =
+      !MHD && !st && !march && tile_ok(m, mx, my, mz, std::min(n, chunk));
   for (int c0 = 0; c0 < n; c0 += chunk) {
     const int c1 = std::min(n, c0 + chunk);
     const int nb = c1 - c0;
@@ -858,6 +898,14 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
         }
         stale += total_staling(recon);
         continue;
+      }
+      if constexpr (!MHD) {
+        if (tile) {
+          KernelTimer kt(s, recon == RC_NN ? "k_tile_nn" : "k_tile_plm", timers);
+          dispatch_tile<FluxT, DE>(recon, primf, d, nb, mx, my, mz, lo, sp, s);
+          stale += total_staling(recon);
+          continue;
+        }
       }
       if constexpr (!DE) {
         if (structure == 5 && persistent_ok(m) && m->d_bar) {

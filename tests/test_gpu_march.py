@@ -95,6 +95,52 @@ def test_marched_stages_equal_the_separate_launches(n, count, riemann, recon, du
     _equal(out[0], out[1])
 
 
+@pytest.mark.parametrize("recon,dual,precision", [
+    ("plm", False, "double"), ("nn", False, "double"), ("plm_athena", False, "double"),
+    ("plm", True, "double"), ("nn", True, "double"), ("plm", False, "mixed"),
+    ("plm", False, "fma")])
+@pytest.mark.parametrize("n,count", [((1, 1, 1), 1), ((16, 16, 16), 1), ((9, 5, 3), 3),
+                                     ((23, 7, 10), 2), ((2, 18, 33), 1)])
+def test_tiled_stages_equal_the_separate_launches(n, count, recon, dual, precision):
+    """Small hydrodynamic blocks, one launch a stage: per-block dt, the fused
+    CFL, cells with NaN and huge values.  The same bits in FP64; the mixed
+    and contracted builds within a few of their own roundings."""
+    ev = _ev()
+    states = [_state(n, 70 + s, dual, mhd=False) for s in range(count)]
+    if precision == "double":
+        states[0]["velocity_x"][-4, 3, 3] = np.nan
+        states[-1]["velocity_z"][3, -5, 4] = 1.5e308
+    prec = {"double": ev.ENZOE_PREC_DOUBLE, "mixed": ev.ENZOE_PREC_MIXED,
+            "fma": ev.ENZOE_PREC_DOUBLE_FMA}[precision]
+    dts = [2e-4 * (1 + i) for i in range(count)]
+    if count > 2:
+        dts[1] = 0.0
+    out, nxt = [], []
+    for structure in (-1, 0):
+        m = ev.VlctMethod(mhd=False, riemann="hllc", reconstruct=recon, theta=2.0, courant=0.4,
+                          precision=prec, dual_energy_eta=0.001 if dual else None)
+        m.set_fused_ct(structure)
+        blocks = _blocks(ev, n, states, count, dual, mhd=False)
+        ev.profiling(True)
+        m.compute_dt(blocks, dts)
+        nxt.append(m.compute_timestep(blocks, 1e-4))
+        names = ev.profile_report()
+        ev.profiling(False)
+        assert ("k_tile_nn" in names) == (structure == -1)
+        out.append(blocks)
+    if precision == "double":
+        assert np.array_equal(*nxt, equal_nan=True)
+        _equal(out[0], out[1])
+        return
+    # two steps, each two sums of some 30 rounded terms of the size of
+    # the largest state value (about 10): 120 roundings
+    tol = 120 * 10 * {"mixed": 2.0 ** -24, "fma": 2.0 ** -53}[precision]
+    for x, y in zip(out[0], out[1]):
+        a, b = x.download(), y.download()
+        for k in a:
+            assert np.abs(a[k] - b[k]).max() <= tol, k
+
+
 @pytest.mark.parametrize("mhd", [True, False])
 def test_marched_stages_spread_nan_and_huge_values_as_the_separate_launches(mhd):
     """Cells with NaN, infinities and magnitudes whose differences overflow
