@@ -639,7 +639,7 @@ inline int device_cus() {
 // of the planes.  cost: the launch's time in units of one plane of 512
 // threads a CU with the device full; a piece of work costs 3 planes more
 // than it updates (the flux work of the planes around it, and its start).
-template <int NT, int PER>
+template <int NT, int PER, bool MHD>
 MarchParams march_tiling(int mx, int my, int mz, int cs, int nb, int cus, double &cost) {
   constexpr double UNIT = NT * PER / 512.0;
   const int nx = mx - 2 * (cs + 1), ny = my - 2 * (cs + 1), nz = mz - 2 * (cs + 1);
@@ -648,7 +648,7 @@ MarchParams march_tiling(int mx, int my, int mz, int cs, int nb, int cus, double
   for (int w2 = 10; w2 <= NT / 9; w2++) {
     if (w2 > nx + 2 && tiles >= 0) break;
     int h2 = std::min(NT / w2, ny + 2);
-    while ((w2 + 2) * (h2 + 2) > march_plane_cells(NT)) h2--;
+    while ((w2 + 2) * (h2 + 2) > march_plane_cells<MHD>(NT)) h2--;
     const int ntx = (nx + w2 - 3) / (w2 - 2), nty = (ny + h2 - 3) / (h2 - 2);
     if (tiles < 0 || (long)ntx * nty <= tiles) {
       tiles = (long)ntx * nty;
@@ -703,8 +703,8 @@ void launch_march(const BlockDesc<T> *d, int nb, int mx, int my, int mz, const S
   double big, small;
   constexpr int W = std::is_same<T, float>::value && RECON == RC_NN && !DE ? 3 : 2;
   constexpr int NT = 256 * W;
-  const MarchParams p5 = march_tiling<NT, 1>(mx, my, mz, sp.cur_stale, nb, cus, big);
-  const MarchParams p2 = march_tiling<256, W>(mx, my, mz, sp.cur_stale, nb, cus, small);
+  const MarchParams p5 = march_tiling<NT, 1, true>(mx, my, mz, sp.cur_stale, nb, cus, big);
+  const MarchParams p2 = march_tiling<256, W, true>(mx, my, mz, sp.cur_stale, nb, cus, small);
   if (big <= small)
     launch_march_nt<T, RECON, RIEMANN, DE, HALF, NT, W>(d, p5, sp, s);
   else
@@ -743,8 +743,8 @@ void launch_march_hd_of(const BlockDesc<T> *d, int nb, int mx, int my, int mz,
                         const StageParams &sp, hipStream_t s) {
   const int cus = device_cus();
   double big, small;
-  const MarchParams p = march_tiling<NT, PER>(mx, my, mz, sp.cur_stale, nb, cus, big);
-  const MarchParams q = march_tiling<NT2, PER2>(mx, my, mz, sp.cur_stale, nb, cus, small);
+  const MarchParams p = march_tiling<NT, PER, false>(mx, my, mz, sp.cur_stale, nb, cus, big);
+  const MarchParams q = march_tiling<NT2, PER2, false>(mx, my, mz, sp.cur_stale, nb, cus, small);
   if (big <= small)
     launch_march_hd_nt<T, RECON, DE, HALF, NT, PER>(d, p, sp, s);
   else

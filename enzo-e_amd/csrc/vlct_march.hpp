@@ -56,9 +56,12 @@ struct MarchParams {
 };
 
 // Cells of the LDS plane of a reconstructing march (the tile, its ring and
-// one more cell around; one less than 5/4 of the threads: with dual energy
-// the FP64 march fills the 160 KB).
-constexpr int march_plane_cells(int nt) { return nt + nt / 4 - 1; }
+// one more cell around; MHD: one less, with dual energy the FP64 march fills
+// the 160 KB).
+template <bool MHD>
+constexpr int march_plane_cells(int nt) {
+  return nt + nt / 4 - (MHD ? 1 : 0);
+}
 
 // dU - dtdx (F_hi - F_lo), never contracted (cell_stage's divergence).
 __device__ __forceinline__ double flux_difference(double dU, double dtdx, double hi, double lo) {
@@ -290,7 +293,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
   // (sE).  sB, the face B of plane k - 1: with LATE behind sE, else in the
   // first rows of sF, whose values (FZ*, FXB) are spent by then.  What takes
   // an area's place is written at least one barrier after its last read.
-  constexpr int WN = PLM ? march_plane_cells(NT) : NT;
+  constexpr int WN = PLM ? march_plane_cells<true>(NT) : NT;
   enum { FZD, FZBX, FZBY, FXB, FX0, FN = FX0 + 5 };
   enum { FY0, FYB = FY0 + 5, FYN };
   constexpr int EB = LATE ? 40 : 24, PB = PLM && 7 * sizeof(T) > EB ? 7 * sizeof(T) : EB;
@@ -752,7 +755,7 @@ k_march_hd(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams 
   fc.dbg = nullptr;
   const T theta = (T)sp.theta;
 
-  constexpr int WN = PLM ? march_plane_cells(NT) : NT;
+  constexpr int WN = PLM ? march_plane_cells<false>(NT) : NT;
   __shared__ T sW[NQ][WN];
   __shared__ T sF[2 * NQ][NT];  // right states, then fluxes: x rows, y rows
   __shared__ double sD[DE ? 4 : 1][DE ? NT : 1];
