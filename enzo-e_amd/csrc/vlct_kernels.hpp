@@ -2,8 +2,10 @@
 // and the ghost refresh, launched over a whole list of blocks at once.
 //
 // A stage (EnzoMHDIntegratorStageCommands::compute_update_stage,
-// src/Enzo/hydro-mhd/EnzoMHDIntegratorStageCommands.cpp:102-203) is four
-// launches, each covering every block of the batch (grid.y = block):
+// src/Enzo/hydro-mhd/EnzoMHDIntegratorStageCommands.cpp:102-203) of a large
+// launch is one marched kernel and of small hydrodynamic blocks one tiled one
+// (vlct_march.hpp); else, with debug counts and where fluxes are stored, it
+// is four launches, each covering every block of the batch (grid.y = block):
 //   k_flux  : primitives -> reconstruction -> Riemann flux on the three low
 //             faces of every cell (one HLLD/HLLE/HLLC solve per face)
 //   k_edge  : upwinded edge EMFs (Gardiner & Stone 2009) of constrained
