@@ -726,7 +726,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
 // completes the divergence and the update of the cell of plane k - 1; then
 // the x and y faces of plane k.  The right states travel through the rows of
 // LDS that take the fluxes afterwards.  Bound as k_march; 8 blocks of 128^3,
-// FP64: 0.81 + 1.17 ms for the two stages against 1.66 + 1.94 of the separate
+// FP64: 0.89 + 1.25 ms for the two stages against 1.66 + 1.94 of the separate
 // launches (a third of which wrote the 15 fluxes of a cell and read them
 // back); mixed 0.46 + 0.61 against 1.12 + 1.11.  WAVES: a SIMD's waves that its
 // registers are held to.
