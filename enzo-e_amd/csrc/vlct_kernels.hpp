@@ -117,8 +117,10 @@ __device__ __forceinline__ void debug_count(unsigned long long *dbg, int slot, b
 // place.  The internal energy is taken from etot - non-thermal energy where
 // the sound speed that implies beats eta times the kinetic and magnetic
 // scales (and it exceeds half the tracked value unless eta = 0).
-// floored (may be null): set when the floor had to be applied.
-template <bool MHD, bool DE>
+// floored (may be null): set when the floor had to be applied.  FUSED (the
+// mixed path): the floor's two sums round once, as that path's results always
+// have.
+template <bool MHD, bool DE, bool FUSED = false>
 __device__ __forceinline__ void floor_and_sync(double rho, const double v[3],
                                                double b2, double gamma,
                                                double pfloor, double eta,
@@ -126,10 +128,16 @@ __device__ __forceinline__ void floor_and_sync(double rho, const double v[3],
                                                double &eint,
                                                bool *floored = nullptr) {
   const double inv_rho = qrcp(rho);
-  const double eint_floor = pfloor * (1. / (gamma - 1.)) * inv_rho;
+  const double p_floor = pfloor * (1. / (gamma - 1.));
+  const double eint_floor = p_floor * inv_rho;
   const double v2 = (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
   double non_thermal_e = 0.5 * v2;
-  if (MHD) non_thermal_e += (0.5 * b2 * inv_rho);
+  if (MHD) {
+    if (FUSED)
+      non_thermal_e = __builtin_fma(0.5 * b2, inv_rho, non_thermal_e);
+    else
+      non_thermal_e += (0.5 * b2 * inv_rho);
+  }
   if (DE) {
     const double half_factor = (eta != 0.) ? 0.5 : 0.;
     const double eint_1 = etot - non_thermal_e;
@@ -143,7 +151,8 @@ __device__ __forceinline__ void floor_and_sync(double rho, const double v[3],
     eint = cur_eint;
     etot = cur_eint + non_thermal_e;
   } else {
-    const double etot_floor = eint_floor + non_thermal_e;
+    const double etot_floor = FUSED ? __builtin_fma(p_floor, inv_rho, non_thermal_e)
+                                    : eint_floor + non_thermal_e;
     if (floored) *floored = etot < etot_floor;
     etot = dmax(etot, etot_floor);
   }
@@ -324,9 +333,25 @@ __device__ __forceinline__ double center_efield(double vj, double vk, double bj,
 
 struct FluxConsts {
   double gm1, gamma, theta, dfloor, pfloor;
-  double igm1;  // 1 / (gamma - 1)
+  double igm1;  // 1 / (gamma - 1), in FP32 the hardware's reciprocal
   unsigned long long *dbg;  // debug counters or null
 };
+template <typename T>
+__device__ __forceinline__ FluxConsts flux_consts(const StageParams &sp, unsigned long long *dbg) {
+  FluxConsts fc;
+  fc.gm1 = sp.gamma - 1.0;
+  fc.gamma = sp.gamma;
+  if constexpr (std::is_same<T, float>::value)
+    fc.igm1 = (double)__uint_as_float(
+        __builtin_amdgcn_readfirstlane(__float_as_uint(qrcp((float)sp.gamma - 1.0f))));
+  else
+    fc.igm1 = sp.igm1;
+  fc.theta = sp.theta;
+  fc.dfloor = sp.density_floor;
+  fc.pfloor = sp.pressure_floor;
+  fc.dbg = dbg;
+  return fc;
+}
 
 // The flux through one face.
 template <typename T>
@@ -337,11 +362,12 @@ struct FaceFlux {
 };
 
 // The Riemann solve of a face along D from its two reconstructed states (by
-// slot; the normal B component of both is bface).
-template <typename T, int RIEMANN, bool MHD, int D, bool DE>
+// slot; the normal B component of both is bface; RECON, HALF as SumOrder).
+template <typename T, int RIEMANN, bool MHD, int D, bool DE, bool RECON, bool HALF>
 __device__ __forceinline__ void solve_face(const T wl[S_N], const T wr[S_N], T bface,
                                            const FluxConsts &fc, FaceFlux<T> &f) {
   constexpr int DJ = (D + 1) % 3, DK = (D + 2) % 3;
+  using O = SumOrder<D, RECON, HALF>;
   const T gamma = (T)fc.gamma;
   T fo[8];
   T vbar = T(0);
@@ -362,9 +388,9 @@ __device__ __forceinline__ void solve_face(const T wl[S_N], const T wr[S_N], T b
     l8[L_VK] = wl[S_VX + DK]; r8[L_VK] = wr[S_VX + DK];
     l8[L_E] = wl[S_E]; r8[L_E] = wr[S_E];
     if (RIEMANN == RS_HLLD) {
-      hlld(l8, r8, gamma, (T)fc.igm1, fo, vb);
+      hlld<O>(l8, r8, gamma, (T)fc.igm1, fo, vb);
     } else {
-      hlle_mhd(l8, r8, gamma, fo, vb);
+      hlle_mhd<O>(l8, r8, gamma, fo, vb);
     }
     f.u[S_RHO] = fo[L_D];
     f.u[S_VX + D] = fo[L_VI];
@@ -380,7 +406,7 @@ __device__ __forceinline__ void solve_face(const T wl[S_N], const T wr[S_N], T b
     l5[H_VJ] = wl[S_VX + DJ]; r5[H_VJ] = wr[S_VX + DJ];
     l5[H_VK] = wl[S_VX + DK]; r5[H_VK] = wr[S_VX + DK];
     l5[H_E] = wl[S_E]; r5[H_E] = wr[S_E];
-    hllc(l5, r5, gamma, fo, vb);
+    hllc<O>(l5, r5, gamma, fo, vb);
     f.u[S_RHO] = fo[H_D];
     f.u[S_VX + D] = fo[H_VI];
     f.u[S_VX + DJ] = fo[H_VJ];
@@ -453,7 +479,7 @@ __device__ __forceinline__ void face_flux(const BlockDesc<FluxT> &b, const Src &
     const int bnx = b.mx + (D == 0), bny = b.my + (D == 1);
     bface = (T)gld(bfi, (k + (D == 2)) * bny * bnx + (j + (D == 1)) * bnx + i + (D == 0));
   }
-  solve_face<T, RIEMANN, MHD, D, DE>(wl, wr, bface, fc, f);
+  solve_face<T, RIEMANN, MHD, D, DE, RECON != RC_NN, PRIMF>(wl, wr, bface, fc, f);
 }
 template <typename T, typename FluxT, int RECON, int RIEMANN, bool MHD, int D,
           bool DE, bool PRIMF, class Src = PrimSource<T, MHD, DE, PRIMF>>
@@ -511,14 +537,7 @@ __device__ __forceinline__ void flux_cells(const BlockDesc<FluxT> *__restrict__ 
     return;
   double *const *U = (sp.stage == 0) ? b.U : b.Ut;
   const double *const *bfr = (sp.stage == 0) ? b.bfi : b.bft;
-  FluxConsts fc;
-  fc.gm1 = sp.gamma - 1.0;
-  fc.gamma = sp.gamma;
-  fc.igm1 = sp.igm1;
-  fc.theta = sp.theta;
-  fc.dfloor = sp.density_floor;
-  fc.pfloor = sp.pressure_floor;
-  fc.dbg = sp.dbg;
+  const FluxConsts fc = flux_consts<T>(sp, sp.dbg);
   const int c = (k * my + j) * mx + i;
   const double *ei = DE ? ((sp.stage == 0) ? b.ei : b.eit) : nullptr;
   const PrimSource<T, MHD, DE, PRIMF> src{U, ei, b.Up, fc.gm1};
@@ -607,14 +626,7 @@ k_flux_zp(const BlockDesc<FluxT> *__restrict__ blocks, StageParams sp, int zplan
   const bool mine = i < mx - cs && j < my - cs;  // a cell of the flux box
   double *const *U = (sp.stage == 0) ? b.U : b.Ut;
   const double *const *bfr = (sp.stage == 0) ? b.bfi : b.bft;
-  FluxConsts fc;
-  fc.gm1 = sp.gamma - 1.0;
-  fc.gamma = sp.gamma;
-  fc.igm1 = sp.igm1;
-  fc.theta = sp.theta;
-  fc.dfloor = sp.density_floor;
-  fc.pfloor = sp.pressure_floor;
-  fc.dbg = sp.dbg;
+  const FluxConsts fc = flux_consts<T>(sp, sp.dbg);
   const double *ei = DE ? ((sp.stage == 0) ? b.ei : b.eit) : nullptr;
   const PrimSource<T, MHD, DE, PRIMF> src{U, ei, b.Up, fc.gm1};
   // the halo cell this thread loads per plane: the +y row past the tile
@@ -857,8 +869,8 @@ k_faces(const BlockDesc<FluxT> *__restrict__ blocks, StageParams sp) {
 // (EnzoComputePressure.cpp:177-189) and min_i dx_i / (|v_i| + c_f) with the
 // fast magnetosonic speed (EnzoEOSIdeal.hpp:111-140) or the sound speed.
 // Shared by k_dt and the final k_cells so both give the same bits; never
-// contracted into FMAs, also where the including unit allows it (the mixed
-// build), so that both round alike.
+// contracted into FMAs, also where the including unit allows it (the
+// contracted build), so that both round alike.
 template <bool MHD>
 __device__ __forceinline__ double cell_pressure(double d, double vx, double vy, double vz,
                                                 double e, double bx, double by, double bz,
@@ -1000,8 +1012,9 @@ __device__ __forceinline__ double cell_finish(const BlockDesc<FluxT> &b, const S
   // energy floor (and synchronisation)
   const double b2 = MHD ? (bc[0] * bc[0] + bc[1] * bc[1] + bc[2] * bc[2]) : 0.;
   bool floored = false;
-  floor_and_sync<MHD, DE>(new_rho, v, b2, sp.gamma, sp.pressure_floor, sp.eta, sp.ggm1, etot,
-                          eint, sp.dbg ? &floored : nullptr);
+  floor_and_sync<MHD, DE, std::is_same<FluxT, float>::value>(
+      new_rho, v, b2, sp.gamma, sp.pressure_floor, sp.eta, sp.ggm1, etot, eint,
+      sp.dbg ? &floored : nullptr);
   if (sp.dbg) {
     debug_count(sp.dbg, DBG_ENERGY_FLOOR, floored);
     bool finite = isfinite(new_rho) && isfinite(v[0]) && isfinite(v[1]) && isfinite(v[2]) &&

@@ -1,7 +1,8 @@
 // vlct_launch.hpp -- host-side launch sequence of the VL+CT step, shared by
 // the FP64 translation unit (vlct_capi.hip, built without FMA contraction
-// for bitwise reference parity) and the mixed-precision one
-// (vlct_mixed.hip, FP32 reconstruction and Riemann fluxes).
+// for bitwise reference parity), the mixed-precision one (vlct_mixed.hip, FP32
+// reconstruction and Riemann fluxes) and the contracted FP64 one
+// (vlct_fp64c.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>

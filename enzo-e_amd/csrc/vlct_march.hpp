@@ -278,14 +278,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
   const unsigned g = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const long last = ((long)g + 1) * mp.share < mp.total ? ((long)g + 1) * mp.share : mp.total;
 
-  FluxConsts fc;
-  fc.gm1 = sp.gamma - 1.0;
-  fc.gamma = sp.gamma;
-  fc.igm1 = sp.igm1;
-  fc.theta = sp.theta;
-  fc.dfloor = sp.density_floor;
-  fc.pfloor = sp.pressure_floor;
-  fc.dbg = nullptr;
+  const FluxConsts fc = flux_consts<T>(sp, nullptr);
   const T theta = (T)sp.theta;
   // LDS.  sW: the plane's primitives; sEc: the centre E of plane k; sF: the z
   // and x face quantities by slot; sX: the x right states on their way to the
@@ -461,7 +454,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
         }
         if (k > k0) {
           FaceFlux<T> f;
-          solve_face<T, RIEMANN, true, 2, DE>(Lz, R, (T)fbz, fc, f);
+          solve_face<T, RIEMANN, true, 2, DE, PLM, HALF>(Lz, R, (T)fbz, fc, f);
           if (k > ks) {
             // the divergence of cell k - 1 (its x and y parts are in dU)
 #pragma unroll
@@ -526,7 +519,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
         T L[S_N], R[S_N];
         exchange(std::integral_constant<int, S_BX>(), sX, wi - 1, wxp, xp, L, R);
         FaceFlux<T> f;
-        solve_face<T, RIEMANN, true, 0, DE>(L, R, (T)fbx, fc, f);
+        solve_face<T, RIEMANN, true, 0, DE, PLM, HALF>(L, R, (T)fbx, fc, f);
 #pragma unroll
         for (int q = 0; q < 5; q++) sF[FX0 + q][tid] = f.u[q];
         sF[FXB][tid] = f.bj;
@@ -541,7 +534,7 @@ k_march(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams mp)
         T L[S_N], R[S_N];
         exchange(std::integral_constant<int, S_BY>(), sY, wi - ws, wyp, yp, L, R);
         FaceFlux<T> f;
-        solve_face<T, RIEMANN, true, 1, DE>(L, R, (T)fby, fc, f);
+        solve_face<T, RIEMANN, true, 1, DE, PLM, HALF>(L, R, (T)fby, fc, f);
 #pragma unroll
         for (int q = 0; q < 5; q++) sX[FY0 + q][tid] = f.u[q];
         FyBz_k = f.bj;
@@ -745,14 +738,7 @@ k_march_hd(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams 
   const unsigned g = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const long last = ((long)g + 1) * mp.share < mp.total ? ((long)g + 1) * mp.share : mp.total;
 
-  FluxConsts fc;
-  fc.gm1 = sp.gamma - 1.0;
-  fc.gamma = sp.gamma;
-  fc.igm1 = sp.igm1;
-  fc.theta = sp.theta;
-  fc.dfloor = sp.density_floor;
-  fc.pfloor = sp.pressure_floor;
-  fc.dbg = nullptr;
+  const FluxConsts fc = flux_consts<T>(sp, nullptr);
   const T theta = (T)sp.theta;
 
   constexpr int WN = PLM ? march_plane_cells<false>(NT) : NT;
@@ -883,7 +869,7 @@ k_march_hd(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams 
           for (int q = 0; q < NQ; q++) R[q] = Ln[q] = a[q];
         }
         FaceFlux<T> f;
-        solve_face<T, RS_HLLC, false, 2, DE>(Lz, R, T(0), fc, f);
+        solve_face<T, RS_HLLC, false, 2, DE, PLM, HALF>(Lz, R, T(0), fc, f);
         if (k > ks) {
 #pragma unroll
           for (int q = 0; q < NQ; q++)
@@ -947,8 +933,8 @@ k_march_hd(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams 
             Ry[q] = sW[q][yp];
           }
         }
-        solve_face<T, RS_HLLC, false, 0, DE>(Lx, Rx, T(0), fc, fx);
-        solve_face<T, RS_HLLC, false, 1, DE>(Ly, Ry, T(0), fc, fy);
+        solve_face<T, RS_HLLC, false, 0, DE, PLM, HALF>(Lx, Rx, T(0), fc, fx);
+        solve_face<T, RS_HLLC, false, 1, DE, PLM, HALF>(Ly, Ry, T(0), fc, fy);
       }
 #pragma unroll
       for (int q = 0; q < NQ; q++) {
@@ -1114,14 +1100,7 @@ k_tile(const BlockDesc<FluxT> *__restrict__ blocks, StageParams sp) {
 
   {
     double *const *U = (sp.stage == 0) ? b.U : b.Ut;
-    FluxConsts fc;
-    fc.gm1 = sp.gamma - 1.0;
-    fc.gamma = sp.gamma;
-    fc.igm1 = sp.igm1;
-    fc.theta = sp.theta;
-    fc.dfloor = sp.density_floor;
-    fc.pfloor = sp.pressure_floor;
-    fc.dbg = nullptr;
+    const FluxConsts fc = flux_consts<T>(sp, nullptr);
     const double *ei = DE ? ((sp.stage == 0) ? b.ei : b.eit) : nullptr;
     const PrimSource<T, false, DE, PRIMF> src{U, ei, b.Up, fc.gm1};
     // thread r of axis D: the low face of the cell (i, j, k); solved where

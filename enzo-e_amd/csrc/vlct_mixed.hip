@@ -1,8 +1,10 @@
 // vlct_mixed.hip -- the mixed-precision VL+CT step: FP32 reconstruction and
 // Riemann fluxes (fast FP32 reciprocal and square root), FP64 primitives,
 // flux divergence, CT EMF / face-B update and dt.  Built with
-// -ffp-contract=fast: this path is checked against the FP64 result by its
-// L1 error, not bit by bit.
+// -ffp-contract=off: the solves' fused multiply-adds are written out, so that
+// the result does not depend on which kernels run the step.  It is checked
+// against the FP64 result by its L1 error and, every launch structure against
+// the separate launches, bit by bit.
 #include <hip/hip_runtime.h>
 
 #include "vlct_launch.hpp"

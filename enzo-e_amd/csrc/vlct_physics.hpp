@@ -4,7 +4,8 @@
 // float for the FP32 reconstruction/Riemann stage of the mixed path).  The
 // expression trees keep the reference's parenthesisation and left-to-right
 // association; the library is built with -ffp-contract=off so the FP64 path
-// rounds exactly like the reference's CPU build.
+// rounds exactly like the reference's CPU build.  The FP32 solves' fused
+// multiply-adds are written out (mad and the others below).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -115,6 +116,106 @@ __device__ __forceinline__ double qdiv_inv(double a, double b, double inv) {
 }
 __device__ __forceinline__ float qdiv_inv(float a, float, float inv) { return a * inv; }
 
+// Multiply-adds of the Riemann solves.  FP32 (the mixed path): one rounding,
+// written out here and never left to the compiler.  The FP32 HLLD solve
+// divides by differences that can cancel down to their rounding (and HLLE
+// takes the root of one), so a multiply-add that is fused in one kernel and
+// not in another can change a cell by as much as it holds; like this every
+// kernel that runs a solve rounds alike.  FP64: the product and the sum
+// rounded in turn, as the reference does (the contracted build's compiler
+// fuses them).
+__device__ __forceinline__ double mad(double a, double b, double c) { return a * b + c; }
+__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// a b - c
+__device__ __forceinline__ double msub(double a, double b, double c) { return a * b - c; }
+__device__ __forceinline__ float msub(float a, float b, float c) {
+  return __builtin_fmaf(a, b, -c);
+}
+// c + a b, c - a b
+__device__ __forceinline__ double add_mul(double c, double a, double b) { return c + a * b; }
+__device__ __forceinline__ float add_mul(float c, float a, float b) {
+  return __builtin_fmaf(a, b, c);
+}
+__device__ __forceinline__ double sub_mul(double c, double a, double b) { return c - a * b; }
+__device__ __forceinline__ float sub_mul(float c, float a, float b) {
+  return __builtin_fmaf(-a, b, c);
+}
+// c + a / b, c - a / b, where inv = 1 / b is at hand
+__device__ __forceinline__ double add_div(double c, double a, double b, double inv) {
+  return c + qdiv_inv(a, b, inv);
+}
+__device__ __forceinline__ float add_div(float c, float a, float, float inv) {
+  return __builtin_fmaf(a, inv, c);
+}
+__device__ __forceinline__ double sub_div(double c, double a, double b, double inv) {
+  return c - qdiv_inv(a, b, inv);
+}
+__device__ __forceinline__ float sub_div(float c, float a, float, float inv) {
+  return __builtin_fmaf(-a, inv, c);
+}
+// ... and where it is not (c - a / b, c + a / b)
+__device__ __forceinline__ double add_div(double c, double a, double b) { return c + qdiv(a, b); }
+__device__ __forceinline__ float add_div(float c, float a, float b) {
+  return __builtin_fmaf(a, __builtin_amdgcn_rcpf(b), c);
+}
+__device__ __forceinline__ double sub_div(double c, double a, double b) { return c - qdiv(a, b); }
+__device__ __forceinline__ float sub_div(float c, float a, float b) {
+  return __builtin_fmaf(-a, __builtin_amdgcn_rcpf(b), c);
+}
+
+// a1 b1 + a2 b2.  FP32: the first product is fused onto the second, with SWAP
+// the second onto the first.
+template <bool SWAP>
+__device__ __forceinline__ double dot2(double a1, double b1, double a2, double b2) {
+  return a1 * b1 + a2 * b2;
+}
+template <bool SWAP>
+__device__ __forceinline__ float dot2(float a1, float b1, float a2, float b2) {
+  return SWAP ? __builtin_fmaf(a2, b2, a1 * b1) : __builtin_fmaf(a1, b1, a2 * b2);
+}
+// Where the FP32 solves fuse the second product of such a sum.  Either order
+// is as good; these are the ones that the path's results have always been
+// formed with, which the ill-conditioned faces hold it to.  D: the face's
+// axis; RECON: reconstructed states (not the nearest-neighbour ones); HALF:
+// states from the half-step primitives (the pressure at hand).  The rules
+// follow the fields: of two transverse components the earlier of x, y, z is
+// fused, of a left and a right value the one whose operands come first.
+template <int D, bool RECON, bool HALF>
+struct SumOrder {
+  static constexpr bool kj = D == 1;              // transverse components j, k
+  static constexpr bool kj_roe = kj && !RECON;    // ... of the Roe average
+  static constexpr bool ji_roe = D == 2 && !RECON;  // normal and first transverse velocity
+  static constexpr bool rl = RECON && HALF;       // sqrt(rho) weighted left and right values
+  static constexpr bool energy = !HALF;           // internal and kinetic energy
+};
+// Internal plus kinetic energy density p / (gamma - 1) + (rho / 2) v^2, where
+// inv = 1 / (gamma - 1).
+template <bool SWAP>
+__device__ __forceinline__ double energy_density(double p, double gm1, double inv, double half_rho,
+                                                 double v2) {
+  return qdiv_inv(p, gm1, inv) + half_rho * v2;
+}
+template <bool SWAP>
+__device__ __forceinline__ float energy_density(float p, float, float inv, float half_rho,
+                                                float v2) {
+  return dot2<SWAP>(p, inv, half_rho, v2);
+}
+// a quotient a / b that sums are formed with
+template <typename T> struct Quotient;
+template <> struct Quotient<double> {
+  double q;
+  __device__ __forceinline__ Quotient(double a, double b) : q(qdiv(a, b)) {}
+  __device__ __forceinline__ double minus(double c) const { return q - c; }  // a / b - c
+  __device__ __forceinline__ double from(double c) const { return c - q; }   // c - a / b
+};
+template <> struct Quotient<float> {
+  float a, inv, q;
+  __device__ __forceinline__ Quotient(float num, float b)
+      : a(num), inv(__builtin_amdgcn_rcpf(b)), q(num * inv) {}
+  __device__ __forceinline__ float minus(float c) const { return __builtin_fmaf(a, inv, -c); }
+  __device__ __forceinline__ float from(float c) const { return __builtin_fmaf(-a, inv, c); }
+};
+
 template <typename T> __device__ __forceinline__ T dmin(T a, T b) {
   return (b < a) ? b : a;  // std::min
 }
@@ -176,22 +277,20 @@ __device__ __forceinline__ T limiter_athena(T vm1, T v, T vp1) {
 // EnzoEOSIdeal::fast_magnetosonic_speed<-1> (EnzoEOSIdeal.hpp:111-140) of
 // the two states of a face, side by side; std::pow(x, 2) == x*x exactly.
 // w in the MHD LUT order.
-template <typename T>
+template <class O, typename T>
 __device__ __forceinline__ void fast_ms_speeds(const T wl[8], const T wr[8], T gamma, T &cl,
                                                T &cr) {
   const T *w[2] = {wl, wr};
-  T sum[2], rad[2], s1[2], rt[2];
+  T sum[2], rad[2], rt[2];
 #pragma unroll
   for (int s = 0; s < 2; s++) {
     const T d = w[s][L_D], bi = w[s][L_BI], bj = w[s][L_BJ], bk = w[s][L_BK];
-    const T B2 = ((bi * bi) + ((bj * bj) + (bk * bk)));
+    const T B2 = mad(bi, bi, dot2<O::kj>(bj, bj, bk, bk));
     const T inv_density = qrcp(d);
     const T cs2 = qdiv_inv(gamma * w[s][L_E], d, inv_density);
-    const T va2 = B2 * inv_density;
     const T va2_cos2 = (bi * bi) * inv_density;
-    sum[s] = va2 + cs2;
-    s1[s] = cs2 + va2;
-    rad[s] = s1[s] * s1[s] - T(4) * cs2 * va2_cos2;
+    sum[s] = mad(B2, inv_density, cs2);  // va2 + cs2
+    rad[s] = msub(sum[s], sum[s], T(4) * cs2 * va2_cos2);
   }
   qsqrt2(rad[0], rad[1], rt[0], rt[1]);
   qsqrt2(T(0.5) * (sum[0] + rt[0]), T(0.5) * (sum[1] + rt[1]), cl, cr);
@@ -222,7 +321,7 @@ __device__ __forceinline__ T upwind_eint_flux(T eint_l, T eint_r, T density_flux
 // interface velocity of :418-447 -- the left/right normal velocity outside
 // the fan, else the contact speed scaled by the outer state's coefficient.
 // igm1: 1 / (gamma - 1), the same for every face of a launch.
-template <typename T>
+template <class O = SumOrder<0, false, false>, typename T>
 __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma, T igm1,
                                      T flx[8], T *vbar = nullptr) {
   const T SMALL_NUMBER = T(1.0e-8);
@@ -237,20 +336,18 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma, T 
   const T bxi = wli[L_BI];
 
   T bxsq = bxi * bxi;
-  T pbl = T(0.5) * (bxsq + (wli[L_BJ] * wli[L_BJ] + wli[L_BK] * wli[L_BK]));
-  T pbr = T(0.5) * (bxsq + (wri[L_BJ] * wri[L_BJ] + wri[L_BK] * wri[L_BK]));
-  T kel = T(0.5) * wli[L_D] *
-          (wli[L_VI] * wli[L_VI] +
-           (wli[L_VJ] * wli[L_VJ] + wli[L_VK] * wli[L_VK]));
-  T ker = T(0.5) * wri[L_D] *
-          (wri[L_VI] * wri[L_VI] +
-           (wri[L_VJ] * wri[L_VJ] + wri[L_VK] * wri[L_VK]));
+  const T bsql = mad(bxi, bxi, dot2<O::kj>(wli[L_BJ], wli[L_BJ], wli[L_BK], wli[L_BK]));
+  const T bsqr = mad(bxi, bxi, dot2<O::kj>(wri[L_BJ], wri[L_BJ], wri[L_BK], wri[L_BK]));
+  T pbl = T(0.5) * bsql;
+  T pbr = T(0.5) * bsqr;
+  const T v2l = mad(wli[L_VI], wli[L_VI], dot2<O::kj>(wli[L_VJ], wli[L_VJ], wli[L_VK], wli[L_VK]));
+  const T v2r = mad(wri[L_VI], wri[L_VI], dot2<O::kj>(wri[L_VJ], wri[L_VJ], wri[L_VK], wri[L_VK]));
 
   ul.d = wli[L_D];
   ul.mx = wli[L_VI] * ul.d;
   ul.my = wli[L_VJ] * ul.d;
   ul.mz = wli[L_VK] * ul.d;
-  ul.e = pressure_l * igm1 + kel + pbl;
+  ul.e = dot2<O::energy>(pressure_l, igm1, T(0.5) * wli[L_D], v2l) + pbl;
   ul.by = wli[L_BJ];
   ul.bz = wli[L_BK];
 
@@ -258,25 +355,26 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma, T 
   ur.mx = wri[L_VI] * ur.d;
   ur.my = wri[L_VJ] * ur.d;
   ur.mz = wri[L_VK] * ur.d;
-  ur.e = pressure_r * igm1 + ker + pbr;
+  ur.e = dot2<O::energy>(pressure_r, igm1, T(0.5) * wri[L_D], v2r) + pbr;
   ur.by = wri[L_BJ];
   ur.bz = wri[L_BK];
 
   T cfl, cfr;
-  fast_ms_speeds(wli, wri, gamma, cfl, cfr);
+  fast_ms_speeds<O>(wli, wri, gamma, cfl, cfr);
 
   spd[0] = dmin(wli[L_VI] - cfl, wri[L_VI] - cfr);
   spd[4] = dmax(wli[L_VI] + cfl, wri[L_VI] + cfr);
 
-  T ptl = pressure_l + pbl;
-  T ptr = pressure_r + pbr;
+  T ptl = add_mul(pressure_l, T(0.5), bsql);
+  T ptr = add_mul(pressure_r, T(0.5), bsqr);
 
   T sdl = spd[0] - wli[L_VI];
   T sdr = spd[4] - wri[L_VI];
-  spd[2] = qdiv(sdr * ur.mx - sdl * ul.mx + (ptl - ptr),
-                sdr * ur.d - sdl * ul.d);
+  const Quotient<T> sm(msub(sdr, ur.mx, sdl * ul.mx) + (ptl - ptr),
+                       msub(sdr, ur.d, sdl * ul.d));
+  spd[2] = sm.q;
 
-  T sdml = spd[0] - spd[2];
+  T sdml = sm.from(spd[0]);
   T sdmr = spd[4] - spd[2];
   T sdml_inv = qrcp(sdml);
   T sdmr_inv = qrcp(sdmr);
@@ -303,11 +401,11 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma, T 
   T sqrtdl, sqrtdr;
   qsqrt2(ulst.d, urst.d, sqrtdl, sqrtdr);
 
-  spd[1] = spd[2] - qdiv(fabs(bxi), sqrtdl);
-  spd[3] = spd[2] + qdiv(fabs(bxi), sqrtdr);
+  spd[1] = sub_div(spd[2], fabs(bxi), sqrtdl);
+  spd[3] = add_div(spd[2], fabs(bxi), sqrtdr);
 
-  T ptstl = ptl + ul.d * sdl * (spd[2] - wli[L_VI]);
-  T ptstr = ptr + ur.d * sdr * (spd[2] - wri[L_VI]);
+  T ptstl = add_mul(ptl, ul.d * sdl, sm.minus(wli[L_VI]));
+  T ptstr = add_mul(ptr, ur.d * sdr, sm.minus(wri[L_VI]));
   T ptst = T(0.5) * (ptstr + ptstl);
 
   // the transverse star states of both sides, side by side, then the rare
@@ -315,16 +413,16 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma, T 
   ulst.mx = ulst.d * spd[2];
   urst.mx = urst.d * spd[2];
   {
-    const T denl = ul.d * sdl * sdml - bxsq, denr = ur.d * sdr * sdmr - bxsq;
+    const T denl = msub(ul.d * sdl, sdml, bxsq), denr = msub(ur.d * sdr, sdmr, bxsq);
     const T denl_inv = qrcp(denl), denr_inv = qrcp(denr);
     T tmpl = qdiv_inv(bxi * (sdl - sdml), denl, denl_inv);
     T tmpr = qdiv_inv(bxi * (sdr - sdmr), denr, denr_inv);
-    ulst.my = ulst.d * (wli[L_VJ] - ul.by * tmpl);
-    ulst.mz = ulst.d * (wli[L_VK] - ul.bz * tmpl);
-    urst.my = urst.d * (wri[L_VJ] - ur.by * tmpr);
-    urst.mz = urst.d * (wri[L_VK] - ur.bz * tmpr);
-    tmpl = qdiv_inv(ul.d * (sdl * sdl) - bxsq, denl, denl_inv);
-    tmpr = qdiv_inv(ur.d * (sdr * sdr) - bxsq, denr, denr_inv);
+    ulst.my = ulst.d * sub_mul(wli[L_VJ], ul.by, tmpl);
+    ulst.mz = ulst.d * sub_mul(wli[L_VK], ul.bz, tmpl);
+    urst.my = urst.d * sub_mul(wri[L_VJ], ur.by, tmpr);
+    urst.mz = urst.d * sub_mul(wri[L_VK], ur.bz, tmpr);
+    tmpl = qdiv_inv(msub(ul.d, sdl * sdl, bxsq), denl, denl_inv);
+    tmpr = qdiv_inv(msub(ur.d, sdr * sdr, bxsq), denr, denr_inv);
     ulst.by = ul.by * tmpl;
     ulst.bz = ul.bz * tmpl;
     urst.by = ur.by * tmpr;
@@ -346,17 +444,17 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma, T 
       }
     }
   }
-  T vbstl =
-      (ulst.mx * bxi + (ulst.my * ulst.by + ulst.mz * ulst.bz)) * ulst_d_inv;
-  ulst.e = (sdl * ul.e - ptl * wli[L_VI] + ptst * spd[2] +
-            bxi * (wli[L_VI] * bxi + (wli[L_VJ] * ul.by + wli[L_VK] * ul.bz) -
-                   vbstl)) *
+  const T mbstl = mad(ulst.mx, bxi, mad(ulst.my, ulst.by, ulst.mz * ulst.bz));
+  T vbstl = mbstl * ulst_d_inv;
+  const T vbl = dot2<O::kj>(wli[L_VJ], ul.by, wli[L_VK], ul.bz);
+  ulst.e = add_mul(add_mul(msub(sdl, ul.e, ptl * wli[L_VI]), ptst, spd[2]), bxi,
+                   sub_mul(mad(wli[L_VI], bxi, vbl), mbstl, ulst_d_inv)) *
            sdml_inv;
-  T vbstr =
-      (urst.mx * bxi + (urst.my * urst.by + urst.mz * urst.bz)) * urst_d_inv;
-  urst.e = (sdr * ur.e - ptr * wri[L_VI] + ptst * spd[2] +
-            bxi * (wri[L_VI] * bxi + (wri[L_VJ] * ur.by + wri[L_VK] * ur.bz) -
-                   vbstr)) *
+  const T mbstr = mad(urst.mx, bxi, mad(urst.my, urst.by, urst.mz * urst.bz));
+  T vbstr = mbstr * urst_d_inv;
+  const T vbr = dot2<O::kj>(wri[L_VJ], ur.by, wri[L_VK], ur.bz);
+  urst.e = add_mul(add_mul(msub(sdr, ur.e, ptr * wri[L_VI]), ptst, spd[2]), bxi,
+                   sub_mul(mad(wri[L_VI], bxi, vbr), mbstr, urst_d_inv)) *
            sdmr_inv;
 
   if (T(0.5) * bxsq < (SMALL_NUMBER)*ptst) {
@@ -370,52 +468,49 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma, T 
     uldst.mx = ulst.mx;
     urdst.mx = urst.mx;
 
-    T tmp = invsumd * (sqrtdl * (ulst.my * ulst_d_inv) +
-                       sqrtdr * (urst.my * urst_d_inv) +
-                       bxsig * (urst.by - ulst.by));
+    T tmp = invsumd * add_mul(mad(sqrtdl, ulst.my * ulst_d_inv, sqrtdr * (urst.my * urst_d_inv)),
+                              bxsig, urst.by - ulst.by);
     uldst.my = uldst.d * tmp;
     urdst.my = urdst.d * tmp;
 
-    tmp = invsumd * (sqrtdl * (ulst.mz * ulst_d_inv) +
-                     sqrtdr * (urst.mz * urst_d_inv) +
-                     bxsig * (urst.bz - ulst.bz));
+    tmp = invsumd * add_mul(mad(sqrtdl, ulst.mz * ulst_d_inv, sqrtdr * (urst.mz * urst_d_inv)),
+                            bxsig, urst.bz - ulst.bz);
     uldst.mz = uldst.d * tmp;
     urdst.mz = urdst.d * tmp;
 
-    tmp = invsumd * (sqrtdl * urst.by + sqrtdr * ulst.by +
-                     bxsig * sqrtdl * sqrtdr *
-                         ((urst.my * urst_d_inv) - (ulst.my * ulst_d_inv)));
+    tmp = invsumd * add_mul(add_mul(sqrtdl * urst.by, sqrtdr, ulst.by),
+                            bxsig * sqrtdl * sqrtdr,
+                            msub(urst.my, urst_d_inv, ulst.my * ulst_d_inv));
     uldst.by = urdst.by = tmp;
 
-    tmp = invsumd * (sqrtdl * urst.bz + sqrtdr * ulst.bz +
-                     bxsig * sqrtdl * sqrtdr *
-                         ((urst.mz * urst_d_inv) - (ulst.mz * ulst_d_inv)));
+    tmp = invsumd * add_mul(add_mul(sqrtdl * urst.bz, sqrtdr, ulst.bz),
+                            bxsig * sqrtdl * sqrtdr,
+                            msub(urst.mz, urst_d_inv, ulst.mz * ulst_d_inv));
     uldst.bz = urdst.bz = tmp;
 
-    tmp = spd[2] * bxi + qdiv_inv(uldst.my * uldst.by + uldst.mz * uldst.bz, uldst.d, ulst_d_inv);
-    uldst.e = ulst.e - sqrtdl * bxsig * (vbstl - tmp);
-    urdst.e = urst.e + sqrtdr * bxsig * (vbstr - tmp);
+    tmp = mad(spd[2], bxi,
+              qdiv_inv(mad(uldst.my, uldst.by, uldst.mz * uldst.bz), uldst.d, ulst_d_inv));
+    uldst.e = sub_mul(ulst.e, sqrtdl * bxsig, vbstl - tmp);
+    urdst.e = add_mul(urst.e, sqrtdr * bxsig, vbstr - tmp);
   }
 
   auto flux_l = [&]() {
     fl.d = ul.mx;
-    fl.mx = ul.mx * wli[L_VI] + ptl - bxsq;
-    fl.my = ul.my * wli[L_VI] - bxi * ul.by;
-    fl.mz = ul.mz * wli[L_VI] - bxi * ul.bz;
-    fl.e = wli[L_VI] * (ul.e + ptl - bxsq) -
-           bxi * (wli[L_VJ] * ul.by + wli[L_VK] * ul.bz);
-    fl.by = ul.by * wli[L_VI] - bxi * wli[L_VJ];
-    fl.bz = ul.bz * wli[L_VI] - bxi * wli[L_VK];
+    fl.mx = mad(ul.mx, wli[L_VI], ptl) - bxsq;
+    fl.my = msub(ul.my, wli[L_VI], bxi * ul.by);
+    fl.mz = msub(ul.mz, wli[L_VI], bxi * ul.bz);
+    fl.e = msub(wli[L_VI], ul.e + ptl - bxsq, bxi * vbl);
+    fl.by = msub(ul.by, wli[L_VI], bxi * wli[L_VJ]);
+    fl.bz = msub(ul.bz, wli[L_VI], bxi * wli[L_VK]);
   };
   auto flux_r = [&]() {
     fr.d = ur.mx;
-    fr.mx = ur.mx * wri[L_VI] + ptr - bxsq;
-    fr.my = ur.my * wri[L_VI] - bxi * ur.by;
-    fr.mz = ur.mz * wri[L_VI] - bxi * ur.bz;
-    fr.e = wri[L_VI] * (ur.e + ptr - bxsq) -
-           bxi * (wri[L_VJ] * ur.by + wri[L_VK] * ur.bz);
-    fr.by = ur.by * wri[L_VI] - bxi * wri[L_VJ];
-    fr.bz = ur.bz * wri[L_VI] - bxi * wri[L_VK];
+    fr.mx = mad(ur.mx, wri[L_VI], ptr) - bxsq;
+    fr.my = msub(ur.my, wri[L_VI], bxi * ur.by);
+    fr.mz = msub(ur.mz, wri[L_VI], bxi * ur.bz);
+    fr.e = msub(wri[L_VI], ur.e + ptr - bxsq, bxi * vbr);
+    fr.by = msub(ur.by, wri[L_VI], bxi * wri[L_VJ]);
+    fr.bz = msub(ur.bz, wri[L_VI], bxi * wri[L_VK]);
   };
   // Select the region of the fan containing the interface; the state
   // differences of each wave are formed lazily (only the ones used).
@@ -429,137 +524,139 @@ __device__ __forceinline__ void hlld(const T wli[8], const T wri[8], T gamma, T 
     flx[L_E] = fr.e; flx[L_BJ] = fr.by; flx[L_BK] = fr.bz;
   } else if (spd[1] >= T(0)) {
     flux_l();
-    flx[L_D] = fl.d + spd[0] * (ulst.d - ul.d);
-    flx[L_VI] = fl.mx + spd[0] * (ulst.mx - ul.mx);
-    flx[L_VJ] = fl.my + spd[0] * (ulst.my - ul.my);
-    flx[L_VK] = fl.mz + spd[0] * (ulst.mz - ul.mz);
-    flx[L_E] = fl.e + spd[0] * (ulst.e - ul.e);
-    flx[L_BJ] = fl.by + spd[0] * (ulst.by - ul.by);
-    flx[L_BK] = fl.bz + spd[0] * (ulst.bz - ul.bz);
+    flx[L_D] = add_mul(fl.d, spd[0], ulst.d - ul.d);
+    flx[L_VI] = add_mul(fl.mx, spd[0], ulst.mx - ul.mx);
+    flx[L_VJ] = add_mul(fl.my, spd[0], ulst.my - ul.my);
+    flx[L_VK] = add_mul(fl.mz, spd[0], ulst.mz - ul.mz);
+    flx[L_E] = add_mul(fl.e, spd[0], ulst.e - ul.e);
+    flx[L_BJ] = add_mul(fl.by, spd[0], ulst.by - ul.by);
+    flx[L_BK] = add_mul(fl.bz, spd[0], ulst.bz - ul.bz);
   } else if (spd[2] >= T(0)) {
     flux_l();
-    flx[L_D] = fl.d + spd[0] * (ulst.d - ul.d) + spd[1] * (uldst.d - ulst.d);
-    flx[L_VI] = fl.mx + spd[0] * (ulst.mx - ul.mx) + spd[1] * (uldst.mx - ulst.mx);
-    flx[L_VJ] = fl.my + spd[0] * (ulst.my - ul.my) + spd[1] * (uldst.my - ulst.my);
-    flx[L_VK] = fl.mz + spd[0] * (ulst.mz - ul.mz) + spd[1] * (uldst.mz - ulst.mz);
-    flx[L_E] = fl.e + spd[0] * (ulst.e - ul.e) + spd[1] * (uldst.e - ulst.e);
-    flx[L_BJ] = fl.by + spd[0] * (ulst.by - ul.by) + spd[1] * (uldst.by - ulst.by);
-    flx[L_BK] = fl.bz + spd[0] * (ulst.bz - ul.bz) + spd[1] * (uldst.bz - ulst.bz);
+    flx[L_D] = add_mul(add_mul(fl.d, spd[0], ulst.d - ul.d), spd[1], uldst.d - ulst.d);
+    flx[L_VI] = add_mul(add_mul(fl.mx, spd[0], ulst.mx - ul.mx), spd[1], uldst.mx - ulst.mx);
+    flx[L_VJ] = add_mul(add_mul(fl.my, spd[0], ulst.my - ul.my), spd[1], uldst.my - ulst.my);
+    flx[L_VK] = add_mul(add_mul(fl.mz, spd[0], ulst.mz - ul.mz), spd[1], uldst.mz - ulst.mz);
+    flx[L_E] = add_mul(add_mul(fl.e, spd[0], ulst.e - ul.e), spd[1], uldst.e - ulst.e);
+    flx[L_BJ] = add_mul(add_mul(fl.by, spd[0], ulst.by - ul.by), spd[1], uldst.by - ulst.by);
+    flx[L_BK] = add_mul(add_mul(fl.bz, spd[0], ulst.bz - ul.bz), spd[1], uldst.bz - ulst.bz);
   } else if (spd[3] > T(0)) {
     flux_r();
-    flx[L_D] = fr.d + spd[4] * (urst.d - ur.d) + spd[3] * (urdst.d - urst.d);
-    flx[L_VI] = fr.mx + spd[4] * (urst.mx - ur.mx) + spd[3] * (urdst.mx - urst.mx);
-    flx[L_VJ] = fr.my + spd[4] * (urst.my - ur.my) + spd[3] * (urdst.my - urst.my);
-    flx[L_VK] = fr.mz + spd[4] * (urst.mz - ur.mz) + spd[3] * (urdst.mz - urst.mz);
-    flx[L_E] = fr.e + spd[4] * (urst.e - ur.e) + spd[3] * (urdst.e - urst.e);
-    flx[L_BJ] = fr.by + spd[4] * (urst.by - ur.by) + spd[3] * (urdst.by - urst.by);
-    flx[L_BK] = fr.bz + spd[4] * (urst.bz - ur.bz) + spd[3] * (urdst.bz - urst.bz);
+    flx[L_D] = add_mul(add_mul(fr.d, spd[4], urst.d - ur.d), spd[3], urdst.d - urst.d);
+    flx[L_VI] = add_mul(add_mul(fr.mx, spd[4], urst.mx - ur.mx), spd[3], urdst.mx - urst.mx);
+    flx[L_VJ] = add_mul(add_mul(fr.my, spd[4], urst.my - ur.my), spd[3], urdst.my - urst.my);
+    flx[L_VK] = add_mul(add_mul(fr.mz, spd[4], urst.mz - ur.mz), spd[3], urdst.mz - urst.mz);
+    flx[L_E] = add_mul(add_mul(fr.e, spd[4], urst.e - ur.e), spd[3], urdst.e - urst.e);
+    flx[L_BJ] = add_mul(add_mul(fr.by, spd[4], urst.by - ur.by), spd[3], urdst.by - urst.by);
+    flx[L_BK] = add_mul(add_mul(fr.bz, spd[4], urst.bz - ur.bz), spd[3], urdst.bz - urst.bz);
   } else {
     flux_r();
-    flx[L_D] = fr.d + spd[4] * (urst.d - ur.d);
-    flx[L_VI] = fr.mx + spd[4] * (urst.mx - ur.mx);
-    flx[L_VJ] = fr.my + spd[4] * (urst.my - ur.my);
-    flx[L_VK] = fr.mz + spd[4] * (urst.mz - ur.mz);
-    flx[L_E] = fr.e + spd[4] * (urst.e - ur.e);
-    flx[L_BJ] = fr.by + spd[4] * (urst.by - ur.by);
-    flx[L_BK] = fr.bz + spd[4] * (urst.bz - ur.bz);
+    flx[L_D] = add_mul(fr.d, spd[4], urst.d - ur.d);
+    flx[L_VI] = add_mul(fr.mx, spd[4], urst.mx - ur.mx);
+    flx[L_VJ] = add_mul(fr.my, spd[4], urst.my - ur.my);
+    flx[L_VK] = add_mul(fr.mz, spd[4], urst.mz - ur.mz);
+    flx[L_E] = add_mul(fr.e, spd[4], urst.e - ur.e);
+    flx[L_BJ] = add_mul(fr.by, spd[4], urst.by - ur.by);
+    flx[L_BK] = add_mul(fr.bz, spd[4], urst.bz - ur.bz);
   }
   flx[L_BI] = T(0);
 }
 
 // conserved state + physical flux, MHD LUT (EnzoRiemannUtils.hpp:48-149)
-template <typename T>
+template <class O, typename T>
 __device__ __forceinline__ void mhd_cons_flux(const T w[8], T gamma, T cons[8],
                                               T flux[8]) {
   for (int i = 0; i < 4; i++) cons[i] = w[i];
   for (int i = 4; i < 8; i++) cons[i] = w[i] * w[L_D];
   {
     T density = w[L_D];
-    T internal_edens = qdiv_inv(w[L_E], gamma - T(1), qrcp(gamma - T(1)));
     const T vi = w[L_VI], vj = w[L_VJ], vk = w[L_VK];
-    const T kinetic = T(0.5) * density * ((vi * vi) + ((vj * vj) + (vk * vk)));
-    T magnetic = T(0.5) * ((w[L_BI] * w[L_BI]) +
-                           ((w[L_BJ] * w[L_BJ]) + (w[L_BK] * w[L_BK])));
-    cons[L_E] = internal_edens + kinetic + magnetic;
+    const T v2 = mad(vi, vi, dot2<O::kj>(vj, vj, vk, vk));
+    const T gm1 = gamma - T(1);
+    // with the magnetic energy density
+    cons[L_E] = add_mul(energy_density<O::energy>(w[L_E], gm1, qrcp(gm1), T(0.5) * density, v2),
+                        T(0.5),
+                        mad(w[L_BI], w[L_BI], dot2<O::kj>(w[L_BJ], w[L_BJ], w[L_BK], w[L_BK])));
   }
   const T vi = w[L_VI], vj = w[L_VJ], vk = w[L_VK];
   const T Bi = w[L_BI], Bj = w[L_BJ], Bk = w[L_BK];
   const T etot = cons[L_E];
-  const T ptot = w[L_E] + T(0.5) * ((Bi * Bi) + ((Bj * Bj) + (Bk * Bk)));
+  const T ptot = add_mul(w[L_E], T(0.5), mad(Bi, Bi, dot2<O::kj>(Bj, Bj, Bk, Bk)));
   const T mom_i = cons[L_VI];
   flux[L_D] = mom_i;
-  flux[L_VI] = mom_i * vi - Bi * Bi + ptot;
-  flux[L_VJ] = mom_i * vj - Bj * Bi;
-  flux[L_VK] = mom_i * vk - Bk * Bi;
-  flux[L_E] = ((etot + ptot) * vi - (Bi * vi + (Bj * vj + Bk * vk)) * Bi);
+  flux[L_VI] = msub(mom_i, vi, Bi * Bi) + ptot;
+  flux[L_VJ] = msub(mom_i, vj, Bj * Bi);
+  flux[L_VK] = msub(mom_i, vk, Bk * Bi);
+  flux[L_E] = msub(etot + ptot, vi, mad(Bi, vi, dot2<O::kj>(Bj, vj, Bk, vk)) * Bi);
   flux[L_BI] = T(0);
-  flux[L_BJ] = Bj * vi - Bi * vj;
-  flux[L_BK] = Bk * vi - Bi * vk;
+  flux[L_BJ] = msub(Bj, vi, Bi * vj);
+  flux[L_BK] = msub(Bk, vi, Bi * vk);
 }
 
 // HLLE for MHD: HLLKernel<EinfeldtWavespeed<MHDLUT>>
 // (EnzoRiemannHLL.hpp:44-172, 238-320); vbar (dual energy, may be null):
 // the normal velocity interpolated between the outer speeds (:330-340)
-template <typename T>
+template <class O = SumOrder<0, false, false>, typename T>
 __device__ __forceinline__ void hlle_mhd(const T wl[8], const T wr[8],
                                          T gamma, T flux[8],
                                          T *vbar = nullptr) {
   T cl[8], cr[8], fl[8], fr[8];
-  mhd_cons_flux(wl, gamma, cl, fl);
-  mhd_cons_flux(wr, gamma, cr, fr);
+  mhd_cons_flux<O>(wl, gamma, cl, fl);
+  mhd_cons_flux<O>(wr, gamma, cr, fr);
   T c_l, c_r;
-  fast_ms_speeds(wl, wr, gamma, c_l, c_r);
+  fast_ms_speeds<O>(wl, wr, gamma, c_l, c_r);
   T left_speed = (wl[L_VI] - c_l);
   T right_speed = (wr[L_VI] + c_r);
   T sqrtrho_l, sqrtrho_r;
   qsqrt2(wl[L_D], wr[L_D], sqrtrho_l, sqrtrho_r);
   T inv_sqrtrho_tot = qrcp(sqrtrho_l + sqrtrho_r);
-  T vi_roe = (sqrtrho_l * wl[L_VI] + sqrtrho_r * wr[L_VI]) * inv_sqrtrho_tot;
-  T vj_roe = (sqrtrho_l * wl[L_VJ] + sqrtrho_r * wr[L_VJ]) * inv_sqrtrho_tot;
-  T vk_roe = (sqrtrho_l * wl[L_VK] + sqrtrho_r * wr[L_VK]) * inv_sqrtrho_tot;
-  T v_roe2 = vi_roe * vi_roe + vj_roe * vj_roe + vk_roe * vk_roe;
-  T ptot_l = wl[L_E];
-  T ptot_r = wr[L_E];
-  ptot_l += T(0.5) * ((wl[L_BI] * wl[L_BI]) +
-                      ((wl[L_BJ] * wl[L_BJ]) + (wl[L_BK] * wl[L_BK])));
-  ptot_r += T(0.5) * ((wr[L_BI] * wr[L_BI]) +
-                      ((wr[L_BJ] * wr[L_BJ]) + (wr[L_BK] * wr[L_BK])));
+  const T vi_sum = dot2<O::rl>(sqrtrho_l, wl[L_VI], sqrtrho_r, wr[L_VI]);
+  T vi_roe = vi_sum * inv_sqrtrho_tot;
+  T vj_roe = dot2<O::rl>(sqrtrho_l, wl[L_VJ], sqrtrho_r, wr[L_VJ]) * inv_sqrtrho_tot;
+  T vk_roe = dot2<O::rl>(sqrtrho_l, wl[L_VK], sqrtrho_r, wr[L_VK]) * inv_sqrtrho_tot;
+  T v_roe2 = add_mul(dot2<O::ji_roe>(vi_roe, vi_roe, vj_roe, vj_roe), vk_roe, vk_roe);
+  const T ptot_l = add_mul(wl[L_E], T(0.5),
+                           mad(wl[L_BI], wl[L_BI], dot2<O::kj>(wl[L_BJ], wl[L_BJ], wl[L_BK], wl[L_BK])));
+  const T ptot_r = add_mul(wr[L_E], T(0.5),
+                           mad(wr[L_BI], wr[L_BI], dot2<O::kj>(wr[L_BJ], wr[L_BJ], wr[L_BK], wr[L_BK])));
   T h_l = qdiv_inv(cl[L_E] + ptot_l, wl[L_D], qrcp(wl[L_D]));
   T h_r = qdiv_inv(cr[L_E] + ptot_r, wr[L_D], qrcp(wr[L_D]));
-  T h_roe = (sqrtrho_l * h_l + sqrtrho_r * h_r) * inv_sqrtrho_tot;
+  const T h_sum = mad(sqrtrho_l, h_l, sqrtrho_r * h_r);
   // roe_cfast_
   T rho_roe = sqrtrho_l * sqrtrho_r;
   T rho_roe_inv = qrcp(rho_roe);
   T bi_roe = wl[L_BI];
-  T bj_roe = (sqrtrho_l * wr[L_BJ] + sqrtrho_r * wl[L_BJ]) * inv_sqrtrho_tot;
-  T bk_roe = (sqrtrho_l * wr[L_BK] + sqrtrho_r * wl[L_BK]) * inv_sqrtrho_tot;
-  T b_roe2 = bi_roe * bi_roe + bj_roe * bj_roe + bk_roe * bk_roe;
+  T bj_roe = add_mul(sqrtrho_l * wr[L_BJ], sqrtrho_r, wl[L_BJ]) * inv_sqrtrho_tot;
+  T bk_roe = add_mul(sqrtrho_l * wr[L_BK], sqrtrho_r, wl[L_BK]) * inv_sqrtrho_tot;
+  T b_roe2 = add_mul(add_mul(bi_roe * bi_roe, bj_roe, bj_roe), bk_roe, bk_roe);
   T gamma_prime = gamma - T(1);
   T dbj = wl[L_BJ] - wr[L_BJ];
   T dbk = wl[L_BK] - wr[L_BK];
   T x_prime =
-      ((dbj * dbj + dbk * dbk) * T(0.5) * (gamma_prime - T(1)) * inv_sqrtrho_tot);
-  T y_prime =
-      qdiv_inv((gamma_prime - T(1)) * (wl[L_D] + wr[L_D]) * T(0.5), rho_roe, rho_roe_inv);
-  T tilde_a2 =
-      (gamma_prime * (h_roe - T(0.5) * v_roe2 - qdiv_inv(b_roe2, rho_roe, rho_roe_inv)) -
-       x_prime);
+      (dot2<O::kj>(dbj, dbj, dbk, dbk) * T(0.5) * (gamma_prime - T(1)) * inv_sqrtrho_tot);
+  // gamma_prime - y_prime
+  const T gy = sub_div(gamma_prime, (gamma_prime - T(1)) * (wl[L_D] + wr[L_D]) * T(0.5), rho_roe,
+                       rho_roe_inv);
+  // (h_roe - v_roe2 / 2 first)
+  T tilde_a2 = msub(gamma_prime,
+                    sub_div(msub(h_sum, inv_sqrtrho_tot, T(0.5) * v_roe2), b_roe2, rho_roe,
+                            rho_roe_inv),
+                    x_prime);
   T tilde_vai2 = qdiv_inv(bi_roe * bi_roe, rho_roe, rho_roe_inv);
-  T tilde_va2 = (tilde_vai2 + qdiv_inv((gamma_prime - y_prime) *
-                                           (bj_roe * bj_roe + bk_roe * bk_roe),
-                                       rho_roe, rho_roe_inv));
+  T tilde_va2 = add_div(tilde_vai2, gy * dot2<O::kj_roe>(bj_roe, bj_roe, bk_roe, bk_roe), rho_roe,
+                        rho_roe_inv);
   T s = tilde_a2 + tilde_va2;
-  T c_roe = qsqrt(T(0.5) * (tilde_a2 + tilde_va2 +
-                            qsqrt(s * s - T(4) * tilde_a2 * tilde_vai2)));
-  T bp = fmax(vi_roe + c_roe, right_speed);
-  T bm = fmin(vi_roe - c_roe, left_speed);
+  T c_roe = qsqrt(T(0.5) * (s + qsqrt(msub(s, s, T(4) * tilde_a2 * tilde_vai2))));
+  T bp = fmax(mad(vi_sum, inv_sqrtrho_tot, c_roe), right_speed);
+  T bm = fmin(msub(vi_sum, inv_sqrtrho_tot, c_roe), left_speed);
   bp = fmax(bp, T(0));
   bm = fmin(bm, T(0));
   T inv_speed_diff = qrcp(bp - bm);
 #pragma unroll
   for (int f = 0; f < 8; f++) {
-    flux[f] = ((bp * fl[f] - bm * fr[f] + (cr[f] - cl[f]) * bp * bm) *
-               inv_speed_diff);
+    const bool mom = f == L_VI || f == L_VJ || f == L_VK;
+    const T diff = mom ? msub(wr[f], wr[L_D], cl[f]) : cr[f] - cl[f];
+    flux[f] = add_mul(msub(bp, fl[f], bm * fr[f]), diff * bp, bm) * inv_speed_diff;
   }
   if (vbar) *vbar = (bp * wl[L_VI] - bm * wr[L_VI]) * inv_speed_diff;
 }
@@ -567,7 +664,7 @@ __device__ __forceinline__ void hlle_mhd(const T wl[8], const T wr[8],
 // HLLC (HLLCKernel::operator(), EnzoRiemannHLLC.hpp:34-172) with
 // EinfeldtWavespeed<HydroLUT> (EnzoRiemannHLL.hpp:44-130).  Hydro LUT.
 // vbar (dual energy, may be null): the weighted outer velocities of :166-170
-template <typename T>
+template <class O = SumOrder<0, false, false>, typename T>
 __device__ __forceinline__ void hllc(const T wl[5], const T wr[5], T gamma,
                                      T flux[5], T *vbar = nullptr) {
   const T pressure_l = wl[H_E];
@@ -581,11 +678,10 @@ __device__ __forceinline__ void hllc(const T wl[5], const T wr[5], T gamma,
       c[s][H_D] = w[s][H_D];
       for (int i = 1; i < 5; i++) c[s][i] = w[s][i] * w[s][H_D];
       T density = w[s][H_D];
-      T internal_edens = qdiv_inv(w[s][H_E], gamma - T(1), qrcp(gamma - T(1)));
       const T vi = w[s][H_VI], vj = w[s][H_VJ], vk = w[s][H_VK];
-      const T kinetic =
-          T(0.5) * density * ((vi * vi) + ((vj * vj) + (vk * vk)));
-      c[s][H_E] = internal_edens + kinetic + T(0);
+      const T gm1 = gamma - T(1);
+      c[s][H_E] = energy_density<O::energy>(w[s][H_E], gm1, qrcp(gm1), T(0.5) * density,
+                                            mad(vi, vi, dot2<O::kj>(vj, vj, vk, vk))) + T(0);
     }
   }
   T cs_l, cs_r;
@@ -599,27 +695,28 @@ __device__ __forceinline__ void hllc(const T wl[5], const T wr[5], T gamma,
     T sqrtrho_l, sqrtrho_r;
     qsqrt2(wl[H_D], wr[H_D], sqrtrho_l, sqrtrho_r);
     T inv_sqrtrho_tot = qrcp(sqrtrho_l + sqrtrho_r);
-    T vi_roe = (sqrtrho_l * wl[H_VI] + sqrtrho_r * wr[H_VI]) * inv_sqrtrho_tot;
-    T vj_roe = (sqrtrho_l * wl[H_VJ] + sqrtrho_r * wr[H_VJ]) * inv_sqrtrho_tot;
-    T vk_roe = (sqrtrho_l * wl[H_VK] + sqrtrho_r * wr[H_VK]) * inv_sqrtrho_tot;
-    T v_roe2 = vi_roe * vi_roe + vj_roe * vj_roe + vk_roe * vk_roe;
+    const T vi_sum = dot2<O::rl>(sqrtrho_l, wl[H_VI], sqrtrho_r, wr[H_VI]);
+    T vi_roe = vi_sum * inv_sqrtrho_tot;
+    T vj_roe = dot2<O::rl>(sqrtrho_l, wl[H_VJ], sqrtrho_r, wr[H_VJ]) * inv_sqrtrho_tot;
+    T vk_roe = dot2<O::rl>(sqrtrho_l, wl[H_VK], sqrtrho_r, wr[H_VK]) * inv_sqrtrho_tot;
+    T v_roe2 = add_mul(dot2<O::ji_roe>(vi_roe, vi_roe, vj_roe, vj_roe), vk_roe, vk_roe);
     T h_l = qdiv_inv(cons_l[H_E] + pressure_l, wl[H_D], inv_l);
     T h_r = qdiv_inv(cons_r[H_E] + pressure_r, wr[H_D], inv_r);
-    T h_roe = (sqrtrho_l * h_l + sqrtrho_r * h_r) * inv_sqrtrho_tot;
-    T temp = h_roe - T(0.5) * v_roe2;
+    // h_roe - v_roe2 / 2
+    T temp = msub(dot2<O::rl>(sqrtrho_l, h_l, sqrtrho_r, h_r), inv_sqrtrho_tot, T(0.5) * v_roe2);
     T c_roe = qsqrt((gamma - T(1)) * dmax(temp, T(0)));
-    cs_r = fmax(vi_roe + c_roe, right_speed);
-    cs_l = fmin(vi_roe - c_roe, left_speed);
+    cs_r = fmax(mad(vi_sum, inv_sqrtrho_tot, c_roe), right_speed);
+    cs_l = fmin(msub(vi_sum, inv_sqrtrho_tot, c_roe), left_speed);
   }
   T bm = fmin(cs_l, T(0));
   T bp = fmax(cs_r, T(0));
-  T tl = (pressure_l - (cs_l - wl[H_VI]) * wl[H_D] * wl[H_VI]);
-  T tr = (pressure_r - (cs_r - wr[H_VI]) * wr[H_D] * wr[H_VI]);
+  T tl = sub_mul(pressure_l, (cs_l - wl[H_VI]) * wl[H_D], wl[H_VI]);
+  T tr = sub_mul(pressure_r, (cs_r - wr[H_VI]) * wr[H_D], wr[H_VI]);
   T dl = wl[H_D] * (cs_l - wl[H_VI]);
   T dr = -wr[H_D] * (cs_r - wr[H_VI]);
-  T q1 = qrcp(dl + dr);
+  T q1 = qrcp(add_mul(dl, -wr[H_D], cs_r - wr[H_VI]));  // 1 / (dl + dr)
   T cw = (tr - tl) * q1;
-  T cp = (dl * tr + dr * tl) * q1;
+  T cp = mad(dl, tr, dr * tl) * q1;
   T sl, sr, sm;
   {
     // the contact's side: its share of the outer flux, |cw| / (its distance
@@ -635,21 +732,21 @@ __device__ __forceinline__ void hllc(const T wl[5], const T wr[5], T gamma,
   cp = dmax(cp, T(0));
   T momentumi_l = cons_l[H_VI];
   T momentumi_r = cons_r[H_VI];
-  T dfl = momentumi_l - bm * wl[H_D];
-  T dfr = momentumi_r - bp * wr[H_D];
-  T ufl = momentumi_l * (wl[H_VI] - bm) + pressure_l;
-  T ufr = momentumi_r * (wr[H_VI] - bp) + pressure_r;
+  T dfl = sub_mul(momentumi_l, bm, wl[H_D]);
+  T dfr = sub_mul(momentumi_r, bp, wr[H_D]);
+  T ufl = mad(momentumi_l, wl[H_VI] - bm, pressure_l);
+  T ufr = mad(momentumi_r, wr[H_VI] - bp, pressure_r);
   T vfl = (wl[H_D] * wl[H_VJ] * (wl[H_VI] - bm));
   T vfr = (wr[H_D] * wr[H_VJ] * (wr[H_VI] - bp));
   T wfl = (wl[H_D] * wl[H_VK] * (wl[H_VI] - bm));
   T wfr = (wr[H_D] * wr[H_VK] * (wr[H_VI] - bp));
-  T efl = (cons_l[H_E] * (wl[H_VI] - bm) + pressure_l * wl[H_VI]);
-  T efr = (cons_r[H_E] * (wr[H_VI] - bp) + pressure_r * wr[H_VI]);
-  flux[H_D] = sl * dfl + sr * dfr;
-  flux[H_VI] = sl * ufl + sr * ufr + (sm * cp);
-  flux[H_VJ] = sl * vfl + sr * vfr;
-  flux[H_VK] = sl * wfl + sr * wfr;
-  flux[H_E] = sl * efl + sr * efr + (sm * cp * cw);
+  T efl = add_mul(cons_l[H_E] * (wl[H_VI] - bm), pressure_l, wl[H_VI]);
+  T efr = add_mul(cons_r[H_E] * (wr[H_VI] - bp), pressure_r, wr[H_VI]);
+  flux[H_D] = add_mul(sl * dfl, sr, dfr);
+  flux[H_VI] = add_mul(add_mul(sl * ufl, sr, ufr), sm, cp);
+  flux[H_VJ] = add_mul(sl * vfl, sr, vfr);
+  flux[H_VK] = add_mul(sl * wfl, sr, wfr);
+  flux[H_E] = add_mul(add_mul(sl * efl, sr, efr), sm * cp, cw);
 }
 
 }  // namespace ENZOE_KNS

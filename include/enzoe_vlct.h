@@ -728,10 +728,10 @@ int enzoe_vlct_transfer_batch(enzoe_vlct_t m, const enzoe_transfer *items,
  * call on, FP64 hydro 3 2^17, where no debug counts, stored fluxes or
  * flux-launch shape are asked for), else variant 2 for MHD launches of fewer
  * than 2^19 cells (ghost zones included), else the four launches.
- * Every variant gives the same bits in FP64 (the mixed and contracted
- * builds: up to the rounding of their contracted flux arithmetic, which the
- * compiler may fuse differently in different kernels).  Not to be changed
- * while work of the method is queued.
+ * Every variant gives the same bits, in FP64 and in mixed precision (the
+ * contracted build: up to the rounding of its flux arithmetic, whose
+ * multiply-adds the compiler may fuse differently in different kernels).  Not
+ * to be changed while work of the method is queued.
  * enzoe_vlct_check_persistent: synchronises and reports ENZOE_ERR_HIP if a
  * barrier wait of a persistent launch ran out (the workgroups of a launch
  * could not all be resident: results since the last check are not valid;
@@ -748,7 +748,7 @@ int enzoe_vlct_check_persistent(enzoe_vlct_t m);
  * (the reconstructing stage as 0); -1 (the default), the autotuner's
  * choice per block shape (until it has run, 1 for launches of fewer than 2^18
  * cells, ghost zones included, else 0).  Every shape gives the same
- * bits in FP64; the mixed and contracted builds fuse their flux
+ * bits in FP64 and in mixed precision; the contracted build fuses its flux
  * multiply-adds as the compiler finds them in each kernel, so there the
  * shapes agree to the rounding of that arithmetic.                         */
 int enzoe_vlct_set_flux_shape(enzoe_vlct_t m, int shape);
