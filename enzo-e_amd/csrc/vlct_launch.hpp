@@ -781,8 +781,10 @@ void dispatch_march_hd(int recon, const BlockDesc<T> *d, int nb, int mx, int my,
     launch_march_hd<T, RC_PLM_ATHENA, DE, true>(d, nb, mx, my, mz, sp, s);
 }
 
-// Whether a hydrodynamic stage of small blocks is one launch of k_tile: no
-// debug counts (the faces between tiles are solved twice), no structure or
+// Whether a hydrodynamic stage of small blocks is one launch of k_tile: a
+// scheme of two stages (the one stage of the other updates the state in
+// place, which tiles beside it still read), no debug counts (the faces between
+// tiles are solved twice), no structure or
 // flux-launch shape asked for or tuned, and fewer than 2^16 cells with ghosts (dual
 // energy: 2^15), where a launch costs more than the repeated faces.  Cycle in
 // us, separate and tiled -- FP64: one block of 12^3 38.4, 36.0; 16^3 39.1,
@@ -790,8 +792,8 @@ void dispatch_march_hd(int recon, const BlockDesc<T> *d, int nb, int mx, int my,
 // 54.8, 57.5; 48^3 65.9, 70.8.  Dual energy: 24^3 44.2, 38.6; 32^3 51.9, 52.3.
 // Mixed: 16^3 35.8, 30.8; 32^3 40.2, 36.7; 8 of 16^3 46.5, 46.0.
 inline bool tile_ok(const enzoe_vlct_method *m, int mx, int my, int mz, int nb) {
-  if (m->mhd || m->d_dbg || m->force_ctu >= 0 || m->force_shape >= 0 || m->ctu >= 0 ||
-      m->flux_shape >= 0 || m->tuned_ctu.count(shape_key(mx, my, mz)) ||
+  if (m->mhd || m->nstages != 2 || m->d_dbg || m->force_ctu >= 0 || m->force_shape >= 0 ||
+      m->ctu >= 0 || m->flux_shape >= 0 || m->tuned_ctu.count(shape_key(mx, my, mz)) ||
       std::min(mx, std::min(my, mz)) < 7)
     return false;
   return (long)mx * my * mz * nb < (m->dual ? 1L << 15 : 1L << 16);

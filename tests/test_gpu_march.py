@@ -266,3 +266,44 @@ def test_refresh_copies_every_field(n, nblocks, bc, mhd, dual):
             want = np.stack([s[name] for s in states])[
                 b, idx[2][:, None, None], idx[1][:, None], idx[0]]
             assert np.array_equal(x, want), (i, name)
+
+
+@pytest.mark.parametrize("n", [(10, 9, 8), (25, 18, 21), (72, 70, 68)])
+@pytest.mark.parametrize("recon,dual", [("nn", False), ("plm", False), ("plm_athena", False),
+                                        ("plm", True)])
+def test_one_stage_scheme_equals_the_oracle(recon, dual, n):
+    """The one-stage ("euler") scheme updates the state in place, so its stage
+    may not be one launch that solves the faces around the cells it updates:
+    small and large hydrodynamic blocks against the oracle, and no tiled or
+    marched launch."""
+    from _states import random_periodic_grid
+    from test_gpu_parity import device_copy
+    ev = _ev()
+    grid = random_periodic_grid(mhd=False, seed=3, n=n, riemann="hllc", recon=(recon,),
+                                theta=1.6, vamp=0.6)
+    assert grid.cfg.nstages == 1
+    if dual:
+        grid.cfg.dual_energy = 1
+        grid.cfg.eta = 0.001
+        arr = grid.block_arrays(0)
+        arr["internal_energy"][...] = arr["total_energy"] - 0.5 * sum(
+            np.square(arr["velocity_" + c]) for c in "xyz")
+    c = grid.cfg
+    m = ev.VlctMethod(mhd=False, riemann="hllc", reconstruct=recon, time_scheme="euler",
+                      theta=c.theta_limiter, courant=c.courant, gamma=c.gamma,
+                      density_floor=c.density_floor, pressure_floor=c.pressure_floor,
+                      dual_energy_eta=c.eta if dual else None)
+    dg = device_copy(grid, m)
+    ev.profiling(True)
+    t = 0.0
+    for _ in range(3):
+        dt = grid.cycle(t, 10.0)
+        assert dg.cycle(t, 10.0) == dt
+        t += dt
+    names = ev.profile_report()
+    ev.profiling(False)
+    assert not any(k.startswith(("k_tile", "k_march")) for k in names)
+    got, want = dg.blocks[0].download(), grid.block_arrays(0)
+    for k in got:
+        if k in want:
+            assert np.array_equal(got[k], want[k]), k
