@@ -480,6 +480,7 @@ int enzoe_vlct_destroy(enzoe_vlct_t m) {
   if (m->scratch) (void)hipFree(m->scratch);
   if (m->d_desc) (void)hipFree(m->d_desc);
   if (m->d_dt) (void)hipFree(m->d_dt);
+  if (m->d_step_dt) (void)hipFree(m->d_step_dt);
   if (m->h_dt) (void)hipHostFree(m->h_dt);
   if (m->d_ptrtab) (void)hipFree(m->d_ptrtab);
   if (m->d_dts) (void)hipFree(m->d_dts);
@@ -709,32 +710,32 @@ int launch_dt(enzoe_vlct_method *m, const enzoe_block *blocks, int n, hipStream_
   long maxcells = 0;
   for (int i = 0; i < n; i++)
     maxcells = std::max<long>(maxcells, (long)blocks[i].mx * blocks[i].my * blocks[i].mz);
-  m->dt_ready = false;
   return launch_dt_on(m, (const BlockDesc<double> *)m->d_ptrtab, n, maxcells, m->d_dt, s,
                       d_time, t_stop);
 }
 
-// Waits for the stream and returns courant * the minimum in m->d_dt.  The
-// word comes over through pinned memory, written by a one-thread kernel that
-// also makes it ready for the next minimum: a copy to pageable memory is a
-// kernel of its own and stages through the runtime's buffers, and the next
-// call would set the word in another launch (cycle of one 16^3 hydro block
-// 47.7 us so, 38.7 this way).
-int read_dt(enzoe_vlct_method *m, hipStream_t s, double *dt) {
+// Waits for the stream and returns courant * the minimum in *word.  It
+// comes over through pinned memory, written by a one-thread kernel that also
+// leaves the word ready for the next minimum (*reset, if not null): a copy to
+// pageable memory is a kernel of its own and stages through the runtime's
+// buffers, and the next call would set the word in another launch (cycle of
+// one 16^3 hydro block 47.7 us so, 38.7 this way).
+int read_dt(enzoe_vlct_method *m, unsigned long long *word, hipStream_t s, double *dt,
+            bool *reset) {
   if (!m->h_dt && hipHostMalloc((void **)&m->h_dt, sizeof(unsigned long long),
                                 hipHostMallocDefault) != hipSuccess)
     m->h_dt = nullptr;
   unsigned long long bits = 0;
   if (m->h_dt) {
-    hipLaunchKernelGGL(k_dt_out, dim3(1), dim3(1), 0, s, m->d_dt, m->h_dt);
+    hipLaunchKernelGGL(k_dt_out, dim3(1), dim3(1), 0, s, word, m->h_dt);
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
       return ENZOE_ERR_HIP;
     bits = *(volatile unsigned long long *)m->h_dt;
-    m->dt_ready = true;
+    if (reset) *reset = true;
   } else {
     // no pinned memory: a plain copy
     (void)hipGetLastError();
-    if (hipMemcpyAsync(&bits, m->d_dt, sizeof(bits), hipMemcpyDeviceToHost, s) != hipSuccess ||
+    if (hipMemcpyAsync(&bits, word, sizeof(bits), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
       return ENZOE_ERR_HIP;
   }
@@ -753,7 +754,7 @@ int enzoe_vlct_timestep(enzoe_vlct_t m, const enzoe_block *blocks, int n,
   if (!m || !blocks || n <= 0 || !dt_out) return ENZOE_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
   if (int rc = launch_dt(m, blocks, n, s)) return rc;
-  return read_dt(m, s, dt_out);
+  return read_dt(m, m->d_dt, s, dt_out, nullptr);
 }
 
 int enzoe_vlct_compute_timestep(enzoe_vlct_t m, const enzoe_block *blocks, int n,
@@ -762,19 +763,18 @@ int enzoe_vlct_compute_timestep(enzoe_vlct_t m, const enzoe_block *blocks, int n
   hipStream_t s = (hipStream_t)stream;
   for (int i = 0; i < n; i++)
     if (int rc = check_block(m, blocks[i])) return rc;
-  if (!m->d_dt &&
-      hipMalloc((void **)&m->d_dt, sizeof(unsigned long long)) != hipSuccess) {
-    m->d_dt = nullptr;
+  if (!m->d_step_dt &&
+      hipMalloc((void **)&m->d_step_dt, sizeof(unsigned long long)) != hipSuccess) {
+    m->d_step_dt = nullptr;
     return ENZOE_ERR_ALLOC;
   }
   // the final k_cells covers every cell: the update, and the CFL term of
-  // each cell of the block into m->d_dt
-  if (!m->dt_ready) hipLaunchKernelGGL(k_dt_init, dim3(1), dim3(1), 0, s, m->d_dt);
-  m->dt_ready = false;
-  if (int rc = compute_runs(m, blocks, n, dt, nullptr, s, nullptr, nullptr,
-                            (unsigned long long *)m->d_dt))
+  // each cell of the block into the word
+  if (!m->step_dt_ready) hipLaunchKernelGGL(k_dt_init, dim3(1), dim3(1), 0, s, m->d_step_dt);
+  m->step_dt_ready = false;
+  if (int rc = compute_runs(m, blocks, n, dt, nullptr, s, nullptr, nullptr, m->d_step_dt))
     return rc;
-  return read_dt(m, s, dt_next);
+  return read_dt(m, m->d_step_dt, s, dt_next, &m->step_dt_ready);
 }
 
 int enzoe_vlct_timestep_device(enzoe_vlct_t m, const enzoe_block *blocks, int n,
@@ -1387,7 +1387,6 @@ struct MethodBuffers {
     std::swap(desc_bytes, m->desc_bytes);
     std::swap(last_desc, m->last_desc);
     void *dt = (void *)m->d_dt;
-    m->dt_ready = false;  // of the word that goes out
     std::swap(d_dt, dt);
     m->d_dt = (unsigned long long *)dt;
     std::swap(d_ptrtab, m->d_ptrtab);

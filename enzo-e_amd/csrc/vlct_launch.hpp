@@ -117,12 +117,16 @@ struct enzoe_vlct_method {
   void *d_desc = nullptr;
   size_t desc_bytes = 0;
   std::vector<char> last_desc;
+  // the CFL minimum of a pass of its own and of device-driven cycles, whose
+  // launches a caller's graph may hold and replay at any time
   unsigned long long *d_dt = nullptr;
-  // the CFL minimum on its way to the host: a pinned word that k_dt_out
-  // writes (null: not allocated), and whether that kernel has left *d_dt
-  // ready for the next minimum
+  // the CFL minimum that a host-driven step takes, a word that no captured
+  // work touches, and whether k_dt_out has left it ready for the next one
+  unsigned long long *d_step_dt = nullptr;
+  bool step_dt_ready = false;
+  // a CFL minimum on its way to the host: a pinned word that k_dt_out writes
+  // (null: not allocated)
   unsigned long long *h_dt = nullptr;
-  bool dt_ready = false;
   void *d_ptrtab = nullptr;
   size_t ptrtab_bytes = 0;
   std::vector<char> last_dt_desc;  // host copy of the dt descriptor table
