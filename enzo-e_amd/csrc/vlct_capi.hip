@@ -861,8 +861,6 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
     for (int mask = 0; mask < 16; mask++)
       if (v == 0 || (mask & (v == 4 ? 4 : 6)) == 0) cand.push_back({v, mask});
   }
-  // the marched stages (setting "auto" of both structure and flux launch)
-  if (m->nstages == 2 && fixed < 0 && m->flux_shape < 0) cand.push_back({MARCH_STRUCTURE, 0});
   if (persistent_ok(m) && (fixed == -1 || fixed == 5))
     if (int rc2 = ensure_barrier(m)) rc = rc2;
   // the time of one step of the sample under the forced settings: a timed
@@ -942,7 +940,7 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
   // workgroups for small blocks; z pencils for the nearest-neighbour
   // stage), for the chosen structure, order and rows
   int best_shape = 0;
-  if (best_ctu < 5 && m->flux_shape < 0 && rc == ENZOE_OK) {
+  if (best_ctu != 5 && m->flux_shape < 0 && rc == ENZOE_OK) {
     m->force_mask = best;
     m->force_ctu = best_ctu;
     m->force_rows = best_rows;
@@ -960,6 +958,24 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
     m->force_rows = -1;
     m->force_shape = -1;
   }
+  // then a whole stage as one launch against the best of those (settings
+  // "auto" of both structure and flux launch)
+  int whole = 0;
+  if (fixed < 0 && m->flux_shape < 0) {
+    for (int v : {MARCH_STRUCTURE, TILE_STRUCTURE}) {
+      if (rc || !(v == MARCH_STRUCTURE ? march_possible(m, mx, my, mz)
+                                       : tile_possible(m, mx, my, mz)))
+        continue;
+      m->force_ctu = v;
+      float ms = 0.f;
+      rc = time_runs(&ms);
+      if (rc == ENZOE_OK && ms < best_ms) {
+        best_ms = ms;
+        whole = v;
+      }
+    }
+    m->force_ctu = -1;
+  }
   g_profiling = prof;
   (void)hipStreamSynchronize(s);
   if (e0) (void)hipEventDestroy(e0);
@@ -970,6 +986,8 @@ int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
   m->tuned_ctu[shape_key(mx, my, mz)] = best_ctu;
   m->tuned_rows[shape_key(mx, my, mz)] = best_rows;
   m->tuned_shape[shape_key(mx, my, mz)] = best_shape;
+  if (fixed < 0 && m->flux_shape < 0)
+    m->tuned_whole[whole_key(mx, my, mz, blocks[0].ghost, ns)] = whole;
   if (mask_out) *mask_out = best;
   return ENZOE_OK;
 }
@@ -983,7 +1001,7 @@ int enzoe_vlct_launch_choice(enzoe_vlct_t m, int mx, int my, int mz, int *mask, 
   if (fused_ct) {
     const int v = ctu_variant(m, mx, my, mz, 1);
     *fused_ct = (v == 5) ? (persistent_ok(m) ? 5 : 0)
-                         : ((m->mhd && ctu_possible(m) && v < 5) ? v : 0);
+                         : ((m->mhd && ctu_possible(m)) ? v : 0);
   }
   return ENZOE_OK;
 }

@@ -92,6 +92,11 @@ struct enzoe_vlct_method {
   int ctu = -1;
   int force_ctu = -1;                    // set while the autotuner times one
   std::map<long long, int> tuned_ctu;    // the autotuner's choice per shape
+  // the autotuner's choice between those separate launches (0) and a whole
+  // stage as one launch (MARCH_STRUCTURE, TILE_STRUCTURE), per shape, ghost
+  // depth and size of the launch (whole_key): which of them wins goes with
+  // the number of blocks
+  std::map<std::pair<long long, int>, int> tuned_whole;
   // rows of the tiled cell order per block shape (the autotuner's choice;
   // tile_rows_for otherwise) and the value forced while it times one
   std::map<long long, int> tuned_rows;
@@ -187,9 +192,22 @@ inline int ctu_variant(const enzoe_vlct_method *m, int mx, int my, int mz, int n
   return (m->mhd && m->nstages == 2 && (long)mx * my * mz * nb < (1L << 19)) ? 2 : 0;
 }
 
-// ... and, chosen by march_ok and not by enzoe_vlct_set_fused_ct, the marched
-// stages
-constexpr int MARCH_STRUCTURE = 6;
+// ... and, chosen by march_ok and tile_ok and not by enzoe_vlct_set_fused_ct,
+// the marched stages and the tiled ones
+constexpr int MARCH_STRUCTURE = 6, TILE_STRUCTURE = 7;
+
+inline long active_cells(int mx, int my, int mz, int ghost) {
+  return (long)(mx - 2 * ghost) * (my - 2 * ghost) * (mz - 2 * ghost);
+}
+// Key of tuned_whole: launches of one shape and ghost depth whose active
+// cells lie in the same octave tune together; from 2^20 on (four waves a SIMD
+// at a cell a thread) the device is full and they are all alike.
+inline std::pair<long long, int> whole_key(int mx, int my, int mz, int ghost, int nb) {
+  const unsigned long cells = (unsigned long)active_cells(mx, my, mz, ghost) * nb;
+  int octave = 0;
+  while (octave < 20 && (cells >> (octave + 1)) != 0) octave++;
+  return {shape_key(mx, my, mz), ghost * 32 + octave};
+}
 
 // The fused CT update needs the two stages of the VL scheme (its final
 // stage reads the first stage's copy of the start-of-step faces); the
@@ -602,25 +620,26 @@ struct StoreArgs {
 // k_march_hd): the VL scheme, fields whose byte offsets fit 32 bits, no debug
 // counts (the marched tiles solve the faces of their rings more than once),
 // and no structure or flux-launch shape asked for; then the autotuner's
-// choice for the shape, or else from 2^18 active cells on (FP64 hydro:
-// 3 2^17).  Below that the launches are bound by latency, a plane after
+// choice for launches like this one, or else from 2^18 active cells on (FP64
+// hydro: 3 2^17).  Below that the launches are bound by latency, a plane after
 // the other costs more than it saves, and the separate launches win.  Cycle
 // in us, separate and marched -- MHD: 4 blocks of 32^3 158, 177; one of 48^3
 // 137, 144; 8 of 32^3 229, 230; one of 64^3 202, 202; 4 of 48^3 293, 268; 16
 // of 64^3 2180, 1545.  FP64 hydro: 8 of 32^3 123, 140; one of 64^3 106, 114;
 // 16 of 32^3 201, 163.  Mixed hydro: 4 of 32^3 70, 75; one of 64^3 77, 76;
 // 64 of 16^3 125, 107.
+inline bool march_possible(const enzoe_vlct_method *m, int mx, int my, int mz) {
+  return (!m->mhd || ctu_possible(m)) && m->nstages == 2 && !m->d_dbg &&
+         8ull * (mx + 1) * (my + 1) * (mz + 1) < (1ull << 32);
+}
 inline bool march_ok(const enzoe_vlct_method *m, int mx, int my, int mz, int ghost, int nb) {
-  if ((m->mhd && !ctu_possible(m)) || m->nstages != 2 || m->d_dbg ||
-      8ull * (mx + 1) * (my + 1) * (mz + 1) >= (1ull << 32))
-    return false;
+  if (!march_possible(m, mx, my, mz)) return false;
   if (m->force_ctu >= 0) return m->force_ctu == MARCH_STRUCTURE;
   if (m->ctu >= 0 || m->flux_shape >= 0) return false;
-  auto it = m->tuned_ctu.find(shape_key(mx, my, mz));
-  if (it != m->tuned_ctu.end()) return it->second == MARCH_STRUCTURE;
-  const long active = (long)(mx - 2 * ghost) * (my - 2 * ghost) * (mz - 2 * ghost);
+  auto it = m->tuned_whole.find(whole_key(mx, my, mz, ghost, nb));
+  if (it != m->tuned_whole.end()) return it->second == MARCH_STRUCTURE;
   const bool light = m->mhd || m->precision == ENZOE_PREC_MIXED;
-  return active * nb >= (light ? 1L << 18 : 3L << 17);
+  return active_cells(mx, my, mz, ghost) * nb >= (light ? 1L << 18 : 3L << 17);
 }
 
 // Compute units of the current device, cached per device; 256 if unknown.
@@ -788,18 +807,23 @@ void dispatch_march_hd(int recon, const BlockDesc<T> *d, int nb, int mx, int my,
 // Whether a hydrodynamic stage of small blocks is one launch of k_tile: a
 // scheme of two stages (the one stage of the other updates the state in
 // place, which tiles beside it still read), no debug counts (the faces between
-// tiles are solved twice), no structure or
-// flux-launch shape asked for or tuned, and fewer than 2^16 cells with ghosts (dual
-// energy: 2^15), where a launch costs more than the repeated faces.  Cycle in
+// tiles are solved twice), and no structure or flux-launch shape asked for;
+// then the autotuner's choice for launches like this one, or else fewer than
+// 2^16 cells with ghosts (dual energy: 2^15), where a launch costs more than
+// the repeated faces.  Cycle in
 // us, separate and tiled -- FP64: one block of 12^3 38.4, 36.0; 16^3 39.1,
 // 36.1; 24^3 41.7, 37.0; 32^3 (54872 cells) 48.4, 45.7; 8 of 16^3 (85184)
 // 54.8, 57.5; 48^3 65.9, 70.8.  Dual energy: 24^3 44.2, 38.6; 32^3 51.9, 52.3.
 // Mixed: 16^3 35.8, 30.8; 32^3 40.2, 36.7; 8 of 16^3 46.5, 46.0.
-inline bool tile_ok(const enzoe_vlct_method *m, int mx, int my, int mz, int nb) {
-  if (m->mhd || m->nstages != 2 || m->d_dbg || m->force_ctu >= 0 || m->force_shape >= 0 ||
-      m->ctu >= 0 || m->flux_shape >= 0 || m->tuned_ctu.count(shape_key(mx, my, mz)) ||
-      std::min(mx, std::min(my, mz)) < 7)
-    return false;
+inline bool tile_possible(const enzoe_vlct_method *m, int mx, int my, int mz) {
+  return !m->mhd && m->nstages == 2 && !m->d_dbg && std::min(mx, std::min(my, mz)) >= 7;
+}
+inline bool tile_ok(const enzoe_vlct_method *m, int mx, int my, int mz, int ghost, int nb) {
+  if (!tile_possible(m, mx, my, mz)) return false;
+  if (m->force_ctu >= 0) return m->force_ctu == TILE_STRUCTURE;
+  if (m->force_shape >= 0 || m->ctu >= 0 || m->flux_shape >= 0) return false;
+  auto it = m->tuned_whole.find(whole_key(mx, my, mz, ghost, nb));
+  if (it != m->tuned_whole.end()) return it->second == TILE_STRUCTURE;
   return (long)mx * my * mz * nb < (m->dual ? 1L << 15 : 1L << 16);
 }
 template <typename FluxT, bool DE>
@@ -851,7 +875,7 @@ int launch_chunks(enzoe_vlct_method *m, const enzoe_block *blocks, int n, int ch
   const bool march =
       !st && march_ok(m, mx, my, mz, blocks[0].ghost, std::min(n, chunk));
   const bool tile =
-      !MHD && !st && !march && tile_ok(m, mx, my, mz, std::min(n, chunk));
+      !MHD && !st && !march && tile_ok(m, mx, my, mz, blocks[0].ghost, std::min(n, chunk));
   for (int c0 = 0; c0 < n; c0 += chunk) {
     const int c1 = std::min(n, c0 + chunk);
     const int nb = c1 - c0;

@@ -168,20 +168,29 @@ int enzoe_vlct_compute_dt(enzoe_vlct_t m, const enzoe_block *blocks, int n,
  * launch structures on a scratch copy of the leading blocks (at most ~2 GiB;
  * the caller's fields are not touched), advancing them by dt, and keeps the
  * fastest for this block shape; later compute calls on blocks of that shape
- * use it.  The candidates: every combination of XCD-contiguous workgroup
+ * use it.  The candidates, first of the separate launches: every combination of XCD-contiguous workgroup
  * order over the four stage kernels (k_flux, k_edge, k_faces, k_cells)
  * and, with the launch-structure setting "auto" (enzoe_vlct_set_fused_ct),
  * for MHD the fused CT + update launch with each of its tile shapes and the
  * orders of its two kernels, and (HLLD MHD or hydro, no dual energy) the
- * persistent launch of a whole stage, and the marched stages; then, for the
- * chosen one of the others, the rows of the tiled cell order (slabs
- * of 8, 16, 32 or 64 rows, or the plain order), and the other shapes of the flux launch (enzoe_vlct_set_flux_shape).
- * *mask_out (optional) gets the chosen mask: bit 0 k_flux, 1 k_edge,
- * 2 k_faces, 3 k_cells (or the fused launch).  enzoe_vlct_launch_choice:
- * the mask, the launch structure (0 = four launches per stage, or where the
- * setting is "auto" the marched stages; 1..5 as enzoe_vlct_set_fused_ct; of a
- * call of one block until the autotuner has run), the tile rows and the flux-launch shape (0..2)
- * calls on blocks of this shape use.                                       */
+ * persistent launch of a whole stage; for the chosen one the rows of the
+ * tiled cell order (slabs of 8, 16, 32 or 64 rows, or the plain order) and
+ * the other shapes of the flux launch (enzoe_vlct_set_flux_shape).  With both
+ * settings "auto" then the whole stage as one launch, marched or (hydro)
+ * tiled, against that one; which wins goes with the number of blocks, so this
+ * choice holds for calls whose active cells lie in the same octave as the
+ * sample's (from 2^20 on, for all of them), and calls of other sizes take the
+ * one or the other by size, as before.  Calls that cannot take a stage as one
+ * launch (stored fluxes, debug counts) use the choice among the separate
+ * launches.
+ * *mask_out (optional) gets the chosen mask of the separate launches: bit 0
+ * k_flux, 1 k_edge, 2 k_faces, 3 k_cells (or the fused launch).
+ * enzoe_vlct_launch_choice: the settings of the separate launches for blocks
+ * of this shape, whether or not a call takes them: the mask, the launch
+ * structure (0 = four launches per stage; 1..5 as enzoe_vlct_set_fused_ct; of
+ * a call of one block until the autotuner has run), the tile rows and the
+ * flux-launch shape (0..2).  Whether a call's stages run marched or tiled is
+ * seen in the kernels of enzoe_profile_report.                             */
 int enzoe_vlct_autotune(enzoe_vlct_t m, const enzoe_block *blocks, int n,
                         double dt, enzoe_stream_t stream, int *mask_out);
 int enzoe_vlct_launch_choice(enzoe_vlct_t m, int mx, int my, int mz, int *mask,
@@ -726,8 +735,11 @@ int enzoe_vlct_transfer_batch(enzoe_vlct_t m, const enzoe_transfer *items,
  * launch that marches tiles of columns through the planes and keeps fluxes,
  * EMFs and faces on the chip (two-stage schemes, from 2^18 active cells of a
  * call on, FP64 hydro 3 2^17, where no debug counts, stored fluxes or
- * flux-launch shape are asked for), else variant 2 for MHD launches of fewer
- * than 2^19 cells (ghost zones included), else the four launches.
+ * flux-launch shape are asked for); of hydro launches of fewer than 2^16
+ * cells (dual energy: 2^15), ghost zones included, each stage as one launch
+ * over tiles of 8 x 4 x 4 cells, under the same conditions; else variant 2 for
+ * MHD launches of fewer than 2^19 cells (ghost zones included), else the four
+ * launches.
  * Every variant gives the same bits, in FP64 and in mixed precision (the
  * contracted build: up to the rounding of its flux arithmetic, whose
  * multiply-adds the compiler may fuse differently in different kernels).  Not

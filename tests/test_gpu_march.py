@@ -307,3 +307,70 @@ def test_one_stage_scheme_equals_the_oracle(recon, dual, n):
     for k in got:
         if k in want:
             assert np.array_equal(got[k], want[k]), k
+
+
+def _names_of_a_step(ev, m, blocks, dt):
+    ev.profiling(True)
+    nxt = m.compute_timestep(blocks, dt)
+    names = set(ev.profile_report())
+    ev.profiling(False)
+    return names, nxt
+
+
+@pytest.mark.parametrize("mhd,n,tuned,called,kernel", [
+    # one block tuned, a batch above the marched stages' size called, and the
+    # other way round
+    (True, (32, 32, 32), 1, 12, "k_march_nn"), (True, (20, 18, 16), 48, 1, "k_flux_nn"),
+    (False, (32, 32, 32), 1, 14, "k_march_nn"), (False, (16, 16, 16), 60, 1, "k_tile_nn")])
+def test_a_tuned_shape_keeps_the_choice_by_size_for_other_batches(mhd, n, tuned, called, kernel):
+    """The autotuner's choice between separate launches and a whole stage as
+    one holds for launches of the sample's size; a batch of another size
+    of the same shape takes the one that its size asks for, with the same
+    bits."""
+    ev = _ev()
+    states = [_state(n, 90 + s, mhd=mhd) for s in range(2)]
+    out, nxt = [], []
+    for tune in (True, False):
+        m = ev.VlctMethod(mhd=mhd, riemann="hlld" if mhd else "hllc", reconstruct="plm",
+                          theta=2.0, courant=0.4)
+        if tune:
+            m.autotune(_blocks(ev, n, states, tuned, mhd=mhd), 1e-4)
+        else:
+            m.set_fused_ct(0)
+        blocks = _blocks(ev, n, states, called, mhd=mhd)
+        names, dt = _names_of_a_step(ev, m, blocks, 1e-4)
+        if tune:
+            assert kernel in names, names
+        nxt.append(dt)
+        out.append(blocks)
+    assert nxt[0] == nxt[1]
+    _equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("mhd,dual,n,count", [(True, False, (32, 32, 32), 12),
+                                              (False, False, (12, 12, 12), 1),
+                                              (False, True, (24, 20, 16), 1)])
+def test_tuned_batches_keep_their_results(mhd, dual, n, count):
+    """At the sample's own size, whatever the autotuner chose: the same bits,
+    and calls with debug counts still take the separate launches."""
+    ev = _ev()
+    states = [_state(n, 95 + s, dual, mhd) for s in range(2)]
+    out = []
+    for tune in (True, False):
+        m = ev.VlctMethod(mhd=mhd, riemann="hlld" if mhd else "hllc", reconstruct="plm",
+                          theta=2.0, courant=0.4, dual_energy_eta=0.001 if dual else None)
+        blocks = _blocks(ev, n, states, count, dual, mhd)
+        if tune:
+            mask = m.autotune(blocks, 1e-4)
+            assert m.launch_choice(tuple(x + 2 * G for x in n))[0] == mask
+        else:
+            m.set_fused_ct(0)
+        m.compute(blocks, 1e-4)
+        m.compute_timestep(blocks, 1e-4)
+        if tune:
+            m.set_debug_checks(True)
+        names, _ = _names_of_a_step(ev, m, blocks, 1e-4)
+        if tune:
+            assert not any(k.startswith(("k_march", "k_tile")) for k in names)
+        out.append(blocks)
+    _equal(out[0], out[1])
