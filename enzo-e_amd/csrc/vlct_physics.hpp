@@ -45,7 +45,14 @@ enum : int { RC_NN = 0, RC_PLM = 1, RC_PLM_ATHENA = 2 };
 // fix-up puts zeros, infinities and NaN right.  9 and 7 instructions instead
 // of 11, and none of the wait states that the scaled form's flag costs.
 // Rounded as IEEE division for 2^-1000 < |b| < 2^1000 and quotients and
-// residuals in the normal range.  With the shared reciprocals (qdiv_inv) and
+// residuals in the normal range.  (For a mantissa of all ones the last
+// correction of 1 / b is a tie that the sign of the seed's error decides; on
+// gfx950 it comes out right: compared with IEEE division over both ends of
+// the mantissas of every binade from 2^-1021 to 2^1021, no difference.)  A
+// subnormal divisor or a quotient that overflows gives NaN where IEEE
+// division gives a large number or infinity: no state gets there whose
+// densities and pressures stay above floors of normal size (1e-200 unless
+// set), speeds and sums of roots included.  With the shared reciprocals (qdiv_inv) and
 // the roots below the FP64 flux kernels, bound by their instruction issue,
 // take 1.51 and 2.11 ms on a 256^3 block (nearest neighbour, PLM) instead
 // of 1.67 and 2.23.

@@ -47,3 +47,67 @@ def test_scaled_states_match_oracle(case, s, d):
         if name in arr:
             # (the HLLE average speed of a 1e120 density is NaN, in both)
             assert np.array_equal(got[name], arr[name], equal_nan=True), name
+
+
+def _step_as_the_oracle(grid, cycles=2):
+    import enzoe_vlct as ev
+    method = method_for(grid.cfg)
+    dg = device_copy(grid, method)
+    t = 0.0
+    for _ in range(cycles):
+        dt = grid.cycle(t, 1e300)
+        assert dg.cycle(t, 1e300) == dt
+        t += dt
+    ev.synchronize()
+    got, want = dg.blocks[0].download(), grid.block_arrays(0)
+    for name in got:
+        if name in want:
+            assert np.array_equal(got[name], want[name], equal_nan=True), name
+
+
+# the divisors (densities, and differences and sums of momenta and pressures)
+# out to both ends of the range for which the divisions are stated.  The MHD
+# solves also divide products of momentum and field, which go with the density
+# to the power 3/2: there the ends come at 2^-640 (numerators may cancel by
+# another 2^-30 and have to keep their residuals normal) and 2^680.
+ENDS = {True: (-600, -450, 450, 650), False: (-930, -700, 700, 930)}
+
+
+@pytest.mark.parametrize("end", range(4))
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "%s-%s" % (c["riemann"], c["recon"][1]))
+def test_divisors_at_the_ends_of_the_range_match_oracle(case, end):
+    exponent = ENDS[case["mhd"]][end]
+    grid = random_periodic_grid(mhd=case["mhd"], seed=29, n=(9, 8, 10),
+                                riemann=case["riemann"], recon=case["recon"],
+                                theta=case["theta"], vamp=0.6, bamp=0.08)
+    grid.cfg.density_floor = grid.cfg.pressure_floor = 1e-300
+    d = 2.0 ** exponent
+    for name, f in grid.block_arrays(0).items():
+        if name == "density":
+            f *= d
+        elif name.startswith("bfield"):
+            f *= 2.0 ** (exponent // 2)
+    _step_as_the_oracle(grid)
+
+
+# a reciprocal of a divisor whose mantissa is all ones is an exact tie of its
+# last correction if the hardware's seed errs to the one side
+@pytest.mark.parametrize("shift", [0, -500, 500])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "%s-%s" % (c["riemann"], c["recon"][1]))
+def test_divisors_of_all_ones_match_oracle(case, shift):
+    """Densities just below powers of two (mantissas of all ones, and the
+    five values below each)."""
+    grid = random_periodic_grid(mhd=case["mhd"], seed=37, n=(9, 8, 10),
+                                riemann=case["riemann"], recon=case["recon"],
+                                theta=case["theta"], vamp=0.3, bamp=0.05)
+    arr = grid.block_arrays(0)
+    rng = np.random.default_rng(5)
+    top = 2.0 ** rng.integers(0, 3, arr["density"].shape)
+    ulps = rng.integers(1, 6, arr["density"].shape) * (rng.random(top.shape) < 0.5)
+    density = (top - (1 + ulps) * np.spacing(top) / 2) * 2.0 ** shift
+    arr["density"][...] = density
+    for name, f in arr.items():
+        if name.startswith("bfield"):
+            f *= 2.0 ** (shift // 2)
+    grid.refresh()
+    _step_as_the_oracle(grid)
