@@ -994,7 +994,6 @@ k_march_hd(const BlockDesc<T> *__restrict__ blocks, StageParams sp, MarchParams 
           march_prim<false>(nx2, fc.gm1, wp);
           if (CHECK && (march_wild<false>(h) || march_wild<false>(wp))) sWild = 1;
         }
-        if (!PLM) lds_barrier();  // (the x and y states of this plane have been read)
         if (lane) {
 #pragma unroll
           for (int q = 0; q < NQ; q++) sW[q][wi] = w[q];
