@@ -208,6 +208,21 @@ def dominant_kernel(prof):
     return "k_march_plm" if "k_march_plm" in prof else "k_flux_plm"
 
 
+def stages_of(prof):
+    """How the timed steps' stages ran: a whole stage as one launch (marched,
+    tiled), or separate launches."""
+    for prefix, how in (("k_march", "marched"), ("k_tile", "tiled")):
+        if any(k.startswith(prefix) for k in prof):
+            return how
+    return "separate"
+
+
+def launch_choice_of(method, shape, prof):
+    """The separate launches' settings for the shape where the steps ran
+    them, else None."""
+    return method.launch_choice(shape) if stages_of(prof) == "separate" else None
+
+
 def step_roofline(prec_name, zones, ms_per_step, gpu_ms_per_step, workload, mhd=True,
                   march=False):
     """The step against the HBM roofline as the metric defines it: the
@@ -381,7 +396,6 @@ def timed_run(precision, n, steps, warmup, dual_energy=False, launch_mask=-1, ke
         mask = launch_mask
     else:
         mask = method.autotune(grid.blocks, dt)
-    choice = method.launch_choice((n + 6,) * 3)
     ev.profiling(True)
     ev.synchronize()
     t0 = time.perf_counter()
@@ -391,6 +405,7 @@ def timed_run(precision, n, steps, warmup, dual_energy=False, launch_mask=-1, ke
     el = time.perf_counter() - t0
     prof = ev.profile_report()
     ev.profiling(False)
+    choice = launch_choice_of(method, (n + 6,) * 3, prof)
     kept = {"grid": grid, "method": method} if keep else {}
     del grid, method
     zones = n ** 3
@@ -411,7 +426,7 @@ def timed_run(precision, n, steps, warmup, dual_energy=False, launch_mask=-1, ke
             "step_gbs": STEP_BYTES_PER_ZONE_FP64 * zones / (gpu_step_ms * 1e-3) / 1e9,
             "workload": "orszag_tang_%d3_%s%s_vlct_plm_hlld" % (
                 n, precision, "_dual_energy" if dual_energy else ""),
-            "launch_mask": mask, "launch_choice": choice, **kept}
+            "stages": stages_of(prof), "launch_mask": mask, "launch_choice": choice, **kept}
 
 
 def _roofline(prof, steps, cells_per_step, prec, mhd, workload):
@@ -562,7 +577,8 @@ def run_batched_amr(a):
                                                       precision, True,
                                                       "batched_amr_%s" % precision),
                           "launch_blocks": lv.launch_sizes(),
-                          "launch_choice": method.launch_choice((38, 38, 38)),
+                          "stages": stages_of(prof),
+                          "launch_choice": launch_choice_of(method, (38, 38, 38), prof),
                           "driver": "HIP graph of %d device-driven coarse steps" % a.steps}
         plan.destroy()
         method.check_persistent()
@@ -579,7 +595,7 @@ def run_batched_amr(a):
         "config": {"workload": "batched_amr_32_512_1536_3000_%s" % a.precision,
                    "blocks_per_level": [512, 1536, 3000], "block": [32, 32, 32],
                    "subcycling": "2:1", "launch_blocks": r["launch_blocks"],
-                   "launch_choice": r["launch_choice"]},
+                   "stages": r["stages"], "launch_choice": r["launch_choice"]},
         "roofline": r["roofline"], "kernels_ms": r["kernels_ms"],
     }
     if len(res) == 2:
@@ -587,6 +603,7 @@ def run_batched_amr(a):
         out["precision_comparison"] = {"fp64_value": f["value"], "mixed_value": m["value"],
                                        "mixed_over_fp64": m["value"] / f["value"],
                                        "mixed_kernels_ms": m["kernels_ms"],
+                                       "mixed_stages": m["stages"],
                                        "mixed_launch_choice": m["launch_choice"]}
     return out
 
@@ -1004,8 +1021,8 @@ def main():
         "config": {"workload": r["workload"],
                    "block": [a.n, a.n, a.n], "ghost": 3, "riemann": "hlld",
                    "reconstruct": "plm", "theta": 2.0, "courant": 0.4,
-                   "precision": a.precision, "launch_mask": r["launch_mask"],
-                   "launch_choice": r["launch_choice"],
+                   "precision": a.precision, "stages": r["stages"],
+                   "launch_mask": r["launch_mask"], "launch_choice": r["launch_choice"],
                    "dual_energy": a.dual_energy},
         # the step against the roofline as the metric defines it (440 B per
         # zone-update, fully fused); the dominant kernel's own figure beside it
