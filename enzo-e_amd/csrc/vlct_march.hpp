@@ -17,8 +17,9 @@
 //   B   the faces of plane k - 1 and the level between, from those EMFs;
 //   U   the cell of plane k - 1.
 // The expressions are the ones of the separate kernels (solve_face,
-// edge_value, face_b_update, cell_finish), so the FP64 results are the same
-// bits.
+// edge_value, face_b_update, cell_finish), so the results are the same bits,
+// FP64 and mixed (in the contracted build the compiler fuses them as it finds
+// them in each kernel).
 //
 // What bounds it: FP64 instruction issue.  A 256^3 block's stages execute
 // 2020 (nearest neighbour) and 2400 (PLM) VALU instructions a column and

@@ -374,3 +374,41 @@ def test_tuned_batches_keep_their_results(mhd, dual, n, count):
             assert not any(k.startswith(("k_march", "k_tile")) for k in names)
         out.append(blocks)
     _equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+@pytest.mark.parametrize("mhd,n,count,kernel", [(True, (32, 32, 32), 12, "k_march_nn"),
+                                                (False, (32, 32, 32), 14, "k_march_nn"),
+                                                (False, (16, 14, 12), 2, "k_tile_nn")])
+def test_gravity_in_whole_stage_launches(mhd, n, count, kernel, precision):
+    """The acceleration of every cell added in the marched and tiled second
+    stage, as in the separate one: the same bits."""
+    ev = _ev()
+    states = [_state(n, 60 + s, mhd=mhd) for s in range(2)]
+    rng = np.random.default_rng(8)
+    m3 = tuple(x + 2 * G for x in n[::-1])
+    out = []
+    acc = []
+    for _ in range(count):
+        buf = ev.DeviceBuffer(3 * 8 * int(np.prod(m3)))
+        ev.to_device(buf.ptr.value, rng.standard_normal((3,) + m3))
+        acc.append(buf)
+    ptrs = [tuple(b.ptr.value + 8 * a * int(np.prod(m3)) for a in range(3)) for b in acc]
+    for structure in (-1, 0):
+        m = ev.VlctMethod(mhd=mhd, riemann="hlld" if mhd else "hllc", reconstruct="plm",
+                          theta=1.5, courant=0.4,
+                          precision=ev.ENZOE_PREC_MIXED if precision == "mixed"
+                          else ev.ENZOE_PREC_DOUBLE)
+        m.set_fused_ct(structure)
+        blocks = _blocks(ev, n, states, count, mhd=mhd)
+        ev.profiling(True)
+        ev.compute_gravity(m, blocks, 2e-4, ptrs)
+        names = ev.profile_report()
+        ev.profiling(False)
+        assert (kernel in names) == (structure == -1)
+        out.append(blocks)
+    _equal(out[0], out[1])
+    plain = _blocks(ev, n, states, count, mhd=mhd)
+    m.compute(plain, 2e-4)
+    assert not np.array_equal(plain[0].download()["velocity_x"],
+                              out[1][0].download()["velocity_x"])
